@@ -48,6 +48,7 @@
 //   batches (256-thread workgroups) groups of 16 x 16 took the batched
 //   forward projection of the 64-problem workload from 104.8 to 98.1 ms.
 #include <algorithm>
+#include <cmath>
 #include <new>
 #include <vector>
 
@@ -401,27 +402,34 @@ __device__ __forceinline__ void fp_tile_at(
 
 // Decode logical block id `bid` (groups of grp_a angles x grp_c column
 // tiles, angle fastest inside a group; groups ordered angle group, then
-// column-tile group, then row band) and trace that tile.  TABLE_IN_MEMORY: the angle table pointer was
-// read from a descriptor (batch kernels); the record is then copied through
-// constant-memory (scalar) loads first.  A table passed as a kernel
-// argument is read in place (the compiler scalarizes it by itself; the
-// explicit copy measured 5% slower at 512^3 / 720 angles).
-template <int R, bool ALL_COLC, bool PIPE, int COLS, bool TABLE_IN_MEMORY,
-          bool PTRS = false>
-__device__ __forceinline__ void fp_tile(const kk::FpAngle* __restrict__ tab,
-                                        const FpArgs& A, int64_t bid) {
+// column-tile group, then row band); false for the grid's padding.
+__device__ __forceinline__ bool fp_decode(const FpArgs& A, int64_t bid,
+                                          int32_t& ang, int32_t& ct,
+                                          int32_t& rt) {
   const int32_t ga = A.grp_a, gc = A.grp_c;
   const int64_t inner = bid % (int64_t(ga) * gc);
   const int64_t outer = bid / (int64_t(ga) * gc);
   const int32_t nag = (A.n_angles + ga - 1) / ga;
   const int32_t ncg = (A.col_tiles + gc - 1) / gc;
-  const int32_t ang = static_cast<int32_t>(outer % nag) * ga +
-                      static_cast<int32_t>(inner % ga);
+  ang = static_cast<int32_t>(outer % nag) * ga +
+        static_cast<int32_t>(inner % ga);
   const int64_t t = outer / nag;
-  const int32_t ct = static_cast<int32_t>(t % ncg) * gc +
-                     static_cast<int32_t>(inner / ga);
-  const int32_t rt = static_cast<int32_t>(t / ncg);
-  if (ang >= A.n_angles || ct >= A.col_tiles) return;  // grid padding
+  ct = static_cast<int32_t>(t % ncg) * gc + static_cast<int32_t>(inner / ga);
+  rt = static_cast<int32_t>(t / ncg);
+  return ang < A.n_angles && ct < A.col_tiles;
+}
+
+// Trace the tile of logical block id `bid`.  TABLE_IN_MEMORY: the angle
+// table pointer was read from a descriptor (batch kernels); the record is
+// then copied through constant-memory (scalar) loads first.  A table passed
+// as a kernel argument is read in place (the compiler scalarizes it by
+// itself; the explicit copy measured 5% slower at 512^3 / 720 angles).
+template <int R, bool ALL_COLC, bool PIPE, int COLS, bool TABLE_IN_MEMORY,
+          bool PTRS = false>
+__device__ __forceinline__ void fp_tile(const kk::FpAngle* __restrict__ tab,
+                                        const FpArgs& A, int64_t bid) {
+  int32_t ang, ct, rt;
+  if (!fp_decode(A, bid, ang, ct, rt)) return;
   if constexpr (TABLE_IN_MEMORY) {
     const kk::FpAngle rec = kk_uniform_load(tab + ang);
     fp_tile_at<R, ALL_COLC, PIPE, COLS, PTRS>(&rec, 0, A, ang, ct, rt);
@@ -453,6 +461,285 @@ __global__ __launch_bounds__(kColsSingle * kWave, fp_min_blocks(R)) void cone_fp
       tab, A, kk_xcd_remap(blockIdx.x, A.total_blocks, A.xcd_group));
 }
 
+
+// ---- column-coherent launches: one volume line per column and slice ------
+//
+// When every angle is column-coherent (circular orbits), the rays of one
+// detector column meet a slice at one b coordinate: all of its samples there
+// interpolate between the same two volume rows, at c coordinates affine in
+// the detector row.  A wavefront owns 64 R consecutive rows of one column.
+// Per slice it reads the window of the two rows that its rays reach (one
+// coalesced 4-byte load per 64 elements and row, from planes: the volume as
+// plain floats), interpolates them along b once per element, keeps that line
+// in its own LDS words, and every ray reads two neighbouring words of it.
+// The arithmetic per sample is bilerp's (along b, then along c).
+//
+// What bounds it (MI355X): a 16-byte gather costs a CU 16 cycles per 64
+// samples whatever its pattern, a coalesced 4-byte load 4.5, an LDS store
+// 5.2 and a paired LDS read at neighbouring addresses 5.0; so with windows
+// of W x 64 elements a sample costs 9 W / R cycles of loads beside
+// (5.2 W + 5 R) / R of LDS and ~9 of vector instructions.  Measured: FP
+// 512^3 / 720 x 768^2 85.7-91 -> 57 ms, 128^3 / 180 x 160^2 0.43 -> 0.27 ms
+// (R = 1, 2, 3, 4 at the former: 141, 91, 64, 57 ms).  Of the 57 ms, 37
+// remain without the loads and 47 when every load hits the L2: what is left
+// is vector issue first, then misses (a second slice in flight, two columns
+// per wavefront and slabs of slices were no faster).
+//
+// c coordinates are 64-bit fixed point (32 fraction bits), stepped by one
+// 64-bit add per slice: the high word is the element, the low word the
+// weight.  Their error (the slope's rounding, 2^-33 per slice) is below the
+// weights' own float32 rounding up to ~1000 slices.
+// Columns (wavefronts) per workgroup.  They walk the same slices behind one
+// barrier per slice, so that neighbouring columns' rows meet in the CU's L1
+// (57.0 ms against 62.5 without; 8 and 16 columns 59.2 and 61.9 ms).
+constexpr int kLineWaves = 4;
+constexpr int32_t kLineGroupAngles = 8;   // workgroup groups, as kGroupAngles
+constexpr int32_t kLineGroupCols = 32;    // (16 x 16: 58.7 ms)
+constexpr int kLineChunks = 4;                  // windows up to 4 x 64
+constexpr int kLineWords = 64 * kLineChunks;    // LDS words per wavefront
+constexpr int64_t kLineEps = int64_t(1) << 18;  // 2^-14 voxel, fixed point
+
+// x as 64-bit fixed point with 32 fraction bits (|x| < 2^31).
+__device__ __forceinline__ int64_t to_fixed(double x) {
+  const double fl = floor(x);
+  const uint32_t lo = static_cast<uint32_t>((x - fl) * 4294967296.0);
+  return static_cast<int64_t>(
+      (static_cast<uint64_t>(static_cast<uint32_t>(static_cast<int32_t>(fl)))
+       << 32) |
+      lo);
+}
+
+__device__ __forceinline__ int64_t bcast64(int64_t v, int32_t lane) {
+  const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_readlane(
+      static_cast<int32_t>(static_cast<uint64_t>(v)), lane));
+  const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_readlane(
+      static_cast<int32_t>(static_cast<uint64_t>(v) >> 32), lane));
+  return static_cast<int64_t>((static_cast<uint64_t>(hi) << 32) | lo);
+}
+
+__device__ __forceinline__ int32_t fixed_int(int64_t x) {
+  return static_cast<int32_t>(static_cast<uint64_t>(x) >> 32);
+}
+__device__ __forceinline__ float fixed_frac(int64_t x) {
+  return static_cast<float>(static_cast<uint32_t>(x)) * 0x1p-32f;
+}
+
+// A wave's state along the slices: per-lane c coordinates and steps of its R
+// rays, wave-uniform b coordinate and window start with their steps.
+template <int R>
+struct LineWalk {
+  int64_t X[R], S[R];
+  int64_t B, SB, E, SE;
+};
+
+// n slices from `slice` (byte address of the plane) with windows of W chunks.
+// The next slice's loads are in flight while a slice is interpolated.
+template <int R, int W>
+__device__ __forceinline__ void line_trace(LineWalk<R>& w, int32_t n,
+                                           const char*& slice, uint64_t sab,
+                                           uint32_t sbb, int32_t row_bytes,
+                                           int32_t nb1, uint32_t line_at,
+                                           uint32_t lane4, float (&acc)[R]) {
+  typedef __attribute__((address_space(3))) float* lds_ptr;
+  if (n <= 0) return;
+  float v0[W], v1[W], fb;
+  int32_t z0;
+  // Both rows' window at the current slice, through buffer descriptors that
+  // hold one row each: elements before the row (negative offsets, i.e. large
+  // unsigned ones) and after it read as zero.
+  auto request = [&]() {
+    const int32_t jb = fixed_int(w.B);
+    const int32_t j = min(max(jb, 0), nb1);
+    fb = fixed_frac(j == jb ? w.B : 0);
+    z0 = __builtin_amdgcn_readfirstlane(fixed_int(w.E));
+    const char* row = slice + static_cast<uint64_t>(
+        static_cast<uint32_t>(j) * sbb);
+    const auto r0 = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<char*>(row), 0, row_bytes, 0x00020000);
+    const auto r1 = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<char*>(row + sbb), 0, row_bytes, 0x00020000);
+#pragma unroll
+    for (int c = 0; c < W; ++c) {
+      // (in asm, so that no negative offset meets an immediate)
+      uint32_t o;
+      asm("v_add_u32 %0, %1, %2"
+          : "=v"(o)
+          : "s"((z0 + c * kWave) * 4), "v"(lane4));
+      v0[c] = __builtin_bit_cast(
+          float, __builtin_amdgcn_raw_buffer_load_b32(r0, o, 0, 0));
+      v1[c] = __builtin_bit_cast(
+          float, __builtin_amdgcn_raw_buffer_load_b32(r1, o, 0, 0));
+    }
+    w.B += w.SB;
+    w.E += w.SE;
+    slice += sab;
+  };
+  const lds_ptr st = (lds_ptr)(line_at + lane4);
+  request();
+  for (;;) {
+    __builtin_amdgcn_s_barrier();
+#pragma unroll
+    for (int c = 0; c < W; ++c)
+      st[c * kWave] = fmaf(fb, v1[c] - v0[c], v0[c]);
+    __builtin_amdgcn_wave_barrier();
+    const uint32_t at = line_at - static_cast<uint32_t>(z0) * 4u;
+    float l0[R], l1[R];
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      uint32_t q;  // one shift-add of the element (not a 64-bit shift)
+      asm("v_lshl_add_u32 %0, %1, 2, %2"
+          : "=v"(q)
+          : "v"(fixed_int(w.X[k])), "s"(at));
+      l0[k] = ((lds_ptr)q)[0];
+      l1[k] = ((lds_ptr)q)[1];
+    }
+    const bool more = --n > 0;
+    if (more) request();
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      acc[k] += fmaf(fixed_frac(w.X[k]), l1[k] - l0[k], l0[k]);
+      w.X[k] += w.S[k];
+    }
+    if (!more) break;
+  }
+}
+
+template <int R, bool PTRS>
+__global__ __launch_bounds__(kLineWaves * kWave, 8) void cone_fp_line_kernel(
+    const kk::FpAngle* __restrict__ tab, FpArgs A) {
+  __shared__ float lines[kLineWaves * kLineWords];
+  int32_t ang, ct, rt;
+  if (!fp_decode(A, kk_xcd_remap(blockIdx.x, A.total_blocks, A.xcd_group),
+                 ang, ct, rt))
+    return;
+  const int32_t lane = int32_t(threadIdx.x) & (kWave - 1);
+  const int32_t wave = __builtin_amdgcn_readfirstlane(
+      int32_t(threadIdx.x) / kWave);
+  // columns past the detector repeat the last one (not written out)
+  const int32_t wcol = ct * kLineWaves + wave;
+  const int32_t col = min(wcol, A.cols - 1);
+  const int32_t row0 = rt * (kWave * R);
+  const kk::FpAngle& P = tab[ang];
+  const float nb1 = static_cast<float>(P.nb + 1);
+  const float nc1 = static_cast<float>(P.nc + 1);
+  const float last = static_cast<float>(P.na - 1);
+
+  double a1 = 0.0, b1 = 0.0, a2[R], b2[R];
+  int32_t ilo = 0x7fffffff, ihi = -1;
+#pragma unroll
+  for (int k = 0; k < R; ++k) {
+    // rows past the detector repeat the last one (not written out)
+    const int32_t row = min(row0 + kWave * k + lane, A.rows - 1);
+    // (no ray is parallel to the slices: line_spacing)
+    kk_fp_ray(P, row, col, a1, b1, a2[k], b2[k]);
+    float lo = 0.f, hi = last;
+    clip_range(static_cast<float>(a1), static_cast<float>(b1), nb1, last, lo,
+               hi);
+    clip_range(static_cast<float>(a2[k]), static_cast<float>(b2[k]), nc1, last,
+               lo, hi);
+    if (lo <= hi + 2.f) {
+      ilo = min(ilo, max(0, static_cast<int32_t>(floorf(lo)) - 1));
+      ihi = max(ihi, min(P.na - 1, static_cast<int32_t>(ceilf(hi)) + 1));
+    }
+  }
+  {
+    __shared__ int32_t lim[2][16];
+    lim[0][wave] = kk_wave_min(ilo);
+    lim[1][wave] = kk_wave_max(ihi);
+    __syncthreads();
+    #pragma unroll
+    for (int32_t t = 0; t < kLineWaves; ++t) {
+      ilo = min(ilo, lim[0][t]);
+      ihi = max(ihi, lim[1][t]);
+    }
+  }
+  ilo = __builtin_amdgcn_readfirstlane(ilo);
+  ihi = __builtin_amdgcn_readfirstlane(ihi);
+
+  float acc[R];
+#pragma unroll
+  for (int k = 0; k < R; ++k) acc[k] = 0.f;
+  if (ilo <= ihi) {
+    const double fi = static_cast<double>(ilo);
+    LineWalk<R> w;
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      w.X[k] = to_fixed(fma(a2[k], fi, b2[k]));
+      w.S[k] = to_fixed(a2[k]);
+    }
+    w.B = bcast64(to_fixed(fma(a1, fi, b1)), 0);
+    w.SB = bcast64(to_fixed(a1), 0);
+    // the window lies between the c coordinates of the first and last rows
+    // (those between lie between up to the rounding that kLineEps covers);
+    // which is the lower does not change along the slices
+    const int64_t E0 = bcast64(w.X[0], 0), E1 = bcast64(w.X[R - 1], kWave - 1);
+    const int64_t S0 = bcast64(w.S[0], 0), S1 = bcast64(w.S[R - 1], kWave - 1);
+    const int32_t n = ihi - ilo + 1;
+    const bool up = E1 + (n >> 1) * S1 >= E0 + (n >> 1) * S0;
+    w.E = bcast64((up ? E0 : E1) - kLineEps, 0);
+    w.SE = bcast64(up ? S0 : S1, 0);
+    // window widths (elements) at the first and the last slice, linear
+    // between; one chunk fewer where the window is that narrow
+    const float d0 = static_cast<float>(up ? E1 - E0 : E0 - E1) * 0x1p-32f;
+    const float ds = static_cast<float>(up ? S1 - S0 : S0 - S1) * 0x1p-32f;
+    const float wa = d0 + 3.1f, wb = fmaf(ds, static_cast<float>(n - 1), wa);
+    const int32_t top = __builtin_amdgcn_readfirstlane(
+        static_cast<int32_t>(ceilf(fmaxf(wa, wb) * (1.f / kWave))));
+    const float fit = static_cast<float>((top - 1) * kWave);
+    int32_t na = 0, nb = 0;  // narrow slices at the start / at the end
+    if (fmaxf(wa, wb) <= fit) na = n;
+    else if (wa <= fit && ds > 0.f)
+      na = min(n, max(0, static_cast<int32_t>((fit - wa) / ds)));
+    else if (wb <= fit && ds < 0.f)
+      nb = min(n, max(0, static_cast<int32_t>((fit - wb) / -ds)));
+    na = __builtin_amdgcn_readfirstlane(na);
+    nb = __builtin_amdgcn_readfirstlane(nb);
+
+    const uint32_t sbb = static_cast<uint32_t>(P.nc + kk::kHalo) * 4u;
+    const uint64_t sab = static_cast<uint64_t>(P.nb + kk::kHalo) * sbb;
+    const char* slice = A.tex + (P.tex_off >> 1) +
+                        static_cast<uint64_t>(ilo) * sab;
+    typedef __attribute__((address_space(3))) float* lds_ptr;
+    const uint32_t line_at = __builtin_amdgcn_readfirstlane(
+        static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
+            (lds_ptr)(lines + wave * kLineWords))));
+    const uint32_t lane4 = static_cast<uint32_t>(lane) * 4u;
+    const int32_t row_bytes = static_cast<int32_t>(sbb);
+#pragma unroll 1
+    for (int32_t pass = 0; pass < 3; ++pass) {
+      const int32_t m = pass == 0 ? na : (pass == 1 ? n - na - nb : nb);
+      const int32_t chunks = pass == 1 ? top : top - 1;
+      if (m <= 0) continue;
+#define KK_LINE(W_)                                                        \
+  line_trace<R, W_>(w, m, slice, sab, sbb, row_bytes, P.nb + 1, line_at, \
+                    lane4, acc)
+      if (chunks <= 1) KK_LINE(1);
+      else if (chunks == 2) KK_LINE(2);
+      else if (chunks == 3) KK_LINE(3);
+      else KK_LINE(4);
+#undef KK_LINE
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < R; ++k) {
+    const int32_t row = row0 + kWave * k + lane;
+    if (row >= A.rows || wcol >= A.cols) continue;
+    double ra1, rb1, ra2, rb2;
+    const float wt = kk_fp_ray(P, row, col, ra1, rb1, ra2, rb2)
+                         ? kk_fp_weight(P, ra1, ra2)
+                         : 0.f;
+    const int64_t o = ang * A.os0 + row * A.os1 + col * A.os2;
+    float* out = A.out;
+    if constexpr (PTRS)
+      out = reinterpret_cast<float*>(
+          A.out_ptrs[A.ptr_axis == 0 ? ang : (A.ptr_axis == 1 ? row : col)]);
+    if (A.mode == 1)
+      out[o] += acc[k] * wt;
+    else
+      out[o] = acc[k] * wt;
+  }
+}
+
 }  // namespace
 
 namespace {
@@ -466,9 +753,10 @@ int auto_rows_per_thread(int32_t rows, int32_t rpt) {
 }
 
 // Validate one forward-projection problem and fill its kernel arguments
-// for `rpt` rows per thread.
+// for `rpt` rows per thread and workgroup groups of at most `cap_angles` x
+// `cap_cols` column tiles.
 int make_fp_args(const kk::FpSpec& S, int32_t rpt, int32_t cols_per_block,
-                 FpArgs& A) {
+                 int32_t cap_angles, int32_t cap_cols, FpArgs& A) {
   using kk::fail;
   if (S.plan == nullptr || !S.plan->fp_set)
     return fail(KK_ERR_NOT_SET,
@@ -511,10 +799,8 @@ int make_fp_args(const kk::FpSpec& S, int32_t rpt, int32_t cols_per_block,
   A.row_tiles = (S.rows + kWave * rpt - 1) / (kWave * rpt);
   A.col_tiles = (S.cols + cols_per_block - 1) / cols_per_block;
   A.mode = S.mode;
-  A.grp_a = group_size(A.n_angles, kGroupAngles);
-  A.grp_c = group_size(
-      A.col_tiles,
-      cols_per_block == kColsSingle ? kGroupCols : kGroupColsBatch);
+  A.grp_a = group_size(A.n_angles, cap_angles);
+  A.grp_c = group_size(A.col_tiles, cap_cols);
   A.xcd_group = A.grp_a * A.grp_c;
   A.total_blocks = int64_t(A.row_tiles) *
                    ((A.n_angles + A.grp_a - 1) / A.grp_a) * A.grp_a *
@@ -616,7 +902,8 @@ int fp_batch_build(const std::vector<FpSpec>& specs, int32_t rows_per_thread,
   std::vector<int64_t> first(specs.size());
   int64_t total = 0;
   for (size_t p = 0; p < specs.size(); ++p) {
-    const int rc = make_fp_args(specs[p], rpt, kColsBatch, items[p].args);
+    const int rc = make_fp_args(specs[p], rpt, kColsBatch, kGroupAngles,
+                                kGroupColsBatch, items[p].args);
     if (rc != KK_OK) return rc;
     items[p].tab = specs[p].plan->fp;
     first[p] = total;
@@ -730,7 +1017,7 @@ int launch_fp_spec(const kk::FpSpec& S, int32_t rows_per_thread,
                    hipStream_t stream) {
   const int32_t rpt = auto_rows_per_thread(S.rows, rows_per_thread);
   FpArgs A;
-  const int rc = make_fp_args(S, rpt, kColsSingle, A);
+  const int rc = make_fp_args(S, rpt, kColsSingle, kGroupAngles, kGroupCols, A);
   if (rc != KK_OK) return rc;
   const dim3 grid(static_cast<unsigned>(A.total_blocks));
   const bool c = S.plan->fp_all_colc, p = S.ptrs != nullptr;
@@ -747,7 +1034,102 @@ int launch_fp_spec(const kk::FpSpec& S, int32_t rows_per_thread,
   return KK_OK;
 }
 
+// Rows per thread of the line kernel for `rows` detector rows at the plan's
+// c spacing (0: the launch is the gather kernel's).  Costs in cycles of a
+// SIMD, fitted on MI355X at 64 to 384 rows and spacings of 0.5 to 1.7 voxels:
+// a slice costs a wavefront 72 + 30 R, the gather 72 per 64 rows, and more
+// where its lanes spread over the cache lines (spacing above 1).  The line
+// kernel then took 0.52-0.90 of the gather's time where it is chosen: at 0.7
+// voxels 128 rows 0.89 -> 0.77 ms (R = 2), 190 rows 1.52 -> 0.91 (R = 3),
+// 384 rows 5.79 -> 4.18 (R = 3); at 1.7 voxels 384 rows 7.12 -> 4.78 (R = 1).
+int line_rows_per_thread(const kk_plan_s* plan, int32_t rows, int32_t cols) {
+  if (!plan->fp_set || plan->fp_line_max < 0.0 || cols > plan->fp_line_cols ||
+      rows > plan->fp_line_rows)
+    return 0;
+  const int32_t groups = (rows + kWave - 1) / kWave;
+  const double spread = std::max(0.0, 1.9 * (plan->fp_line_mean - 1.0));
+  int best = 0;
+  double best_cost = 0.92 * 72.0 * groups * (1.0 + spread);
+  for (int r = 1; r <= 4; ++r) {
+    // the widest window must fit (its ends' rounding and margins: 4)
+    const int32_t span = std::min(kWave * r, rows) - 1;
+    if (span * plan->fp_line_max + 4.0 > kLineWords) break;
+    const double cost = (72.0 + 30.0 * r) * ((groups + r - 1) / r);
+    if (cost < best_cost) {
+      best = r;
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+
+template <bool P>
+void launch_line(int32_t r, dim3 grid, hipStream_t stream,
+                 const kk::FpAngle* tab, const FpArgs& A) {
+  const dim3 block(kLineWaves * kWave);
+  switch (r) {
+    case 1:
+      hipLaunchKernelGGL((cone_fp_line_kernel<1, P>), grid, block, 0, stream,
+                         tab, A);
+      break;
+    case 2:
+      hipLaunchKernelGGL((cone_fp_line_kernel<2, P>), grid, block, 0, stream,
+                         tab, A);
+      break;
+    case 3:
+      hipLaunchKernelGGL((cone_fp_line_kernel<3, P>), grid, block, 0, stream,
+                         tab, A);
+      break;
+    default:
+      hipLaunchKernelGGL((cone_fp_line_kernel<4, P>), grid, block, 0, stream,
+                         tab, A);
+      break;
+  }
+}
+
+int launch_fp_planes(const kk::FpSpec& S, hipStream_t stream) {
+  if (S.plan == nullptr || !S.plan->fp_set)
+    return kk::fail(KK_ERR_NOT_SET,
+                    "Please set the projection geometry with `set_params()`.");
+  const int32_t r = line_rows_per_thread(S.plan, S.rows, S.cols);
+  if (r == 0)
+    return kk::fail(KK_ERR_UNSUPPORTED,
+                    "kk_cone_fp_planes: not a geometry for planes (see "
+                    "kk_fp_reads_planes)");
+  FpArgs A;
+  const int rc = make_fp_args(S, r, kLineWaves, kLineGroupAngles,
+                              kLineGroupCols, A);
+  if (rc != KK_OK) return rc;
+  const dim3 grid(static_cast<unsigned>(A.total_blocks));
+  if (S.ptrs != nullptr)
+    launch_line<true>(r, grid, stream, S.plan->fp, A);
+  else
+    launch_line<false>(r, grid, stream, S.plan->fp, A);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return kk::hip_fail(e, "cone_fp_line_kernel");
+  return KK_OK;
+}
+
 }  // namespace
+
+extern "C" int32_t kk_fp_reads_planes(const kk_plan* plan, int32_t rows,
+                                      int32_t cols) {
+  if (plan == nullptr || rows <= 0 || cols <= 0) return 0;
+  return line_rows_per_thread(plan, rows, cols) > 0 ? 1 : 0;
+}
+
+extern "C" int kk_cone_fp_planes(const kk_plan* plan, const float* planes,
+                                 float* proj, const int64_t* ptrs,
+                                 int32_t ptr_axis, const int64_t ps[3],
+                                 int32_t rows, int32_t cols, int32_t additive,
+                                 void* stream) {
+  kk::FpSpec S;
+  const int rc = kk::fp_spec(S, plan, planes, proj, ps, rows, cols, additive);
+  if (rc != KK_OK) return rc;
+  S.ptrs = ptrs;
+  S.ptr_axis = ptr_axis;
+  return launch_fp_planes(S, static_cast<hipStream_t>(stream));
+}
 
 extern "C" int kk_cone_fp(const kk_plan* plan, const float* vol_tex,
                           float* proj, const int64_t ps[3], int32_t rows,

@@ -204,6 +204,11 @@ struct kk_plan_s {
   bool fp_set = false;
   bool fp_all_colc = false;  // every angle column-coherent (FpAngle.colc)
   bool fp_any_colc = false;  // some angle column-coherent
+  // c distance of neighbouring detector rows' samples over the volume, its
+  // largest value (negative: not a geometry for the line kernel) and its
+  // mean, for detectors of at most fp_line_rows x fp_line_cols
+  double fp_line_max = -1.0, fp_line_mean = 0.0;
+  int32_t fp_line_rows = 0, fp_line_cols = 0;
   // angle ids grouped by ray axis: fr_idx[fr_start[a] .. fr_start[a+1])
   int32_t* fr_idx = nullptr;
   int32_t fr_cap = 0;

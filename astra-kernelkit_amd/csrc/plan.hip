@@ -214,6 +214,69 @@ static int build_fp_table(const double* params, int32_t n,
   return KK_OK;
 }
 
+// The c spacing of neighbouring rows' samples for the line kernel
+// (kk_plan_s.fp_line_*).  With every angle column-coherent a sample at slice i
+// has c coordinate tauc + (i + sig) D_c / D_a, D_a free of the row, so the
+// spacing is |v_c| t with t = (i + sig) / D_a, the share of the way from the
+// source to the detector.  t is linear in the sample's place (a, b) there, so
+// its largest value over the volume is at a corner; the corners are moved
+// outwards by what a workgroup's slices exceed its columns' own supports
+// (slices by a few, b by up to four columns' distance).  Negative if an angle
+// is not column-coherent, if a ray may run parallel to the slices (D_a
+// changes sign or nearly vanishes), if the source lies among the slices, or
+// if coordinates leave the fixed-point range.
+static void line_spacing(const std::vector<kk::FpAngle>& tab, int32_t rows,
+                         int32_t cols, kk_plan_s& plan) {
+  plan.fp_line_max = -1.0;
+  plan.fp_line_mean = 0.0;
+  plan.fp_line_rows = rows;
+  plan.fp_line_cols = cols;
+  if (rows <= 0 || cols <= 0) return;
+  double most = 0.0, sum = 0.0;
+  for (const kk::FpAngle& e : tab) {
+    if (!e.colc || e.na > 16384) return;
+    const double da[2] = {e.qa, e.qa + (cols - 1) * e.ua};
+    const double least = std::fmin(std::fabs(da[0]), std::fabs(da[1]));
+    if (!(da[0] * da[1] > 0.0) ||
+        !(least > 1e-9 * std::fmax(std::fabs(da[0]), std::fabs(da[1]))))
+      return;
+    // the source lies before or after all slices
+    const double i0 = e.sig, i1 = e.na - 1 + e.sig;
+    if (!(i0 / da[0] > 0.0 && i1 / da[0] > 0.0)) return;
+    for (int ic = 0; ic < 2; ++ic)
+      for (int is = 0; is < 2; ++is) {
+        const double t = (is ? i1 : i0) / da[ic];
+        const double fc = ic ? cols - 1 : 0;
+        const double xb = e.taub + t * (e.qb + fc * e.ub);
+        for (int ir = 0; ir < 2; ++ir) {
+          const double xc = e.tauc + t * (e.qc + fc * e.uc +
+                                          (ir ? rows - 1 : 0) * e.vc);
+          if (!(std::fabs(xb) < 1e8) || !(std::fabs(xc) < 1e8)) return;
+        }
+      }
+    // t(a, b) = (ub a' - ua b') / (ub qa - ua qb), a' and b' from the source
+    const double det = e.ub * e.qa - e.ua * e.qb;
+    if (!(std::fabs(det) > 0.0)) return;
+    auto at = [&](double ai, double xb) {
+      return (e.ub * (ai + e.sig) - e.ua * (xb - e.taub)) / det;
+    };
+    double far = 0.0;
+    for (int k = 0; k < 4; ++k)
+      far = std::fmax(far, at(k & 1 ? e.na - 1 : 0, k & 2 ? e.nb + 1 : 0));
+    const double step = std::sqrt(e.ua * e.ua + e.ub * e.ub) * far;
+    const double mb = 8.0 + 12.0 * step;
+    for (int k = 0; k < 4; ++k)
+      far = std::fmax(far, at(k & 1 ? e.na + 7 : -8,
+                              k & 2 ? e.nb + 1 + mb : -mb));
+    most = std::fmax(most, std::fabs(e.vc) * far);
+    const double mid = e.qa + 0.5 * (cols - 1) * e.ua;
+    sum += std::fabs(e.vc * (0.5 * (e.na - 1) + e.sig) / mid);
+  }
+  if (!std::isfinite(most) || !std::isfinite(sum)) return;
+  plan.fp_line_max = most;
+  plan.fp_line_mean = sum / double(tab.size());
+}
+
 extern "C" int kk_set_params_fp(kk_plan* plan, const double* params,
                                 int32_t n, const int32_t* axes, int32_t rows,
                                 int32_t cols, const int32_t shape[3],
@@ -249,6 +312,7 @@ extern "C" int kk_set_params_fp(kk_plan* plan, const double* params,
     plan->fp_all_colc = plan->fp_all_colc && tab[k].colc != 0;
     plan->fp_any_colc = plan->fp_any_colc || tab[k].colc != 0;
   }
+  line_spacing(tab, rows, cols, *plan);
   plan->fp_n = n;
   for (int t = 0; t < 3; ++t) plan->fp_shape[t] = shape[t];
   plan->fp_mask = mask;
@@ -340,6 +404,11 @@ extern "C" int64_t kk_fp_texture_elems(const int32_t s[3], int32_t mask) {
   return n;
 }
 
+extern "C" int64_t kk_fp_planes_elems(const int32_t s[3], int32_t mask) {
+  const int64_t n = kk_fp_texture_elems(s, mask);
+  return n < 0 ? n : n / 2;
+}
+
 extern "C" int64_t kk_bp_texture_elems(int32_t n, int32_t rows,
                                        int32_t cols) {
   if (n <= 0 || rows <= 0 || cols <= 0) return -1;
@@ -356,6 +425,23 @@ extern "C" int kk_fp_table(const double* params, int32_t n,
                                 voxel_size, tab, mask);
   if (rc != KK_OK) return rc;
   std::memcpy(out, tab.data(), sizeof(kk::FpAngle) * tab.size());
+  return KK_OK;
+}
+
+extern "C" int kk_fp_line_spacing(const double* params, int32_t n,
+                                  const int32_t* axes, int32_t rows,
+                                  int32_t cols, const int32_t shape[3],
+                                  const double voxel_size[3], double out[2]) {
+  if (out == nullptr)
+    return kk::fail(KK_ERR_INVALID, "kk_fp_line_spacing: null");
+  std::vector<kk::FpAngle> tab;
+  const int rc = build_fp_table(params, n, axes, rows, cols, shape,
+                                voxel_size, tab, nullptr);
+  if (rc != KK_OK) return rc;
+  kk_plan_s plan;
+  line_spacing(tab, rows, cols, plan);
+  out[0] = plan.fp_line_max;
+  out[1] = plan.fp_line_mean;
   return KK_OK;
 }
 

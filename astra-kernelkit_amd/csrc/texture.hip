@@ -48,6 +48,33 @@ __global__ __launch_bounds__(256) void fp_frame_kernel(
   }
 }
 
+// Plane frame of ray axis a: element (i, jb, jc) of a [na][nb+3][nc+3] float
+// array = V(i, jb-1, jc-1), zero outside (the layout of cone_fp_line_kernel).
+// A pure copy: one thread per element, jc fastest.
+__global__ __launch_bounds__(256) void fp_plane_kernel(
+    const float* __restrict__ vol, int64_t sa, int64_t sb, int64_t sc,
+    int32_t nb, int32_t nc, float* __restrict__ out) {
+  const int32_t tc = nc + kk::kHalo;
+  const int32_t tb = nb + kk::kHalo;
+  const int32_t jc = blockIdx.x * 256 + threadIdx.x;
+  const int32_t jb0 = blockIdx.y * kTexRows;
+  const int32_t i = blockIdx.z;
+  if (jc >= tc) return;
+  const int32_t c = jc - kk::kHaloLo;
+  const bool col = c >= 0 && c < nc;
+  const float* p = vol + i * sa + (col ? c : 0) * sc;
+  float* q = out + (int64_t(i) * tb + jb0) * tc + jc;
+  float v[kTexRows];
+#pragma unroll
+  for (int32_t t = 0; t < kTexRows; ++t) {
+    const int32_t b = jb0 + t - kk::kHaloLo;
+    v[t] = col && b >= 0 && b < nb ? p[b * sb] : 0.f;
+  }
+#pragma unroll
+  for (int32_t t = 0; t < kTexRows; ++t)
+    if (jb0 + t < tb) q[int64_t(t) * tc] = v[t];
+}
+
 // Projection texture: element (a, jv, ju) of a [n][rows+3][cols+3] float2
 // array = (P(a, jv-1, ju-1), P(a, jv, ju-1)), zero outside.
 // RESID: the texture of (proj - y) * R instead (the SIRT residual), with y
@@ -176,6 +203,34 @@ extern "C" int kk_volume_to_fp_texture(const float* vol,
                        reinterpret_cast<float2*>(tex) + off);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return kk::hip_fail(e, "fp_frame_kernel");
+    off += kk::frame_elems(shape, a);
+  }
+  return KK_OK;
+}
+
+extern "C" int kk_volume_to_fp_planes(const float* vol, const int32_t shape[3],
+                                      const int64_t st[3], int32_t mask,
+                                      float* planes, void* stream) {
+  if (vol == nullptr || planes == nullptr || shape == nullptr || st == nullptr)
+    return kk::fail(KK_ERR_INVALID, "kk_volume_to_fp_planes: null");
+  if (shape[0] <= 0 || shape[1] <= 0 || shape[2] <= 0 || mask <= 0 ||
+      mask > 7)
+    return kk::fail(KK_ERR_INVALID, "kk_volume_to_fp_planes: bad args");
+  int64_t off = 0;
+  for (int a = 0; a < 3; ++a) {
+    if (!(mask & (1 << a))) continue;
+    const int b = kk::kFrameB[a], c = kk::kFrameC[a];
+    if (shape[b] + kk::kHalo > 65535 || shape[a] > 65535)
+      return kk::fail(KK_ERR_UNSUPPORTED, "kk_volume_to_fp_planes: large");
+    const dim3 grid(unsigned((shape[c] + kk::kHalo + 255) / 256),
+                    unsigned((shape[b] + kk::kHalo + kTexRows - 1) /
+                             kTexRows),
+                    unsigned(shape[a]));
+    hipLaunchKernelGGL(fp_plane_kernel, grid, dim3(256), 0,
+                       static_cast<hipStream_t>(stream), vol, st[a], st[b],
+                       st[c], shape[b], shape[c], planes + off);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return kk::hip_fail(e, "fp_plane_kernel");
     off += kk::frame_elems(shape, a);
   }
   return KK_OK;

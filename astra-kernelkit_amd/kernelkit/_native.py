@@ -69,6 +69,14 @@ _SIGNATURES = {
                                              ctypes.c_int32]),
     "kk_volume_to_fp_texture": (ctypes.c_int, [_vp, _c_i32p, _c_i64p,
                                                ctypes.c_int32, _vp, _vp]),
+    "kk_fp_reads_planes": (ctypes.c_int32, [_vp, ctypes.c_int32,
+                                            ctypes.c_int32]),
+    "kk_fp_planes_elems": (ctypes.c_int64, [_c_i32p, ctypes.c_int32]),
+    "kk_volume_to_fp_planes": (ctypes.c_int, [_vp, _c_i32p, _c_i64p,
+                                              ctypes.c_int32, _vp, _vp]),
+    "kk_cone_fp_planes": (ctypes.c_int, [
+        _vp, _vp, _vp, _vp, ctypes.c_int32, _c_i64p, ctypes.c_int32,
+        ctypes.c_int32, ctypes.c_int32, _vp]),
     "kk_projections_to_bp_texture": (ctypes.c_int, [_vp, ctypes.c_int32,
                                                     ctypes.c_int32,
                                                     ctypes.c_int32, _c_i64p,
@@ -168,6 +176,9 @@ _SIGNATURES = {
     "kk_fp_table": (ctypes.c_int, [_c_f64p, ctypes.c_int32, _c_i32p,
                                    ctypes.c_int32, ctypes.c_int32, _c_i32p,
                                    _c_f64p, _vp, _c_i32p]),
+    "kk_fp_line_spacing": (ctypes.c_int, [
+        _c_f64p, ctypes.c_int32, _c_i32p, ctypes.c_int32, ctypes.c_int32,
+        _c_i32p, _c_f64p, _c_f64p]),
     "kk_bp_table": (ctypes.c_int, [_c_f64p, ctypes.c_int32, _vp]),
     "kk_filter_create": (ctypes.c_int, [ctypes.POINTER(_vp)]),
     "kk_filter_destroy": (ctypes.c_int, [_vp]),

@@ -218,10 +218,7 @@ class _SirtState:
         # projection into a buffer, then one coalesced pass (cheaper on
         # MI355X than the forward kernel's residual epilogue, which reads
         # y and R one detector row per lane)
-        _native.check(lib.kk_cone_fp(
-            fk._plan.ptr, _native._vp(self.xtex.ptr),
-            _native._vp(self.p.data_ptr()), _native.i64(self.p.stride()),
-            self.rows, self.cols, 0, st))
+        fk._launch(self.xtex, self.p, self.rows, self.cols, False, None)
         _native.check(lib.kk_residual_to_bp_texture(
             _native._vp(self.p.data_ptr()), _native.i64(self.p.stride()),
             _native._vp(self.y.data_ptr()), _native.i64(self.y.stride()),
@@ -242,7 +239,7 @@ class _SirtState:
             _native._vp(self.C.data_ptr()), _native.i64(self.C.stride()),
             mask_ptr, mask_st, self.lo, self.hi, self.clip_lo, self.clip_hi,
             None, 0, self.scale, st))
-        self.xtex.update(self.x)
+        self.xtex.update(self.x, planes=fk.reads_planes)
 
     def capture(self):
         """Record one iteration in a HIP graph (the library's own stream

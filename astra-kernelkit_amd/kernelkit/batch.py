@@ -61,7 +61,8 @@ class ConeBatch:
         projections = [as_device_array(p) for p in projections]
         self._check(projections, self.range_shapes, "projection")
         for op, v in zip(self.ops, vols):
-            op.projector.volume = v          # builds the frame textures
+            op.projector._vol_ref = v
+            op.projector._build_texture(pairs=True)
         key = tuple(p.data_ptr() for p in projections) + tuple(
             op.projector._texture.ptr for op in self.ops)
         if self._fp_cache is None or self._fp_cache[0] != key:

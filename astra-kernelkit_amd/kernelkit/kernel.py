@@ -142,28 +142,80 @@ class Texture:
 
 
 class VolumeTexture:
-    """Forward-projection layout of a volume: one slice-major frame of
-    (value, neighbour) float2 pairs with a zero halo per ray axis in
-    ``mask`` (bit a = world axis a); see ``include/kernelkit_hip.h``."""
+    """Forward-projection layout of a volume: per ray axis in ``mask`` (bit
+    a = world axis a) one slice-major frame with a zero halo, as float2
+    pairs (value, neighbour) for the general kernel, or as planes (plain
+    floats) for the kernel of column-coherent geometries; see
+    ``include/kernelkit_hip.h``.
+
+    ``update(..., planes=True)`` builds planes only.  :attr:`data` and
+    :attr:`ptr` are the pairs: they are made from the planes when first
+    asked for, and count as the texture's content from then on (a caller may
+    write them), until the next update.
+    """
 
     def __init__(self, world_shape, mask: int, device=None, like=None):
         self.world_shape = tuple(int(s) for s in world_shape)
         self.mask = int(mask)
-        n = _native.lib().kk_fp_texture_elems(_native.i32(self.world_shape),
-                                              self.mask)
-        if n < 0:
+        self._n = _native.lib().kk_fp_texture_elems(
+            _native.i32(self.world_shape), self.mask)
+        if self._n < 0:
             raise ValueError(f"bad volume shape {self.world_shape} or frame "
                              f"mask {mask}")
-        self.data = _alloc(n, like, device)
+        self._pairs = self._planes = None
+        self._holds_planes = False   # the content is in _planes, not _pairs
+        # buffers are allocated when first written, of the kind of `like`
+        self._like = like
+        if like is None:
+            self._pairs = self._like = _alloc(self._n, like, device)
+
+    def _buffer(self, n):
+        self._like = _alloc(n, self._like)
+        return self._like
+
+    @property
+    def data(self):
+        if self._pairs is None:
+            self._pairs = self._buffer(self._n)
+        if self._holds_planes:
+            self._planes_to_pairs()
+            self._holds_planes = False
+        return self._pairs
 
     @property
     def ptr(self):
         return self.data.data_ptr()
 
+    @property
+    def planes(self):
+        """Device address of the planes, None unless the texture's content
+        is held as such."""
+        return self._planes.data_ptr() if self._holds_planes else None
+
     def covers(self, mask: int) -> bool:
         return (int(mask) & ~self.mask) == 0
 
-    def update(self, volume, volume_axes=(0, 1, 2), stream=None) -> None:
+    def _planes_to_pairs(self):
+        # a frame of planes is a strided view of the volume in itself
+        off = 0
+        src = self._planes.data_ptr()
+        dst = self._pairs.data_ptr()
+        for a, (b, c) in enumerate(((1, 2), (0, 2), (1, 0))):
+            if not self.mask & (1 << a):
+                continue
+            tb = self.world_shape[b] + _native.HALO
+            tc = self.world_shape[c] + _native.HALO
+            st = [0, 0, 0]
+            st[a], st[b], st[c] = tb * tc, tc, 1
+            first = off + _native.HALO_LO * (tc + 1)
+            _native.check(_native.lib().kk_volume_to_fp_texture(
+                _native._vp(src + 4 * first), _native.i32(self.world_shape),
+                _native.i64(st), 1 << a, _native._vp(dst + 8 * off),
+                _native.stream_ptr()))
+            off += self.world_shape[a] * tb * tc
+
+    def update(self, volume, volume_axes=(0, 1, 2), stream=None,
+               planes: bool = False) -> None:
         """Copy ``volume`` (array axis k = world axis ``volume_axes[k]``)."""
         volume = as_device_array(volume)
         if not _is_f32(volume):
@@ -177,10 +229,19 @@ class VolumeTexture:
         if tuple(wshape) != self.world_shape:
             raise ValueError(f"volume of world shape {tuple(wshape)} does "
                              f"not match texture shape {self.world_shape}")
-        _native.check(_native.lib().kk_volume_to_fp_texture(
+        if planes:
+            if self._planes is None:
+                self._planes = self._buffer(self._n // 2)
+            build, dst = _native.lib().kk_volume_to_fp_planes, self._planes
+        else:
+            if self._pairs is None:
+                self._pairs = self._buffer(self._n)
+            build, dst = _native.lib().kk_volume_to_fp_texture, self._pairs
+        _native.check(build(
             _native._vp(volume.data_ptr()), _native.i32(self.world_shape),
-            _native.i64(wstride), self.mask, _native._vp(self.ptr),
+            _native.i64(wstride), self.mask, _native._vp(dst.data_ptr()),
             _native.stream_ptr(stream)))
+        self._holds_planes = bool(planes)
 
 
 class ProjectionTexture:

@@ -194,14 +194,21 @@ class RayDrivenConeFP(BaseKernel):
             self._plan.ptr, _native.f64_ptr(self._params), n, axes_ptr,
             rows, cols, _native.i32(vg.shape), _native.f64(vg.voxel_size)))
         self._uploaded_key = key
+        self._frame_mask = int(_native.lib().kk_fp_frame_mask(self._plan.ptr))
+        self._reads_planes = bool(_native.lib().kk_fp_reads_planes(
+            self._plan.ptr, rows, cols))
 
     @property
     def frame_mask(self) -> int:
         """Frames of the volume texture the uploaded parameters use (bit a:
         ray axis a), 0 before the first upload."""
-        if not self.is_compiled or self._uploaded_key is None:
-            return 0
-        return int(_native.lib().kk_fp_frame_mask(self._plan.ptr))
+        return 0 if self._uploaded_key is None else self._frame_mask
+
+    @property
+    def reads_planes(self) -> bool:
+        """Whether the uploaded parameters are of a geometry that the kernel
+        projects from planes (:class:`~kernelkit.kernel.VolumeTexture`)."""
+        return self._uploaded_key is not None and self._reads_planes
 
     def volume_texture(self, volume, volume_geometry: VolumeGeometry,
                        texture: VolumeTexture | None = None) -> VolumeTexture:
@@ -214,7 +221,7 @@ class RayDrivenConeFP(BaseKernel):
         if (texture is None or texture.world_shape != shape
                 or not texture.covers(mask)):
             texture = VolumeTexture(shape, mask, like=volume)
-        texture.update(volume, self._vol_axs)
+        texture.update(volume, self._vol_axs, planes=self.reads_planes)
         return texture
 
     def __call__(self, volume_texture, projection_geometry,
@@ -367,6 +374,13 @@ class RayDrivenConeFP(BaseKernel):
 
     def _launch_ptrs(self, tex: VolumeTexture, table, strides, rows, cols,
                      additive, stream):
+        if tex.planes is not None and self.reads_planes:
+            _native.check(_native.lib().kk_cone_fp_planes(
+                self._plan.ptr, _native._vp(tex.planes), None,
+                _native._vp(table.data_ptr()), self._proj_axs[0],
+                _native.i64(strides), rows, cols, 1 if additive else 0,
+                _native.stream_ptr(stream)))
+            return
         _native.check(_native.lib().kk_cone_fp_ptrs(
             self._plan.ptr, _native._vp(tex.ptr),
             _native._vp(table.data_ptr()), self._proj_axs[0],
@@ -376,6 +390,13 @@ class RayDrivenConeFP(BaseKernel):
     def _launch(self, tex: VolumeTexture, proj, rows, cols, additive,
                 stream):
         strides = _logical_strides(proj, self._proj_axs)
+        if tex.planes is not None and self.reads_planes:
+            _native.check(_native.lib().kk_cone_fp_planes(
+                self._plan.ptr, _native._vp(tex.planes),
+                _native._vp(proj.data_ptr()), None, 0, _native.i64(strides),
+                rows, cols, 1 if additive else 0,
+                _native.stream_ptr(stream)))
+            return
         _native.check(_native.lib().kk_cone_fp(
             self._plan.ptr, _native._vp(tex.ptr), _native._vp(proj.data_ptr()),
             _native.i64(strides), rows, cols, 1 if additive else 0,

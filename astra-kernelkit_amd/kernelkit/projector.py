@@ -218,7 +218,9 @@ class ForwardProjector(Projector):
         self._vol_ref = value
         self._build_texture()
 
-    def _build_texture(self):
+    def _build_texture(self, pairs: bool = False):
+        """Texture of the volume as the kernel reads it, or as ``pairs``
+        (the batch launches')."""
         value = self._vol_ref
         world = [0, 0, 0]
         for k, ax in enumerate(self.volume_axes):
@@ -229,7 +231,15 @@ class ForwardProjector(Projector):
                 or not tex.covers(mask)):
             tex = VolumeTexture(world, mask, like=as_device_array(value))
             self._texture = tex
-        tex.update(value, self.volume_axes)
+        tex.update(value, self.volume_axes,
+                   planes=self._K.reads_planes and not pairs)
+
+    def _update_params(self):
+        super()._update_params()
+        tex = getattr(self, "_texture", None)
+        if (tex is not None and tex.planes is not None
+                and not self._K.reads_planes):
+            tex.data  # noqa: B018 -- the set volume as the new kernel reads it
 
     @volume.deleter
     def volume(self):

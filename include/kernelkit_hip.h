@@ -94,6 +94,18 @@ int kk_volume_to_fp_texture(const float* vol, const int32_t vol_shape[3],
                             const int64_t vol_strides[3], int32_t frame_mask,
                             float* tex, void* stream);
 
+/* Planes: the FP texture's frames as plain floats (no pairs), which the
+ * launches of kk_cone_fp_planes read: for column-coherent geometries
+ * (circular orbits about z and the like) whose neighbouring detector rows
+ * sample the volume about a voxel apart or closer.  kk_fp_reads_planes says
+ * whether the plan's parameters with a rows x cols detector are such
+ * (1) or not (0).  Same frames and halo as the FP texture, half its size. */
+int32_t kk_fp_reads_planes(const kk_plan* plan, int32_t rows, int32_t cols);
+int64_t kk_fp_planes_elems(const int32_t vol_shape[3], int32_t frame_mask);
+int kk_volume_to_fp_planes(const float* vol, const int32_t vol_shape[3],
+                           const int64_t vol_strides[3], int32_t frame_mask,
+                           float* planes, void* stream);
+
 /* Projections -> BP texture (the projections setter, projector.py:503-556).
  * strides: element strides of (angle, row, col) in the source (any
  * projection_axes permutation or pitch). */
@@ -181,6 +193,13 @@ int kk_cone_fp_ptrs(const kk_plan* plan, const float* vol_tex,
                     const int64_t* ptrs, int32_t ptr_axis,
                     const int64_t proj_strides[3], int32_t rows,
                     int32_t cols, int32_t additive, void* stream);
+
+/* kk_cone_fp (ptrs NULL) or kk_cone_fp_ptrs (proj NULL) from planes:
+ * KK_ERR_UNSUPPORTED where kk_fp_reads_planes gives 0. */
+int kk_cone_fp_planes(const kk_plan* plan, const float* planes, float* proj,
+                      const int64_t* ptrs, int32_t ptr_axis,
+                      const int64_t proj_strides[3], int32_t rows,
+                      int32_t cols, int32_t additive, void* stream);
 
 /* Voxel-driven backprojection, all angles in one launch (cone_bp,
  * kernelkit/cuda/cone_bp.cu:35-159, kernels/cone_bp.py:292-302).
@@ -313,6 +332,14 @@ int kk_fp_table(const double* params, int32_t n_angles,
                 const int32_t* ray_axes, int32_t rows, int32_t cols,
                 const int32_t vol_shape[3], const double voxel_size[3],
                 void* out, int32_t* frame_mask);
+/* Host-only: bound and mean of the distance, in voxels along c, between the
+ * samples of neighbouring detector rows over the volume (out[0], out[1]);
+ * out[0] < 0 if the geometry is not column-coherent throughout.  What
+ * kk_fp_reads_planes decides on. */
+int kk_fp_line_spacing(const double* params, int32_t n_angles,
+                       const int32_t* ray_axes, int32_t rows, int32_t cols,
+                       const int32_t vol_shape[3], const double voxel_size[3],
+                       double out[2]);
 int kk_bp_table(const double* params, int32_t n_angles, void* out);
 
 /* ---- SIRT (kernelkit/algo.py:226-368) ---------------------------------- */
