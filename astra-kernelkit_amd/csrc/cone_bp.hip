@@ -26,6 +26,7 @@
 //   in groups of 4 x 4 x 4 neighbouring tiles, whose detector patches
 //   overlap, otherwise in runs of 16 tiles along x.
 #include <algorithm>
+#include <cmath>
 
 #include "kk_internal.h"
 
@@ -107,6 +108,51 @@ __device__ __forceinline__ bool run_inside(int32_t base, float lo,
   return b + lo >= 1.f && b + hi_off <= static_cast<float>(hi - 1);
 }
 
+// Tile (tx, ty, tz) of logical block id `bid`: groups of gx x gy x gz tiles
+// (x fastest inside), groups ordered x -> y -> z (the group sides divide the
+// tile counts; 1 x 1 x 1 is plain x -> y -> z order).
+__device__ __forceinline__ bool bp_decode(const BpArgs& A, int64_t bid,
+                                          int32_t& tx, int32_t& ty,
+                                          int32_t& tz) {
+  const int32_t gx = A.gx, gy = A.gy, gz = A.gz;
+  const int64_t inner = bid % (gx * gy * gz);
+  const int64_t outer = bid / (gx * gy * gz);
+  const int32_t ngx = (A.tiles_x + gx - 1) / gx;
+  const int32_t ngy = (A.tiles_y + gy - 1) / gy;
+  tx = static_cast<int32_t>(outer % ngx) * gx +
+       static_cast<int32_t>(inner % gx);
+  const int64_t o2 = outer / ngx;
+  ty = static_cast<int32_t>(o2 % ngy) * gy +
+       static_cast<int32_t>((inner / gx) % gy);
+  tz = static_cast<int32_t>(o2 / ngy) * gz +
+       static_cast<int32_t>(inner / (gx * gy));
+  return tx < A.tiles_x && ty < A.tiles_y && tz < A.tiles_z;
+}
+
+// Write the sum `acc` of voxel (ix, iy, iz) as the launch's mode says.
+__device__ __forceinline__ void bp_store(const BpArgs& A, int32_t ix,
+                                         int32_t iy, int32_t iz, float acc) {
+  const int64_t o = ix * A.vs0 + iy * A.vs1 + iz * A.vs2;
+  const float b = acc * A.scale;
+  if (A.mode == 0) {
+    A.out[o] = b;
+  } else if (A.mode == 1) {
+    A.out[o] += b;
+  } else {
+    float x = A.out[o] - A.C[ix * A.cs0 + iy * A.cs1 + iz * A.cs2] * b;
+    if (A.mask) x *= A.mask[ix * A.ms0 + iy * A.ms1 + iz * A.ms2];
+    if (A.clip_lo) x = fmaxf(x, A.lo);
+    if (A.clip_hi) x = fminf(x, A.hi);
+    A.out[o] = x;
+    for (int f = 0; f < A.n_frames; ++f) {
+      const int64_t q = A.fr_origin[f] + ix * A.fr_s0[f] +
+                        iy * A.fr_s1[f] + iz * A.fr_s2[f];
+      A.xtex[q] = x;
+      A.xtex[q + A.fr_dual[f]] = x;
+    }
+  }
+}
+
 // One workgroup's tile (16 x 16 columns of K voxels) of logical block id
 // `bid`.  TABLE_IN_MEMORY: the angle table pointer was read from a
 // descriptor (batch kernel), so each record is copied through
@@ -114,22 +160,8 @@ __device__ __forceinline__ bool run_inside(int32_t base, float lo,
 template <int K, bool TABLE_IN_MEMORY>
 __device__ __forceinline__ void bp_tile(const kk::BpAngle* __restrict__ tab,
                                         const BpArgs& A, int64_t bid) {
-  // groups of gx x gy x gz tiles (x fastest inside), groups ordered
-  // x -> y -> z (the group sides divide the tile counts; 1 x 1 x 1 is
-  // plain x -> y -> z order)
-  const int32_t gx = A.gx, gy = A.gy, gz = A.gz;
-  const int64_t inner = bid % (gx * gy * gz);
-  const int64_t outer = bid / (gx * gy * gz);
-  const int32_t ngx = (A.tiles_x + gx - 1) / gx;
-  const int32_t ngy = (A.tiles_y + gy - 1) / gy;
-  const int32_t tx = static_cast<int32_t>(outer % ngx) * gx +
-                     static_cast<int32_t>(inner % gx);
-  const int64_t o2 = outer / ngx;
-  const int32_t ty = static_cast<int32_t>(o2 % ngy) * gy +
-                     static_cast<int32_t>((inner / gx) % gy);
-  const int32_t tz = static_cast<int32_t>(o2 / ngy) * gz +
-                     static_cast<int32_t>(inner / (gx * gy));
-  if (tx >= A.tiles_x || ty >= A.tiles_y || tz >= A.tiles_z) return;
+  int32_t tx, ty, tz;
+  if (!bp_decode(A, bid, tx, ty, tz)) return;
   const int32_t ix = tx * 16 + int32_t(threadIdx.x & 15);
   const int32_t iy = ty * 16 + int32_t(threadIdx.x >> 4);
   const int32_t iz0 = tz * K;
@@ -333,30 +365,10 @@ __device__ __forceinline__ void bp_tile(const kk::BpAngle* __restrict__ tab,
     }
   }
 
-  const int64_t base = ix * A.vs0 + iy * A.vs1;
 #pragma unroll
   for (int k = 0; k < K; ++k) {
-    const int32_t iz = iz0 + k;
-    if (iz >= A.nz) break;
-    const int64_t o = base + iz * A.vs2;
-    const float b = acc[k] * A.scale;
-    if (A.mode == 0) {
-      A.out[o] = b;
-    } else if (A.mode == 1) {
-      A.out[o] += b;
-    } else {
-      float x = A.out[o] - A.C[ix * A.cs0 + iy * A.cs1 + iz * A.cs2] * b;
-      if (A.mask) x *= A.mask[ix * A.ms0 + iy * A.ms1 + iz * A.ms2];
-      if (A.clip_lo) x = fmaxf(x, A.lo);
-      if (A.clip_hi) x = fminf(x, A.hi);
-      A.out[o] = x;
-      for (int f = 0; f < A.n_frames; ++f) {
-        const int64_t q = A.fr_origin[f] + ix * A.fr_s0[f] +
-                          iy * A.fr_s1[f] + iz * A.fr_s2[f];
-        A.xtex[q] = x;
-        A.xtex[q + A.fr_dual[f]] = x;
-      }
-    }
+    if (iz0 + k >= A.nz) break;
+    bp_store(A, ix, iy, iz0 + k, acc[k]);
   }
 }
 
@@ -370,6 +382,228 @@ __global__ __launch_bounds__(256, bp_min_blocks(K)) void cone_bp_kernel(
     const kk::BpAngle* __restrict__ tab, BpArgs A) {
   bp_tile<K, false>(tab, A,
                     kk_xcd_remap(blockIdx.x, A.total_blocks, A.xcd_group));
+}
+
+
+// ---- circular orbits: detector patches in LDS -----------------------------
+//
+// A workgroup is a tile of 16 x 16 columns of K voxels.  Per angle it stages
+// the detector patch that the tile projects onto in LDS (from planes: the
+// projections column-major, each column followed by zeros), and every update
+// reads its four taps there: two paired reads.  The next angle's patch is on
+// its way into registers meanwhile.  Patches of 64 angles are located at a
+// time, one angle per lane, from the tile's corners.  Reads outside the
+// detector become zeros by the buffer descriptor (columns) and the zeros
+// between columns (rows), so nothing is clamped per update.
+//
+// What bounds it (MI355X): a gather from global memory costs a CU 16 cycles
+// per 64 updates (it took 20 with 16.5 vector instructions beside), the two
+// LDS reads 10, the patch ~3, vector issue ~10.  Measured: 512^3 / 720
+// 50.8 -> 38.0 ms, 256^3 / 360 3.2 -> 2.3 ms, 128^3 / 180 0.25 -> 0.18 ms.
+// LDS is 72% busy, vector issue about as much.
+// * Bank conflicts decide the layout: a wavefront is 8 x 8 columns and the
+//   patch pitch 64 + 6 words (512^3: 38.1 ms; pitches 64 + 1, 2, 3, 4, 5, 8,
+//   11 and 13: 47.5, 39.1, 37.9, 41.6, 38.1, 59.9, 46.0 and 42.5 ms, and at
+//   256^3 64 + 6 is 3% ahead of 64 + 3; a wavefront of 16 x 4 columns: 41).
+// * K = 16: runs of 8 and 24 took 71 and 38.9 ms (at 256^3 4.0 and 2.8).
+// * SPLIT > 1: the angles are dealt to that many groups of 256 threads and
+//   the groups' sums added at the end, where the tiles alone leave the chip
+//   idle (128^3: 0.244, 0.179 and 0.194 ms with 1, 2 and 4 parts).
+//
+// The row of an update is 64-bit fixed point (32 fraction bits), stepped by
+// one 64-bit add per voxel.
+constexpr int kPatchRun = 16;                  // K
+constexpr int kPatchLanes = 64;                // rows per patch column
+constexpr int kPatchPitch = kPatchLanes + 6;   // LDS words per column
+constexpr int kPatchCols = 64;
+constexpr int kPatchGap = KK_PLANE_GAP;        // zero rows after a column
+static_assert(kPatchGap >= kPatchLanes, "a patch column ends in its own gap");
+
+// x as 64-bit fixed point with 32 fraction bits, |x| < 2^19: the mantissa of
+// x + 1.5 * 2^20.  The high word carries kFixedHi besides.
+constexpr double kFixedMagic = 1572864.0;
+constexpr uint32_t kFixedHi = 0x41380000u;
+__device__ __forceinline__ uint64_t fixed_bits(double x) {
+  return __builtin_bit_cast(uint64_t, x + kFixedMagic);
+}
+
+template <int K, int SPLIT>
+__global__ __launch_bounds__(256 * SPLIT, 5) void cone_bp_patch_kernel(
+    const kk::BpAngle* __restrict__ tab, BpArgs A) {
+  typedef __attribute__((address_space(3))) const float* lds_ptr;
+  __shared__ float patch_s[SPLIT][kPatchCols * kPatchPitch];
+  int32_t tx, ty, tz;
+  if (!bp_decode(A, kk_xcd_remap(blockIdx.x, A.total_blocks, A.xcd_group), tx,
+                 ty, tz))
+    return;  // the whole workgroup
+  const int32_t lane = int32_t(threadIdx.x) & 63;
+  const int32_t sub = __builtin_amdgcn_readfirstlane(int32_t(threadIdx.x) >> 8);
+  const int32_t wave =
+      __builtin_amdgcn_readfirstlane((int32_t(threadIdx.x) >> 6) & 3);
+  const int32_t tid = int32_t(threadIdx.x) & 255;
+  // a wavefront is 8 x 8 columns
+  const int32_t ix = tx * 16 + (tid & 7) + ((tid >> 3) & 8);
+  const int32_t iy = ty * 16 + ((tid >> 3) & 7) + ((tid >> 4) & 8);
+  const int32_t iz0 = tz * K;
+  // columns outside the volume repeat its last ones (not written)
+  const double X = min(ix, A.nx - 1) - 0.5 * A.nx + 0.5;
+  const double Y = min(iy, A.ny - 1) - 0.5 * A.ny + 0.5;
+  const double Z0 = iz0 - 0.5 * A.nz + 0.5;
+  float* patch = patch_s[sub];
+  const uint32_t patch_at = __builtin_amdgcn_readfirstlane(
+      static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr)patch)));
+  const int32_t pitch = static_cast<int32_t>(A.trb);  // bytes per column
+
+  float acc[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) acc[k] = 0.f;
+  // patches of 64 of this part's angles at a time, one per lane: origin
+  // column and row, number of columns (0: the tile projects off the detector)
+  int32_t pc = 0, pr = 0, pn = 0;
+  auto bounds = [&](int32_t a) {
+    pn = 0;
+    if (a >= A.n_angles) return;
+    const kk::BpAngle& P = tab[a];
+    // (from integers, here: kept in registers they would cost the loop)
+    int32_t ex = tx * 16, ey = ty * 16;
+    asm volatile("" : "+v"(ex), "+v"(ey));
+    double ul = 1e30, uh = -1e30, vl = 1e30, vh = -1e30;
+#pragma unroll 1
+    for (int e = 0; e < 4; ++e) {
+      const double x =
+          min(ex + (e & 1 ? 15 : 0), A.nx - 1) - 0.5 * A.nx + 0.5;
+      const double y =
+          min(ey + (e & 2 ? 15 : 0), A.ny - 1) - 0.5 * A.ny + 0.5;
+      const double d = fma(y, P.dy, fma(x, P.dx, P.dw));
+      const double r =
+          refine_rcp(d, __builtin_amdgcn_rcpf(static_cast<float>(d)));
+      const double u = fma(y, P.nuy, fma(x, P.nux, P.nuw)) * r;
+      const double v = fma(Z0, P.nvz, fma(y, P.nvy, fma(x, P.nvx, P.nvw))) * r;
+      const double w = fma(static_cast<double>(K - 1), P.nvz * r, v);
+      ul = fmin(ul, u);
+      uh = fmax(uh, u);
+      vl = fmin(vl, fmin(v, w));
+      vh = fmax(vh, fmax(v, w));
+    }
+    // (without the halo that the padded coordinates count; 1e-6 covers the
+    // rounding of the threads' own coordinates)
+    const double c0 = floor(ul - 1e-6) - kk::kHaloLo;
+    const double r0 = floor(vl - 1e-6) - kk::kHaloLo;
+    const double c1 = floor(uh + 1e-6) - kk::kHaloLo + 1;
+    const double r1 = floor(vh + 1e-6) - kk::kHaloLo + 1;
+    if (c1 < 0 || c0 >= A.cols || r1 < 0 || r0 >= A.rows) return;
+    pc = static_cast<int32_t>(c0);
+    pr = static_cast<int32_t>(r0);
+    pn = static_cast<int32_t>(c1 - c0) + 1;
+  };
+  // (the compiler would otherwise wait for all loads wherever the registers
+  // of these are used again)
+  auto settle = [] { __builtin_amdgcn_s_waitcnt(0x0f70); };  // vmcnt(0)
+  constexpr int NS = kPatchCols / 4;
+  float st[NS];
+  int32_t c0 = 0, r0 = 0, nc = 0;   // the staged patch
+  auto stage = [&](int32_t a, int32_t l) {
+    c0 = __builtin_amdgcn_readlane(pc, l);
+    r0 = __builtin_amdgcn_readlane(pr, l);
+    nc = __builtin_amdgcn_readlane(pn, l);
+    if (nc == 0) return;
+    const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<char*>(A.tex) + static_cast<uint64_t>(a) * A.tab_b, 0,
+        static_cast<int32_t>(A.tab_b), 0x00020000);
+    uint32_t o = static_cast<uint32_t>((c0 + wave) * pitch + (r0 + lane) * 4);
+#pragma unroll
+    for (int j = 0; j < NS; ++j) {
+      if (wave + 4 * j >= nc) break;
+      asm volatile("" : "+v"(o));
+      st[j] = __builtin_bit_cast(
+          float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, o, 0, 0));
+      o += 4 * pitch;
+    }
+  };
+  const int32_t mine = (A.n_angles - sub + SPLIT - 1) / SPLIT;
+  const int32_t most = (A.n_angles + SPLIT - 1) / SPLIT;
+  bounds(sub + lane * SPLIT);
+  settle();
+  stage(sub, 0);
+  for (int32_t q = 0; q < most; ++q) {
+    const int32_t a = sub + q * SPLIT;
+    const int32_t cc = c0, cr = r0, n = q < mine ? nc : 0;
+    __syncthreads();  // the previous patch has been read
+#pragma unroll
+    for (int j = 0; j < NS; ++j) {
+      if (wave + 4 * j >= n) break;
+      patch[(wave + 4 * j) * kPatchPitch + lane] = st[j];
+    }
+    __syncthreads();
+    if (q + 1 < mine) {
+      if (((q + 1) & 63) == 0) {
+        bounds(a + SPLIT + lane * SPLIT);
+        settle();
+      }
+      stage(a + SPLIT, (q + 1) & 63);
+    }
+    if (n == 0) continue;
+    const kk::BpAngle& P = tab[a];
+    const double den = fma(Y, P.dy, fma(X, P.dx, P.dw));
+    const double nu = fma(Y, P.nuy, fma(X, P.nux, P.nuw));
+    const double nv = fma(Y, P.nvy, fma(X, P.nvx, P.nvw));
+    const float rf = __builtin_amdgcn_rcpf(static_cast<float>(den));
+    const double r = refine_rcp(den, rf);
+    const double u = fma(nu, r, -static_cast<double>(cc + kk::kHaloLo));
+    uint32_t iu;
+    float fu;
+    kk_split_nonneg(u, iu, fu);
+    const double v0 =
+        fma(fma(Z0, P.nvz, nv), r, -static_cast<double>(cr + kk::kHaloLo));
+    uint64_t V = fixed_bits(v0);
+    const uint64_t G = fixed_bits(P.nvz * r) -
+                       (static_cast<uint64_t>(kFixedHi) << 32);
+    const float w = rf * rf;
+    const uint32_t at =
+        patch_at + __umul24(iu, kPatchPitch * 4u) - (kFixedHi << 2);
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      uint32_t p;  // one shift-add of the row (not a 64-bit shift)
+      asm("v_lshl_add_u32 %0, %1, 2, %2"
+          : "=v"(p)
+          : "v"(static_cast<uint32_t>(V >> 32)), "v"(at));
+      const lds_ptr t = (lds_ptr)p;
+      const float l0 = fmaf(fu, t[kPatchPitch] - t[0], t[0]);
+      const float l1 = fmaf(fu, t[kPatchPitch + 1] - t[1], t[1]);
+      const float fv = static_cast<float>(static_cast<uint32_t>(V)) * 0x1p-32f;
+      acc[k] = fmaf(w, fmaf(fv, l1 - l0, l0), acc[k]);
+      V += G;
+      // (four voxels' reads in flight, within the register cap)
+      if (k % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+
+  if constexpr (SPLIT == 1) {
+    if (ix >= A.nx || iy >= A.ny) return;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      if (iz0 + k >= A.nz) break;
+      bp_store(A, ix, iy, iz0 + k, acc[k]);
+    }
+  } else {
+    // the parts' sums, in order; every part writes K / SPLIT of the run
+    static_assert(K % SPLIT == 0 && 256 * K <= kPatchCols * kPatchPitch,
+                  "a part's sums take its patch");
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < K; ++k) patch[k * 256 + tid] = acc[k];
+    __syncthreads();
+    if (ix >= A.nx || iy >= A.ny) return;
+#pragma unroll
+    for (int k = 0; k < K / SPLIT; ++k) {
+      const int32_t z = sub * (K / SPLIT) + k;
+      if (iz0 + z >= A.nz) break;
+      float sum = patch_s[0][z * 256 + tid];
+#pragma unroll
+      for (int p = 1; p < SPLIT; ++p) sum += patch_s[p][z * 256 + tid];
+      bp_store(A, ix, iy, iz0 + z, sum);
+    }
+  }
 }
 
 struct BpItem {
@@ -683,6 +917,170 @@ int sirt_update_spec(BpSpec& S, const kk_plan* plan, const float* res_tex,
 }
 
 }  // namespace kk
+
+namespace {
+
+// Largest |du/dx| + |du/dy| (and v alike) over the volume's columns for a
+// coordinate f = num / den of affine forms in (x, y): df/dx = ((nx dy - ny dx)
+// y + nx dw - nw dx) / den^2 is monotonic in x and has at most one extremum in
+// y between the ends (df/dy alike).
+double steepest(double nx, double ny, double nw, double dx, double dy,
+                double dw, double hx, double hy) {
+  auto partial = [&](double n1, double n2, double d1, double d2, double h1,
+                     double h2) {  // d/dx1, (x1, x2) in [-h1, h1] x [-h2, h2]
+    const double A = n1 * d2 - n2 * d1, B = n1 * dw - nw * d1;
+    double most = 0.0;
+    for (int e = 0; e < 2; ++e) {
+      const double c = dw + d1 * (e ? h1 : -h1);
+      const double at[3] = {-h2, h2,
+                            A * d2 != 0.0 ? (A * c - 2.0 * d2 * B) / (d2 * A)
+                                          : 0.0};
+      for (double x2 : at) {
+        if (!(std::fabs(x2) <= h2)) continue;
+        const double den = c + d2 * x2;
+        most = std::fmax(most, std::fabs((A * x2 + B) / (den * den)));
+      }
+    }
+    return most;
+  };
+  return partial(nx, ny, dx, dy, hx, hy) + partial(ny, nx, dy, dx, hy, hx);
+}
+
+// Bounds of the columns and rows of the patch of any tile at any angle
+// (ext[0], ext[1]), for circular orbits (the host table in `tab`); false for
+// other geometries, and where a denominator may vanish over the volume or
+// coordinates leave the kernel's ranges.
+bool patch_extent(const std::vector<kk::BpAngle>& tab, const int32_t shape[3],
+                  double ext[2]) {
+  ext[0] = ext[1] = 0.0;
+  if (tab.empty()) return false;
+  for (int t = 0; t < 3; ++t)
+    if (shape[t] <= 0 || shape[t] > 65536) return false;
+  const double hx = 0.5 * (shape[0] - 1), hy = 0.5 * (shape[1] - 1);
+  const double hz = 0.5 * shape[2] + kPatchRun;
+  for (const kk::BpAngle& e : tab) {
+    if (e.fast != 1) return false;
+    double least = INFINITY, most = 0.0;
+    bool pos = true, neg = true;
+    for (int k = 0; k < 4; ++k) {
+      const double x = k & 1 ? hx : -hx, y = k & 2 ? hy : -hy;
+      const double d = e.dw + e.dx * x + e.dy * y;
+      pos = pos && d > 0.0;
+      neg = neg && d < 0.0;
+      least = std::fmin(least, std::fabs(d));
+      most = std::fmax(most, std::fabs(d));
+      const double u = (e.nuw + e.nux * x + e.nuy * y) / d;
+      const double v = (std::fabs(e.nvw + e.nvx * x + e.nvy * y) +
+                        hz * std::fabs(e.nvz)) / std::fabs(d);
+      if (!(std::fabs(u) < 1e5) || !(v < 1e5)) return false;
+    }
+    if (!(pos || neg) || !(least > 1e-6 * most)) return false;
+    const double du = steepest(e.nux, e.nuy, e.nuw, e.dx, e.dy, e.dw, hx, hy);
+    double dv = 0.0;
+    for (int k = 0; k < 2; ++k)
+      dv = std::fmax(dv, steepest(e.nvx, e.nvy,
+                                  e.nvw + (k ? hz : -hz) * e.nvz, e.dx, e.dy,
+                                  e.dw, hx, hy));
+    const double run = (kPatchRun - 1) * std::fabs(e.nvz) / least;
+    // 15 voxels along x and y; three texels for the ends' floors and the
+    // second tap, and rounding
+    ext[0] = std::fmax(ext[0], 15.0 * du + 3.01);
+    ext[1] = std::fmax(ext[1], 15.0 * dv + run + 3.01);
+  }
+  return true;
+}
+
+// Whether every patch fits kPatchCols columns and kPatchLanes rows.  The
+// answer for the last detector and volume is kept with the plan.
+bool patches_fit(const kk_plan_s& plan, int32_t rows, int32_t cols,
+                 const int32_t shape[3]) {
+  if (rows <= 0 || cols <= 0) return false;
+  if (int64_t(rows + kPatchGap) * cols * 4 >= (int64_t(1) << 31)) return false;
+  const std::lock_guard<std::mutex> hold(plan.bp_patch_lock);
+  if (plan.bp_patch_fits < 0 ||
+      !std::equal(shape, shape + 3, plan.bp_patch_shape)) {
+    double ext[2];
+    const bool ok = patch_extent(plan.bp_host, shape, ext);
+    plan.bp_patch_fits =
+        ok && ext[0] <= kPatchCols && ext[1] <= kPatchLanes ? 1 : 0;
+    std::copy(shape, shape + 3, plan.bp_patch_shape);
+  }
+  return plan.bp_patch_fits == 1;
+}
+
+int launch_bp_planes(const kk::BpSpec& S, hipStream_t stream) {
+  BpArgs A;
+  const int rc = make_bp_args(S, kPatchRun, A);
+  if (rc != KK_OK) return rc;
+  if (!patches_fit(*S.plan, S.rows, S.cols, S.shape))
+    return kk::fail(KK_ERR_UNSUPPORTED,
+                    "kk_cone_bp_planes: not a geometry for planes (see "
+                    "kk_bp_reads_planes)");
+  const int64_t pitch = int64_t(S.rows + kPatchGap) * 4;
+  A.trb = uint32_t(pitch);
+  A.tab_b = uint32_t(pitch * S.cols);
+  // parts so that a CU (of 256) holds at least four wavefronts per SIMD
+  const int64_t per_cu = (A.total_blocks + 255) / 256;
+  const dim3 grid(unsigned(A.total_blocks));
+  if (per_cu >= 4)
+    hipLaunchKernelGGL((cone_bp_patch_kernel<kPatchRun, 1>), grid, dim3(256),
+                       0, stream, S.plan->bp, A);
+  else if (per_cu >= 2)
+    hipLaunchKernelGGL((cone_bp_patch_kernel<kPatchRun, 2>), grid, dim3(512),
+                       0, stream, S.plan->bp, A);
+  else
+    hipLaunchKernelGGL((cone_bp_patch_kernel<kPatchRun, 4>), grid, dim3(1024),
+                       0, stream, S.plan->bp, A);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return kk::hip_fail(e, "cone_bp_patch_kernel");
+  return KK_OK;
+}
+
+}  // namespace
+
+extern "C" int32_t kk_bp_reads_planes(const kk_plan* plan, int32_t rows,
+                                      int32_t cols, const int32_t shape[3]) {
+  if (plan == nullptr || !plan->bp_set || shape == nullptr) return 0;
+  return patches_fit(*plan, rows, cols, shape) ? 1 : 0;
+}
+
+extern "C" int kk_bp_patch_extent(const double* params, int32_t n,
+                                  const int32_t shape[3], double out[2]) {
+  if (shape == nullptr || out == nullptr)
+    return kk::fail(KK_ERR_INVALID, "kk_bp_patch_extent: null");
+  std::vector<kk::BpAngle> tab;
+  const int rc = kk::bp_table_host(params, n, tab);
+  if (rc != KK_OK) return rc;
+  if (!patch_extent(tab, shape, out)) out[0] = out[1] = -1.0;
+  return KK_OK;
+}
+
+extern "C" int kk_cone_bp_planes(const kk_plan* plan, const float* planes,
+                                 int32_t n_angles, int32_t rows, int32_t cols,
+                                 float* vol, const int32_t shape[3],
+                                 const int64_t vs[3], float output_scale,
+                                 int32_t additive, void* stream) {
+  kk::BpSpec S;
+  const int rc = kk::bp_spec(S, plan, planes, n_angles, rows, cols, vol,
+                             shape, vs, output_scale, additive);
+  if (rc != KK_OK) return rc;
+  return launch_bp_planes(S, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int kk_sirt_bp_update_planes(
+    const kk_plan* plan, const float* planes, int32_t n_angles, int32_t rows,
+    int32_t cols, float* x, const int32_t shape[3], const int64_t xs[3],
+    const float* C, const int64_t cs[3], const float* mask,
+    const int64_t ms[3], float lo, float hi, int32_t clip_lo, int32_t clip_hi,
+    float output_scale, void* stream) {
+  kk::BpSpec S;
+  const int rc = kk::sirt_update_spec(S, plan, planes, n_angles, rows, cols, x,
+                                      shape, xs, C, cs, mask, ms, lo, hi,
+                                      clip_lo, clip_hi, nullptr, 0,
+                                      output_scale);
+  if (rc != KK_OK) return rc;
+  return launch_bp_planes(S, static_cast<hipStream_t>(stream));
+}
 
 extern "C" int kk_cone_bp(const kk_plan* plan, const float* proj_tex,
                           int32_t n_angles, int32_t rows, int32_t cols,

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <mutex>
 #include <vector>
 
 #include "kernelkit_hip.h"
@@ -172,6 +173,8 @@ int sirt_update_spec(BpSpec& S, const kk_plan_s* plan, const float* res_tex,
                      const int64_t ms[3], float lo, float hi,
                      int32_t clip_lo, int32_t clip_hi, float* x_tex,
                      int32_t x_tex_mask, float scale);
+// The host table of kk_set_params_bp's parameters (plan.hip).
+int bp_table_host(const double* params, int32_t n, std::vector<BpAngle>& tab);
 // FpSpec of kk_cone_fp / kk_sirt_fp_residual.
 int fp_spec(FpSpec& S, const kk_plan_s* plan, const float* tex, float* out,
             const int64_t os[3], int32_t rows, int32_t cols,
@@ -218,6 +221,12 @@ struct kk_plan_s {
   int32_t bp_n = 0, bp_cap = 0;
   bool bp_set = false;
   bool bp_all_circ = false;  // every angle on the circular path (fast == 1)
+  std::vector<kk::BpAngle> bp_host;  // host copy of the table
+  // whether the patch kernel's tiles fit their patches, for one volume shape
+  // (-1: not looked at since the parameters were set)
+  mutable std::mutex bp_patch_lock;
+  mutable int32_t bp_patch_fits = -1;
+  mutable int32_t bp_patch_shape[3] = {0, 0, 0};
 };
 
 // Map a hardware workgroup id to a logical tile id such that, inside every

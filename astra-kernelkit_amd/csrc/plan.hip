@@ -369,6 +369,11 @@ static int build_bp_table(const double* params, int32_t n,
   return KK_OK;
 }
 
+int kk::bp_table_host(const double* params, int32_t n,
+                      std::vector<kk::BpAngle>& tab) {
+  return build_bp_table(params, n, tab);
+}
+
 extern "C" int kk_set_params_bp(kk_plan* plan, const double* params,
                                 int32_t n) {
   if (plan == nullptr)
@@ -386,6 +391,11 @@ extern "C" int kk_set_params_bp(kk_plan* plan, const double* params,
   plan->bp_all_circ = true;
   for (int32_t k = 0; k < n; ++k)
     plan->bp_all_circ = plan->bp_all_circ && tab[k].fast == 1;
+  {
+    const std::lock_guard<std::mutex> hold(plan->bp_patch_lock);
+    plan->bp_host.swap(tab);
+    plan->bp_patch_fits = -1;
+  }
   plan->bp_set = true;
   return KK_OK;
 }
@@ -413,6 +423,11 @@ extern "C" int64_t kk_bp_texture_elems(int32_t n, int32_t rows,
                                        int32_t cols) {
   if (n <= 0 || rows <= 0 || cols <= 0) return -1;
   return 2 * int64_t(n) * (rows + kk::kHalo) * (cols + kk::kHalo);
+}
+
+extern "C" int64_t kk_bp_planes_elems(int32_t n, int32_t rows, int32_t cols) {
+  if (n <= 0 || rows <= 0 || cols <= 0) return -1;
+  return int64_t(n) * cols * (rows + KK_PLANE_GAP);
 }
 
 extern "C" int kk_fp_table(const double* params, int32_t n,

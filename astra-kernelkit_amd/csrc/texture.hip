@@ -117,6 +117,46 @@ __global__ __launch_bounds__(256) void bp_tex_kernel(
   }
 }
 
+// Projection planes: element (a, c, r) of a [n][cols][rows + KK_PLANE_GAP]
+// float array = P(a, r, c), zeros after each column (the layout of
+// cone_bp_patch_kernel), through an LDS tile: both sides coalesced.  RESID:
+// of the residual (proj - y) * R.
+constexpr int kPlaneGap = KK_PLANE_GAP;
+template <bool RESID>
+__global__ __launch_bounds__(256) void bp_plane_kernel(
+    const float* __restrict__ proj, int64_t s0, int64_t s1, int64_t s2,
+    int32_t rows, int32_t cols, float* __restrict__ out, ResidArgs res) {
+  __shared__ float tile[64][65];
+  const int32_t c0 = blockIdx.x * 64, r0 = blockIdx.y * 64;
+  const int32_t a = blockIdx.z;
+  const int32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int32_t c = c0 + lane;
+  float v[16];
+#pragma unroll
+  for (int t = 0; t < 16; ++t) {
+    const int32_t r = r0 + 4 * t + w;
+    v[t] = 0.f;
+    if (r < rows && c < cols) {
+      v[t] = proj[a * s0 + r * s1 + c * s2];
+      if constexpr (RESID)
+        v[t] = (v[t] - res.y[a * res.y0 + r * res.y1 + c * res.y2]) *
+               res.R[a * res.r0 + r * res.r1 + c * res.r2];
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < 16; ++t) tile[4 * t + w][lane] = v[t];
+  __syncthreads();
+  const int32_t pitch = rows + kPlaneGap;
+  const int32_t r = r0 + lane;
+  if (r >= pitch) return;
+  float* o = out + (int64_t(a) * cols + c0) * pitch + r;
+#pragma unroll
+  for (int t = 0; t < 16; ++t) {
+    const int32_t k = 4 * t + w;
+    if (c0 + k < cols) o[int64_t(k) * pitch] = tile[lane][k];
+  }
+}
+
 // Many texture builds in one launch: a grid-stride loop over the jobs'
 // tiles (one image's band of kTexRows texture rows by 256 columns, column
 // chunks fastest), each found by binary search over the jobs' first tile
@@ -259,6 +299,27 @@ extern "C" int kk_projections_to_bp_texture(const float* proj, int32_t n,
   return KK_OK;
 }
 
+extern "C" int kk_projections_to_bp_planes(const float* proj, int32_t n,
+                                           int32_t rows, int32_t cols,
+                                           const int64_t st[3], float* planes,
+                                           void* stream) {
+  if (proj == nullptr || planes == nullptr || st == nullptr)
+    return kk::fail(KK_ERR_INVALID, "kk_projections_to_bp_planes: null");
+  if (n <= 0 || rows <= 0 || cols <= 0)
+    return kk::fail(KK_ERR_INVALID, "kk_projections_to_bp_planes: shape");
+  if (rows + kk::kHalo > 65535 || n > 65535)
+    return kk::fail(KK_ERR_UNSUPPORTED,
+                    "kk_projections_to_bp_planes: too large");
+  const dim3 grid(unsigned((cols + 63) / 64),
+                  unsigned((rows + kPlaneGap + 63) / 64), unsigned(n));
+  hipLaunchKernelGGL(bp_plane_kernel<false>, grid, dim3(256), 0,
+                     static_cast<hipStream_t>(stream), proj, st[0], st[1],
+                     st[2], rows, cols, planes, ResidArgs{});
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return kk::hip_fail(e, "bp_plane_kernel");
+  return KK_OK;
+}
+
 extern "C" int kk_residual_to_bp_texture(
     const float* proj, const int64_t ps[3], const float* y,
     const int64_t ys[3], const float* R, const int64_t rs[3],
@@ -280,6 +341,29 @@ extern "C" int kk_residual_to_bp_texture(
                      ps[2], rows, cols, reinterpret_cast<float2*>(tex), res);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return kk::hip_fail(e, "bp_tex_kernel");
+  return KK_OK;
+}
+
+extern "C" int kk_residual_to_bp_planes(
+    const float* proj, const int64_t ps[3], const float* y,
+    const int64_t ys[3], const float* R, const int64_t rs[3],
+    int32_t n_angles, int32_t rows, int32_t cols, float* planes,
+    void* stream) {
+  if (proj == nullptr || ps == nullptr || y == nullptr || ys == nullptr ||
+      R == nullptr || rs == nullptr || planes == nullptr)
+    return kk::fail(KK_ERR_INVALID, "kk_residual_to_bp_planes: null");
+  if (n_angles <= 0 || rows <= 0 || cols <= 0)
+    return kk::fail(KK_ERR_INVALID, "kk_residual_to_bp_planes: bad sizes");
+  if (n_angles > 65535 || rows + kk::kHalo > 65535)
+    return kk::fail(KK_ERR_UNSUPPORTED, "kk_residual_to_bp_planes: too large");
+  const dim3 grid(unsigned((cols + 63) / 64),
+                  unsigned((rows + kPlaneGap + 63) / 64), unsigned(n_angles));
+  const ResidArgs res{y, ys[0], ys[1], ys[2], R, rs[0], rs[1], rs[2]};
+  hipLaunchKernelGGL(bp_plane_kernel<true>, grid, dim3(256), 0,
+                     static_cast<hipStream_t>(stream), proj, ps[0], ps[1],
+                     ps[2], rows, cols, planes, res);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return kk::hip_fail(e, "bp_plane_kernel");
   return KK_OK;
 }
 

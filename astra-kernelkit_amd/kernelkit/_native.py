@@ -15,6 +15,7 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import gc
 import os
 import sys
 import threading
@@ -36,6 +37,7 @@ KK_COPY_D2D = 3
 HALO_LO = 1
 HALO_HI = 2
 HALO = HALO_LO + HALO_HI
+PLANE_GAP = 64
 
 
 class NativeLibraryError(RuntimeError):
@@ -154,6 +156,23 @@ _SIGNATURES = {
     "kk_cone_fp_transpose_static_capacity": (ctypes.c_int64, []),
     "kk_cone_fp_transpose_work_elems": (ctypes.c_int64, [
         _vp, ctypes.c_int32, ctypes.c_int32]),
+    "kk_projections_to_bp_planes": (ctypes.c_int, [
+        _vp, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, _c_i64p, _vp,
+        _vp]),
+    "kk_bp_reads_planes": (ctypes.c_int32, [_vp, ctypes.c_int32,
+                                            ctypes.c_int32, _c_i32p]),
+    "kk_bp_planes_elems": (ctypes.c_int64, [ctypes.c_int32, ctypes.c_int32,
+                                            ctypes.c_int32]),
+    "kk_residual_to_bp_planes": (ctypes.c_int, [
+        _vp, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, ctypes.c_int32,
+        ctypes.c_int32, ctypes.c_int32, _vp, _vp]),
+    "kk_sirt_bp_update_planes": (ctypes.c_int, [
+        _vp, _vp, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, _vp,
+        _c_i32p, _c_i64p, _vp, _c_i64p, _vp, _c_i64p, ctypes.c_float,
+        ctypes.c_float, ctypes.c_int32, ctypes.c_int32, ctypes.c_float, _vp]),
+    "kk_cone_bp_planes": (ctypes.c_int, [
+        _vp, _vp, ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, _vp,
+        _c_i32p, _c_i64p, ctypes.c_float, ctypes.c_int32, _vp]),
     "kk_cone_bp":(ctypes.c_int, [_vp, _vp, ctypes.c_int32, ctypes.c_int32,
                                   ctypes.c_int32, _vp, _c_i32p, _c_i64p,
                                   ctypes.c_float, ctypes.c_int32, _vp]),
@@ -179,6 +198,8 @@ _SIGNATURES = {
     "kk_fp_line_spacing": (ctypes.c_int, [
         _c_f64p, ctypes.c_int32, _c_i32p, ctypes.c_int32, ctypes.c_int32,
         _c_i32p, _c_f64p, _c_f64p]),
+    "kk_bp_patch_extent": (ctypes.c_int, [_c_f64p, ctypes.c_int32, _c_i32p,
+                                          _c_f64p]),
     "kk_bp_table": (ctypes.c_int, [_c_f64p, ctypes.c_int32, _vp]),
     "kk_filter_create": (ctypes.c_int, [ctypes.POINTER(_vp)]),
     "kk_filter_destroy": (ctypes.c_int, [_vp]),
@@ -482,6 +503,11 @@ class Graph:
     @classmethod
     def capture(cls, fn) -> "Graph":
         s = Stream()
+        # no cycle collection while capturing: it may free device memory of
+        # objects long out of use (plans of dropped operators), which a
+        # capture does not survive
+        collects = gc.isenabled()
+        gc.disable()
         check(lib().kk_graph_begin_capture(s.ptr))
         try:
             with use_stream(s.ptr):
@@ -491,6 +517,9 @@ class Graph:
             if lib().kk_graph_end_capture(s.ptr, ctypes.byref(dead)) == KK_OK:
                 lib().kk_graph_destroy(dead)
             raise
+        finally:
+            if collects:
+                gc.enable()
         exec_ptr = _vp()
         check(lib().kk_graph_end_capture(s.ptr, ctypes.byref(exec_ptr)))
         return cls(exec_ptr)

@@ -25,7 +25,7 @@ from kernelkit.kernel import (BaseKernel, ProjectionTexture, as_device_array,
                               default_device, is_device_array)
 from kernelkit.kernels.cone_bp import VoxelDrivenConeBP
 from kernelkit.operator import XrayTransform
-from kernelkit.processing import filter_into
+from kernelkit.processing import filter_into, filter_rows_into
 from kernelkit.projector import BackProjector, ForwardProjector
 
 
@@ -86,9 +86,15 @@ def bp(projections: Any, projection_geometry, volume_geometry: VolumeGeometry,
         if projection_axes != (0, 1, 2):
             raise NotImplementedError()
         tex = ProjectionTexture(*proj.shape, like=proj)
-        tex.zero()
-        filter_into(proj, tex, geoms=list(projection_geometry),
-                    filter=filter)
+        if K.reads_planes:
+            filtered = device.empty(tuple(proj.shape), like=proj)
+            filter_rows_into(proj, filtered, geoms=list(projection_geometry),
+                             filter=filter)
+            tex.update(filtered, planes=True)
+        else:
+            tex.zero()
+            filter_into(proj, tex, geoms=list(projection_geometry),
+                        filter=filter)
         ptor._textures = tex
     else:
         ptor.projections = proj
@@ -193,11 +199,14 @@ class _SirtState:
         _native.check(lib.kk_recip_or_zero(_native._vp(R.data_ptr()),
                                            R.numel(), st))
         self.C, self.R = C, R
-        # textures: x for the FP, residual for the BP (halo stays zero)
+        # textures: x for the FP, residual for the BP (halo stays zero; every
+        # element of planes is written by each residual pass)
         self.fptor.volume = self.x
         self.xtex = self.fptor._texture
         self.rtex = self.bptor._textures
-        self.rtex.zero()
+        self.planes = self.rtex.planes is not None
+        if not self.planes:
+            self.rtex.zero()
         self.res = self.rtex.values()
         # a broadcast view: stride 0 along the mask's broadcast axes
         self.mask = (None if mask is None else device.broadcast_to(
@@ -219,11 +228,15 @@ class _SirtState:
         # MI355X than the forward kernel's residual epilogue, which reads
         # y and R one detector row per lane)
         fk._launch(self.xtex, self.p, self.rows, self.cols, False, None)
-        _native.check(lib.kk_residual_to_bp_texture(
+        rtex = _native._vp(self.rtex.hold_planes() if self.planes
+                           else self.rtex.ptr)
+        residual = (lib.kk_residual_to_bp_planes if self.planes
+                    else lib.kk_residual_to_bp_texture)
+        _native.check(residual(
             _native._vp(self.p.data_ptr()), _native.i64(self.p.stride()),
             _native._vp(self.y.data_ptr()), _native.i64(self.y.stride()),
             _native._vp(self.R.data_ptr()), _native.i64(self.R.stride()),
-            self.n, self.rows, self.cols, _native._vp(self.rtex.ptr), st))
+            self.n, self.rows, self.cols, rtex, st))
         mask_ptr = None if self.mask is None else _native._vp(
             self.mask.data_ptr())
         mask_st = None if self.mask is None else _native.i64(
@@ -232,13 +245,16 @@ class _SirtState:
         # the texture kernel (coalesced), which on MI355X costs ~1.2 ms at
         # 512^3 against ~7.8 ms for the update epilogue's scattered
         # frame stores
-        _native.check(lib.kk_sirt_bp_update(
-            bk._plan.ptr, _native._vp(self.rtex.ptr),
-            self.n, self.rows, self.cols, _native._vp(self.x.data_ptr()),
-            _native.i32(self.shape), _native.i64(self.x.stride()),
-            _native._vp(self.C.data_ptr()), _native.i64(self.C.stride()),
-            mask_ptr, mask_st, self.lo, self.hi, self.clip_lo, self.clip_hi,
-            None, 0, self.scale, st))
+        args = (bk._plan.ptr, rtex, self.n, self.rows, self.cols,
+                _native._vp(self.x.data_ptr()), _native.i32(self.shape),
+                _native.i64(self.x.stride()), _native._vp(self.C.data_ptr()),
+                _native.i64(self.C.stride()), mask_ptr, mask_st, self.lo,
+                self.hi, self.clip_lo, self.clip_hi)
+        if self.planes:
+            _native.check(lib.kk_sirt_bp_update_planes(*args, self.scale, st))
+        else:
+            _native.check(lib.kk_sirt_bp_update(*args, None, 0, self.scale,
+                                                st))
         self.xtex.update(self.x, planes=fk.reads_planes)
 
     def capture(self):

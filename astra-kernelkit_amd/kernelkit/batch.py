@@ -99,7 +99,7 @@ class ConeBatch:
         volumes = [as_device_array(v) for v in volumes]
         self._check(volumes, self.domain_shapes, "volume")
         for op, y in zip(self.ops, projs):
-            op.backprojector.projections = y  # builds the BP textures
+            op.backprojector._set_projections(y, pairs=True)
         key = tuple(v.data_ptr() for v in volumes) + tuple(
             op.backprojector._textures.ptr for op in self.ops)
         if self._bp_cache is None or self._bp_cache[0] != key:

@@ -246,28 +246,71 @@ class VolumeTexture:
 
 class ProjectionTexture:
     """Backprojection layout of projections: ``[angle][rows+3][cols+3]`` of
-    (value, next-row) float2 pairs with a zero halo; see
-    ``include/kernelkit_hip.h``."""
+    (value, next-row) float2 pairs with a zero halo for the general kernel,
+    or planes (plain floats, column-major) for the kernel of circular orbits;
+    see ``include/kernelkit_hip.h``.  :attr:`data` and :attr:`ptr` are the
+    pairs, made from the planes when asked for, as in
+    :class:`VolumeTexture`."""
 
     def __init__(self, n_angles: int, rows: int, cols: int, device=None,
                  like=None):
         self.shape = (int(n_angles), int(rows), int(cols))
-        n = _native.lib().kk_bp_texture_elems(*self.shape)
-        if n < 0:
+        self._n = _native.lib().kk_bp_texture_elems(*self.shape)
+        if self._n < 0:
             raise ValueError(f"bad projection shape {self.shape}")
-        self.data = _alloc(n, like, device)
+        self._pairs = self._planes = None
+        self._holds_planes = False
+        self._like = like
+        if like is None:
+            self._pairs = self._like = _alloc(self._n, like, device)
+
+    def _buffer(self, n):
+        self._like = _alloc(n, self._like)
+        return self._like
+
+    @property
+    def data(self):
+        if self._pairs is None:
+            self._pairs = self._buffer(self._n)
+        if self._holds_planes:
+            n, rows, cols = self.shape
+            pitch = rows + _native.PLANE_GAP
+            _native.check(_native.lib().kk_projections_to_bp_texture(
+                _native._vp(self._planes.data_ptr()), *self.shape,
+                _native.i64((cols * pitch, 1, pitch)),
+                _native._vp(self._pairs.data_ptr()), _native.stream_ptr()))
+            self._holds_planes = False
+        return self._pairs
 
     @property
     def ptr(self):
         return self.data.data_ptr()
 
+    @property
+    def planes(self):
+        """Device address of the planes, None unless the texture's content
+        is held as such."""
+        return self._planes.data_ptr() if self._holds_planes else None
+
+    def hold_planes(self) -> int:
+        """Device address of the planes, which become the texture's content
+        (for launches that write every element of them)."""
+        if self._planes is None:
+            self._planes = self._buffer(
+                _native.lib().kk_bp_planes_elems(*self.shape))
+        self._holds_planes = True
+        return self._planes.data_ptr()
+
     def zero(self, stream=None) -> None:
+        if self._pairs is None:
+            self._pairs = self._buffer(self._n)
+        self._holds_planes = False
         _native.check(_native.lib().kk_fill(
             _native._vp(self.ptr), self.data.numel(), 0.0,
             _native.stream_ptr(stream)))
 
     def update(self, projections, projection_axes=(0, 1, 2),
-               stream=None) -> None:
+               stream=None, planes: bool = False) -> None:
         """Copy projections (array axis k = logical axis
         ``projection_axes[k]`` of (angle, row, col))."""
         projections = as_device_array(projections)
@@ -282,14 +325,30 @@ class ProjectionTexture:
         if tuple(lshape) != self.shape:
             raise ValueError(f"projections of shape {tuple(lshape)} do not "
                              f"match texture shape {self.shape}")
-        _native.check(_native.lib().kk_projections_to_bp_texture(
+        lib = _native.lib()
+        if planes:
+            build, dst = lib.kk_projections_to_bp_planes, self.hold_planes()
+        else:
+            if self._pairs is None:
+                self._pairs = self._buffer(self._n)
+            self._holds_planes = False
+            build, dst = lib.kk_projections_to_bp_texture, self.ptr
+        _native.check(build(
             _native._vp(projections.data_ptr()), *self.shape,
-            _native.i64(lstride), _native._vp(self.ptr),
+            _native.i64(lstride), _native._vp(dst),
             _native.stream_ptr(stream)))
 
     def values(self):
         """The stored projections as an (angle, row, col) strided view."""
         n, rows, cols = self.shape
+        if self._holds_planes:
+            buf, pitch = self._planes, rows + _native.PLANE_GAP
+            if _dev.is_torch(buf):
+                return buf.view(n, cols, pitch)[:, :, :rows].permute(0, 2, 1)
+            return _dev.DeviceArray((n, rows, cols), np.float32,
+                                    ptr=buf.data_ptr(),
+                                    strides=(cols * pitch, 1, pitch),
+                                    owner=buf, device=buf.device.index)
         h = _native.HALO
         lo = _native.HALO_LO
         if _dev.is_torch(self.data):

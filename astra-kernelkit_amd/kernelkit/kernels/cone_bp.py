@@ -20,6 +20,7 @@ from kernelkit import device as _dev
 from kernelkit.kernel import (BaseKernel, KernelMemoryUnpreparedException,
                               KernelNotCompiledException, ProjectionTexture,
                               Texture, as_device_array, is_device_array)
+from kernelkit.kernels.cone_fp import detector_shape
 
 
 def _world_strides(tensor, volume_axes) -> list:
@@ -73,6 +74,8 @@ class VoxelDrivenConeBP(BaseKernel):
         self._proj_axs = tuple(projection_axes)
         self._params_are_set = False
         self._n_params = 0
+        self._planes_key = None
+        self._reads_planes = False
 
     @property
     def volume_axes(self):
@@ -134,6 +137,28 @@ class VoxelDrivenConeBP(BaseKernel):
             self._plan.ptr, _native.f64_ptr(arr), n))
         self._n_params = n
         self._params_are_set = True
+        self._planes_key = None
+        self._reads_planes = False
+        if projection_geometry is not None and volume_geometry is not None:
+            rows, cols = detector_shape(projection_geometry)
+            self.reads_planes_for(rows, cols, volume_geometry)
+
+    @property
+    def reads_planes(self) -> bool:
+        """Whether the parameters set with their geometries are ones that the
+        kernel backprojects from planes
+        (:class:`~kernelkit.kernel.ProjectionTexture`)."""
+        return self._reads_planes
+
+    def reads_planes_for(self, rows, cols, volume_geometry) -> bool:
+        """:attr:`reads_planes` for a detector and volume given."""
+        key = (rows, cols, tuple(volume_geometry.shape))
+        if key != self._planes_key:
+            self._planes_key = key
+            self._reads_planes = bool(_native.lib().kk_bp_reads_planes(
+                self._plan.ptr, rows, cols,
+                _native.i32(volume_geometry.shape)))
+        return self._reads_planes
 
     def __call__(self, textures, volume, volume_geometry: VolumeGeometry, *,
                  additive: bool = True, stream=None):
@@ -175,25 +200,33 @@ class VoxelDrivenConeBP(BaseKernel):
                 f"Volume shape {tuple(volume.shape)} does not match volume "
                 f"geometry {tuple(volume_geometry.shape)} with axes "
                 f"{self._vol_axs}.")
-        _native.check(_native.lib().kk_cone_bp(
-            self._plan.ptr, _native._vp(textures.ptr), n, rows, cols,
+        planes = textures.planes
+        if planes is not None and n == self._n_params and \
+                self.reads_planes_for(rows, cols, volume_geometry):
+            launch, tex = _native.lib().kk_cone_bp_planes, planes
+        else:
+            launch, tex = _native.lib().kk_cone_bp, textures.ptr
+        _native.check(launch(
+            self._plan.ptr, _native._vp(tex), n, rows, cols,
             _native._vp(volume.data_ptr()), _native.i32(volume_geometry.shape),
             _native.i64(_world_strides(volume, self._vol_axs)),
             float(volume_geometry.voxel_volume()), 1 if additive else 0,
             _native.stream_ptr(stream)))
 
     def projection_texture(self, projections,
-                           texture: ProjectionTexture | None = None
-                           ) -> ProjectionTexture:
+                           texture: ProjectionTexture | None = None,
+                           pairs: bool = False) -> ProjectionTexture:
         """Build (or refresh) the backprojection texture of projections
-        given in ``projection_axes`` order."""
+        given in ``projection_axes`` order, as the kernel reads it or as
+        ``pairs`` (the batch launches')."""
         projections = as_device_array(projections)
         logical = [0, 0, 0]
         for k, ax in enumerate(self._proj_axs):
             logical[ax] = projections.shape[k]
         if texture is None or texture.shape != tuple(logical):
             texture = ProjectionTexture(*logical, like=projections)
-        texture.update(projections, self._proj_axs)
+        texture.update(projections, self._proj_axs,
+                       planes=self.reads_planes and not pairs)
         return texture
 
     def _from_snapshot(self, snap: Texture) -> ProjectionTexture:

@@ -207,13 +207,30 @@ def filter_into(projections, texture, geoms=None, filter: str = "ramlak",
     if tuple(texture.shape) != (n, rows, cols):
         raise ValueError(f"texture of shape {texture.shape} does not match "
                          f"projections of shape {(n, rows, cols)}")
+    f = _fused_tables(projections, geoms, filter, detector_piercings)
+    _native.check(_native.lib().kk_filter_rows_to_bp_texture(
+        f.ptr, _native._vp(projections.data_ptr()),
+        _native.i64(projections.stride()), _native._vp(texture.ptr), n, rows,
+        cols, 1 if geoms is not None else 0, _native.stream_ptr()))
+
+
+def _fused_tables(projections, geoms, filter, detector_piercings):
+    n, rows, cols = projections.shape
     num = padded_length(cols)
     P = None if geoms is None else np.ascontiguousarray(
         preweight_params(geoms, detector_piercings))
     if P is not None and P.shape[0] != n:
         raise ValueError(f"{P.shape[0]} geometries for {n} projections")
-    f = _filter_tables(num, filter, P)
-    _native.check(_native.lib().kk_filter_rows_to_bp_texture(
+    return _filter_tables(num, filter, P)
+
+
+def filter_rows_into(projections, out, geoms=None, filter: str = "ramlak",
+                     detector_piercings=None) -> None:
+    """:func:`filter_into` with a plain array ``out`` of the same shape."""
+    n, rows, cols = projections.shape
+    f = _fused_tables(projections, geoms, filter, detector_piercings)
+    _native.check(_native.lib().kk_filter_rows(
         f.ptr, _native._vp(projections.data_ptr()),
-        _native.i64(projections.stride()), _native._vp(texture.ptr), n, rows,
-        cols, 1 if geoms is not None else 0, _native.stream_ptr()))
+        _native.i64(projections.stride()), _native._vp(out.data_ptr()),
+        _native.i64(out.stride()), n, rows, cols,
+        1 if geoms is not None else 0, _native.stream_ptr()))

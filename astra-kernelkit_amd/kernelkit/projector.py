@@ -359,6 +359,9 @@ class BackProjector(Projector):
     @projections.setter
     def projections(self, value: Any):
         """Copy projections into the padded texture (``:448-556``)."""
+        self._set_projections(value)
+
+    def _set_projections(self, value: Any, pairs: bool = False):
         if not (is_device_array(value) or isinstance(value, (np.ndarray,
                                                              list))):
             raise TypeError("Projections must be a `ndarray`, device tensor "
@@ -391,7 +394,14 @@ class BackProjector(Projector):
                              "projection axis is 0.")
         value = as_device_array(value)
         self._textures = self._K.projection_texture(
-            value, getattr(self, "_textures", None))
+            value, getattr(self, "_textures", None), pairs)
+
+    def _update_params(self):
+        super()._update_params()
+        tex = getattr(self, "_textures", None)
+        if (tex is not None and tex.planes is not None
+                and not self._K.reads_planes):
+            tex.data  # noqa: B018 -- as the new kernel reads them
 
     @projections.deleter
     def projections(self):

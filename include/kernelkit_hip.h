@@ -114,6 +114,27 @@ int kk_projections_to_bp_texture(const float* proj, int32_t n_angles,
                                  const int64_t strides[3], float* tex,
                                  void* stream);
 
+/* BP planes: projections as plain floats, column-major, [angle][col][rows +
+ * KK_PLANE_GAP] with zeros after each column, which the launches of
+ * kk_cone_bp_planes and kk_sirt_bp_update_planes read: for circular orbits
+ * about z whose 16 x 16 x 16 voxel tiles project onto at most 64 x 64 pixels.
+ * kk_bp_reads_planes says whether the plan's parameters with a rows x cols
+ * detector and the volume's shape are such (1) or not (0).
+ * kk_residual_to_bp_planes: planes of the SIRT residual (proj - y) * R. */
+#define KK_PLANE_GAP 64
+int32_t kk_bp_reads_planes(const kk_plan* plan, int32_t rows, int32_t cols,
+                           const int32_t vol_shape[3]);
+int64_t kk_bp_planes_elems(int32_t n_angles, int32_t rows, int32_t cols);
+int kk_projections_to_bp_planes(const float* proj, int32_t n_angles,
+                                int32_t rows, int32_t cols,
+                                const int64_t strides[3], float* planes,
+                                void* stream);
+int kk_residual_to_bp_planes(const float* proj, const int64_t proj_strides[3],
+                             const float* y, const int64_t y_strides[3],
+                             const float* R, const int64_t R_strides[3],
+                             int32_t n_angles, int32_t rows, int32_t cols,
+                             float* planes, void* stream);
+
 /* value-fill of n floats (a kernel, not hipMemsetAsync: graph-safe). */
 int kk_fill(float* ptr, int64_t n, float value, void* stream);
 
@@ -211,6 +232,13 @@ int kk_cone_bp(const kk_plan* plan, const float* proj_tex, int32_t n_angles,
                int32_t rows, int32_t cols, float* vol,
                const int32_t vol_shape[3], const int64_t vol_strides[3],
                float output_scale, int32_t additive, void* stream);
+
+/* kk_cone_bp from planes: KK_ERR_UNSUPPORTED where kk_bp_reads_planes gives
+ * 0. */
+int kk_cone_bp_planes(const kk_plan* plan, const float* planes,
+                      int32_t n_angles, int32_t rows, int32_t cols, float* vol,
+                      const int32_t vol_shape[3], const int64_t vol_strides[3],
+                      float output_scale, int32_t additive, void* stream);
 
 /* Exact transpose of kk_cone_fp (matched adjoint, for gradients): every
  * (ray, slice) sample of the forward projection adds proj * scale *
@@ -342,6 +370,12 @@ int kk_fp_line_spacing(const double* params, int32_t n_angles,
                        double out[2]);
 int kk_bp_table(const double* params, int32_t n_angles, void* out);
 
+/* Host-only: bounds of the detector columns and rows that any 16 x 16 x 16
+ * voxel tile projects onto (out[0], out[1]); -1 if the orbit is not circular
+ * about z.  What kk_bp_reads_planes decides on. */
+int kk_bp_patch_extent(const double* params, int32_t n_angles,
+                       const int32_t vol_shape[3], double out[2]);
+
 /* ---- SIRT (kernelkit/algo.py:226-368) ---------------------------------- */
 
 /* res = (FP(x) - y) * R for every ray: the residual step of one SIRT
@@ -383,6 +417,14 @@ int kk_sirt_bp_update(const kk_plan* plan, const float* res_tex,
                       float lo, float hi, int32_t clip_lo, int32_t clip_hi,
                       float* x_tex, int32_t x_tex_mask, float output_scale,
                       void* stream);
+
+/* kk_sirt_bp_update from planes of the residual (x alone: no x_tex). */
+int kk_sirt_bp_update_planes(
+    const kk_plan* plan, const float* planes, int32_t n_angles, int32_t rows,
+    int32_t cols, float* x, const int32_t vol_shape[3],
+    const int64_t x_strides[3], const float* C, const int64_t C_strides[3],
+    const float* mask, const int64_t mask_strides[3], float lo, float hi,
+    int32_t clip_lo, int32_t clip_hi, float output_scale, void* stream);
 
 /* p = 1/p with +inf mapped to 0, n contiguous floats (algo.py:324-332). */
 int kk_recip_or_zero(float* ptr, int64_t n, void* stream);
