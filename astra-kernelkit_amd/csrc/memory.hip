@@ -6,9 +6,45 @@
 // directly.  These entry points let the Python drop-in own device buffers
 // (kernelkit.DeviceArray) when no torch tensor is involved, and let any
 // C caller do the same through this library alone.
+#include <algorithm>
+#include <cstring>
+#include <system_error>
+#include <thread>
+
 #include "kk_internal.h"
 
 namespace {
+
+// Device -> pageable host memory in pieces through pinned buffers, one per
+// worker: while one worker's piece is on the bus the others copy theirs out
+// (and take the page faults of fresh host memory).  Buffers and threads live
+// for one call.  A 64 MiB result on MI355X with 16 host cores: 2.5 ms, against
+// 15.6 ms for the runtime's copy into fresh pages and 6.2 ms into numpy's.
+constexpr int64_t kHostPiece = int64_t(2) << 20;
+constexpr int kHostWorkers = 6;
+
+// One worker's pieces w, w + workers, ...: the first error, or success.
+hipError_t copy_pieces(int device, char* dst, const char* src, int64_t bytes,
+                       int w, int workers, hipStream_t stream) {
+  hipError_t e = hipSetDevice(device);
+  if (e != hipSuccess) return e;
+  void* buf = nullptr;
+  hipEvent_t done = nullptr;
+  e = hipHostMalloc(&buf, size_t(std::min(kHostPiece, bytes)), 0);
+  if (e == hipSuccess)
+    e = hipEventCreateWithFlags(&done, hipEventDisableTiming);
+  for (int64_t at = w * kHostPiece; e == hipSuccess && at < bytes;
+       at += workers * kHostPiece) {
+    const size_t n = size_t(std::min(kHostPiece, bytes - at));
+    e = hipMemcpyAsync(buf, src + at, n, hipMemcpyDeviceToHost, stream);
+    if (e == hipSuccess) e = hipEventRecord(done, stream);
+    if (e == hipSuccess) e = hipEventSynchronize(done);
+    if (e == hipSuccess) std::memcpy(dst + at, buf, n);
+  }
+  if (done) hipEventDestroy(done);
+  if (buf) hipHostFree(buf);
+  return e;
+}
 
 // dst[i, j, k] = src[i, j, k] for a 3-D index space of n0 x n1 x n2
 // elements (element strides, any signs and orders).  One thread per
@@ -94,6 +130,45 @@ extern "C" int kk_memcpy(void* dst, const void* src, int64_t bytes,
   const hipError_t e = hipMemcpyAsync(dst, src, static_cast<size_t>(bytes), k,
                                       static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return kk::hip_fail(e, "hipMemcpyAsync");
+  return KK_OK;
+}
+
+extern "C" int kk_copy_to_host(void* dst, const void* src, int64_t bytes,
+                               void* stream) {
+  if (bytes < 0 || (bytes > 0 && (dst == nullptr || src == nullptr)))
+    return kk::fail(KK_ERR_INVALID, "kk_copy_to_host: bad arguments");
+  if (bytes == 0) return KK_OK;
+  int device = 0;
+  hipError_t e = hipGetDevice(&device);
+  if (e != hipSuccess) return kk::hip_fail(e, "hipGetDevice");
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  const int64_t pieces = (bytes + kHostPiece - 1) / kHostPiece;
+  const int workers =
+      static_cast<int>(std::min<int64_t>(kHostWorkers, pieces));
+  hipError_t errors[kHostWorkers] = {};
+  std::thread threads[kHostWorkers];
+  auto work = [&](int w) {
+    errors[w] = copy_pieces(device, static_cast<char*>(dst),
+                            static_cast<const char*>(src), bytes, w, workers,
+                            st);
+  };
+  for (int w = 1; w < workers; ++w) {
+    try {
+      threads[w] = std::thread(work, w);
+    } catch (const std::system_error&) {
+      // no thread to be had: this thread does its share below
+    }
+  }
+  work(0);
+  for (int w = 1; w < workers; ++w) {
+    if (threads[w].joinable())
+      threads[w].join();
+    else
+      work(w);
+  }
+  for (int w = 0; w < workers; ++w)
+    if (errors[w] != hipSuccess)
+      return kk::hip_fail(errors[w], "kk_copy_to_host");
   return KK_OK;
 }
 

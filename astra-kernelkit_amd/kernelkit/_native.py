@@ -91,6 +91,7 @@ _SIGNATURES = {
     "kk_free": (ctypes.c_int, [_vp]),
     "kk_memcpy": (ctypes.c_int, [_vp, _vp, ctypes.c_int64, ctypes.c_int32,
                                  _vp]),
+    "kk_copy_to_host": (ctypes.c_int, [_vp, _vp, ctypes.c_int64, _vp]),
     "kk_stream_synchronize": (ctypes.c_int, [_vp]),
     "kk_copy_strided": (ctypes.c_int, [_vp, _c_i64p, _vp, _c_i64p, _c_i64p,
                                        ctypes.c_int32, _vp]),

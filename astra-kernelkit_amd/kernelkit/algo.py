@@ -30,11 +30,7 @@ from kernelkit.projector import BackProjector, ForwardProjector
 
 
 def _to_host(t, out=None):
-    host = device.to_host(t)
-    if out is not None:
-        out[...] = host
-        return out
-    return host
+    return device.to_host(t, out)
 
 
 def fp(volume: Any, projection_geometry, volume_geometry: VolumeGeometry,

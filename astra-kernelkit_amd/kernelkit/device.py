@@ -337,6 +337,12 @@ class DeviceArray:
         """Copy to a new host array (synchronises the stream)."""
         src = self.contiguous()
         out = np.empty(self.shape, dtype=self.dtype)
+        if out.nbytes >= _THREADED_COPY:
+            _native.check(_native.lib().kk_copy_to_host(
+                out.ctypes.data_as(ctypes.c_void_p),
+                ctypes.c_void_p(src._ptr), out.nbytes,
+                _native.stream_ptr(stream)))
+            return out
         _native.check(_native.lib().kk_memcpy(
             out.ctypes.data_as(ctypes.c_void_p), ctypes.c_void_p(src._ptr),
             out.nbytes, _native.KK_COPY_D2H, _native.stream_ptr(stream)))
@@ -427,8 +433,36 @@ def broadcast_to(x, shape):
     return asarray(x).expand(tuple(shape))
 
 
-def to_host(x) -> np.ndarray:
-    """A host copy (numpy) of a device array."""
+# Bytes from which copies to the host go through kk_copy_to_host's threads
+# (8 MiB: 2.0 -> 0.5 ms, 64 MiB: 15.4 -> 2.4 ms, 512 MiB: 125 -> 14 ms;
+# below, its buffers and threads cost what they save).
+_THREADED_COPY = 4 << 20
+
+
+def to_host(x, out=None) -> np.ndarray:
+    """A host copy (numpy) of a device array: ``out`` filled if given, else
+    a new array."""
     if is_torch(x):
-        return x.detach().cpu().numpy()
-    return asarray(x).get()
+        x = x.detach()
+        torch = _torch_module()
+        if (x.is_cuda and x.dtype == torch.float32 and x.is_contiguous()
+                and 4 * x.numel() >= _THREADED_COPY
+                and x.device.index == torch.cuda.current_device()):
+            direct = (isinstance(out, np.ndarray) and out.dtype == np.float32
+                      and out.shape == tuple(x.shape)
+                      and out.flags.c_contiguous and out.flags.writeable)
+            host = out if direct else np.empty(tuple(x.shape), np.float32)
+            _native.check(_native.lib().kk_copy_to_host(
+                host.ctypes.data_as(ctypes.c_void_p),
+                ctypes.c_void_p(x.data_ptr()), host.nbytes,
+                _native.stream_ptr()))
+            if direct:
+                return out
+        else:
+            host = x.cpu().numpy()
+    else:
+        host = asarray(x).get()
+    if out is None:
+        return host
+    out[...] = host
+    return out

@@ -158,6 +158,9 @@ int kk_malloc(void** ptr, int64_t bytes);
 int kk_free(void* ptr);
 int kk_memcpy(void* dst, const void* src, int64_t bytes, int32_t kind,
               void* stream);
+/* Contiguous device memory into pageable host memory after the stream's work
+ * so far, with several host threads; returns when the bytes are there. */
+int kk_copy_to_host(void* dst, const void* src, int64_t bytes, void* stream);
 int kk_stream_synchronize(void* stream);
 int kk_copy_strided(const void* src, const int64_t src_strides[3], void* dst,
                     const int64_t dst_strides[3], const int64_t shape[3],
