@@ -16,33 +16,26 @@
 //    workspace through an LDS tile.  The gather below then reads, for one
 //    column, the rows of 64 neighbouring voxels: a few cache lines per
 //    wavefront instead of 64.
-// 2. cone_fp_t_kernel: a gather, so that no atomics are needed (an LDS
-//    float atomic add costs ~190 cycles per wavefront instruction on this
-//    part, against ~8 for a plain LDS read-modify-write).  A lane owns kJB x kJC
-//    voxels (kJB along b, kJC consecutive along c) of one slice, the 64
-//    lanes of a wavefront consecutive c pairs, accumulated in the lane's
-//    own LDS words over all angles of the launch's ray axis and written
-//    once.  Owning
-//    two c voxels, a lane evaluates each of its samples once for both
-//    (a sample has two c taps): 3/2 evaluations per sample instead of 2.  Per angle:
-//    * circular orbits ("column-coherent" angles: the row step has no a/b
-//      part): the b coordinate of a sample depends on the detector column
-//      only, so the columns reaching the wavefront's b-run are a
-//      wave-uniform interval (inverse of the column -> b map).  The lanes
-//      compute 64 columns' ray data at a time and broadcast them with
-//      readlane (scalar registers); per column, the c coordinate is affine
-//      in the row, so each lane sums the rows reaching its voxel and the
-//      sum enters the b-run with the column's two b taps (a wave-uniform
-//      LDS row);
-//    * other geometries: each lane projects the support rectangle of its
-//      voxels (at its slice) onto the detector and walks the pixels of the
-//      bounding box; the b taps, whose index differs per lane, are summed
-//      in the lane's own LDS words (one read-modify-write pair per sample
-//      instead of a select over all kJB registers).
+// 2. A gather, so that no atomics are needed (an LDS float atomic add costs
+//    ~190 cycles per wavefront instruction on this part, against ~8 for a
+//    plain LDS read-modify-write).  A lane owns 8 voxels along b by 2
+//    consecutive ones along c of one slice, summed over all angles of the
+//    launch's ray axis and written once.  Owning two c voxels, a lane
+//    evaluates each of its samples once for both (a sample has two c taps):
+//    3/2 evaluations per sample instead of 2.
+//    * cone_fp_t_col_kernel, circular orbits ("column-coherent" angles: the
+//      row step has no a/b part): below.
+//    * cone_fp_t_kernel, other geometries: each lane projects the support
+//      rectangle of its voxels (at its slice) onto the detector and walks
+//      the pixels of the bounding box; the b taps, whose index differs per
+//      lane, are summed in the lane's own LDS words (one read-modify-write
+//      pair per sample instead of a select over all registers).
+//    A plan with both kinds of angles launches both; each skips the other's.
 // Candidate intervals are widened by 1e-6 voxel in coordinate space, far
 // above the float64 rounding of the sample coordinates; samples outside
 // the support get zero weight.
 #include <algorithm>
+#include <type_traits>
 
 #include "kk_internal.h"
 
@@ -53,7 +46,6 @@ constexpr int kJC = 2;       // consecutive voxels along c per lane
 constexpr int kWaves = 4;    // wavefronts per workgroup (b-runs)
 constexpr int kThreads = 64 * kWaves;
 constexpr double kEps = 1e-6;
-constexpr int kRU = 4;       // rows per load group (column-coherent path)
 
 struct FptArgs {
   const float* yw;        // weighted projections [angle][col][row]
@@ -142,6 +134,12 @@ __device__ __forceinline__ double rcp64(double d) {
   return fma(r, fma(-d, r, 1.0), r);
 }
 
+// 1 / d to the last bits: a second Newton step.
+__device__ __forceinline__ double rcp64x2(double d) {
+  const double r = rcp64(d);
+  return fma(r, fma(-d, r, 1.0), r);
+}
+
 // Least / greatest value over a wavefront whose 64 lanes are all active
 // (DPP steps and a readlane, no LDS round trips), as a scalar.
 __device__ __forceinline__ int32_t wave_min_all(int32_t v) {
@@ -165,16 +163,6 @@ __device__ __forceinline__ void int_range(float lo, float hi, int32_t n,
   hi = fminf(hi, static_cast<float>(n));
   a = max(0, static_cast<int32_t>(ceilf(lo)));
   b = min(n - 1, static_cast<int32_t>(floorf(hi)));
-}
-
-// A sample at c offset x from the centre of a lane's first voxel, carrying
-// value y: adds y times the tents of the lane's two voxels, 1 - |x| and
-// 1 - |x - 1|, written max(0, 1 - |x|) and med3(0, x, 2 - x) (exact for
-// x in [0, 2]).
-static_assert(kJC == 2, "tent_pair covers two c voxels per lane");
-__device__ __forceinline__ void tent_pair(float x, float y, float* colsum) {
-  colsum[0] = fmaf(y, fmaxf(0.f, 1.f - fabsf(x)), colsum[0]);
-  colsum[1] = fmaf(y, __builtin_amdgcn_fmed3f(0.f, x, 2.f - x), colsum[1]);
 }
 
 // Ends a run of samples whose b tap index is the float t: S - T goes to
@@ -208,15 +196,7 @@ __device__ __forceinline__ int32_t bcast(int32_t v, int32_t l) {
   return __builtin_amdgcn_readlane(v, l);
 }
 
-// Paths a launch compiles (its plan's angles need): the column-coherent
-// one, the general one, or both.  A launch without column-coherent angles
-// does not reserve the column records' LDS, which keeps a sixth workgroup
-// per CU resident.
-constexpr int kPathColumn = 1;
-constexpr int kPathGeneral = 2;
-
-template <int PATHS>
-__global__ __launch_bounds__(kThreads, PATHS == 3 ? 5 : 6) void cone_fp_t_kernel(
+__global__ __launch_bounds__(kThreads, 6) void cone_fp_t_kernel(
     const kk::FpAngle* __restrict__ tab, FptArgs A) {
   // slice fastest, then b tile, then c tile; runs of kSliceRun
   // consecutive ids (neighbouring slices of one tile, which read nearly
@@ -234,31 +214,16 @@ __global__ __launch_bounds__(kThreads, PATHS == 3 ? 5 : 6) void cone_fp_t_kernel
   if (jw >= A.nb) return;  // no barriers below: idle wavefronts may leave
 
   const double fi = static_cast<double>(i);
-  const double nb1 = static_cast<double>(A.nb + 1);
   const double kd = static_cast<double>(k);
-  const float kf = static_cast<float>(k);
   const int32_t cstride = A.rows + 2 * kRowPad;  // workspace column stride
   const int64_t angle_elems = static_cast<int64_t>(cstride) * A.cols;
   // b-tap sums of this lane's voxels (row t: b voxel jw + t), indexed per
   // lane: every lane owns its words, so no atomics and no cross-lane
   // ordering are needed; taps just outside the b-run are not written out.
-  // (A register array indexed by the wave-uniform tap row was compiled
-  // into private scratch memory.)  The general path's run flushes use a
-  // spare row on either side of the b-run (g[-1], g[kJB]); launches
-  // without that path keep the LDS smaller.
-  constexpr int kSpare = (PATHS & kPathGeneral) != 0 ? 1 : 0;
+  // The run flushes use a spare row on either side of it (g[-1], g[kJB]).
+  constexpr int kSpare = 1;
   __shared__ float gacc[kWaves][kJB + 2 * kSpare][kJC][64];
   float(*g)[kJC][64] = gacc[threadIdx.x >> 6] + kSpare;
-  // column records of the column-coherent path, written lane-parallel and
-  // read back per column at a wave-uniform address (an LDS broadcast, which
-  // costs no vector-ALU slot, unlike a readlane): {alpha, beta} in float64
-  // and {alpha, 1 / alpha, window origin, b fraction} in float32.  Each
-  // wavefront uses its own records, in program order: no barrier.
-  constexpr int kRec = (PATHS & kPathColumn) != 0 ? 64 : 1;
-  __shared__ double2 crd_s[kWaves][kRec];
-  __shared__ float4 crf_s[kWaves][kRec];
-  double2* crd = crd_s[threadIdx.x >> 6];
-  float4* crf = crf_s[threadIdx.x >> 6];
 #pragma unroll
   for (int t = -kSpare; t < kJB + kSpare; ++t)
 #pragma unroll
@@ -269,292 +234,149 @@ __global__ __launch_bounds__(kThreads, PATHS == 3 ? 5 : 6) void cone_fp_t_kernel
     const kk::FpAngle& P = tab[ang];
     const float* img = A.yw + ang * angle_elems + kRowPad;
     const double arel = fi + P.sig;  // slice centre, relative to the source
-    if (P.colc) { if constexpr ((PATHS & kPathColumn) != 0) {
-      // columns whose b coordinate at this slice lies in
-      // [jw, jw + kJB + 1): a1 = (x_b - taub) / arel, and for these
-      // angles a1 = (col ub + qb) / (col ua + qa)
-      const double t1 = (jw - kEps - P.taub) / arel;
-      const double t2 = (jw + kJB + 1 + kEps - P.taub) / arel;
-      const double d1 = fma(t1, P.ua, -P.ub), d2 = fma(t2, P.ua, -P.ub);
-      int32_t c_lo = 0, c_hi = A.cols - 1;
-      if (d1 * d2 > 0.0) {
-        const double c1 = fma(-t1, P.qa, P.qb) / d1;
-        const double c2 = fma(-t2, P.qa, P.qb) / d2;
-        if (isfinite(c1) && isfinite(c2))
-          int_range(fmin(c1, c2), fmax(c1, c2), A.cols, c_lo, c_hi);
+    if (P.colc) continue;  // cone_fp_t_col_kernel's
+    // pixels whose rays meet the support rectangle of this lane's voxels
+    // at this slice: bounding box of its projected corners.  The ray
+    // through the source-relative point X meets the detector at
+    // col = (V x Q).X / N.X, row = (Q x U).X / N.X with N = U x V
+    // (q + col U + row V = lam X, lam = U.(V x Q) / N.X > 0 in front of
+    // the source): linear forms in X, whose a and b parts (the slice and
+    // the wave's b-run) are shared by the wave; each lane adds its c part.
+    const double nva = P.ub * P.vc - P.uc * P.vb;
+    const double nvb = P.uc * P.va - P.ua * P.vc;
+    const double nvc = P.ua * P.vb - P.ub * P.va;
+    const double mva = P.vb * P.qc - P.vc * P.qb;
+    const double mvb = P.vc * P.qa - P.va * P.qc;
+    const double mvc = P.va * P.qb - P.vb * P.qa;
+    const double rva = P.qb * P.uc - P.qc * P.ub;
+    const double rvb = P.qc * P.ua - P.qa * P.uc;
+    const double rvc = P.qa * P.ub - P.qb * P.ua;
+    const double lamn = P.ua * mva + P.ub * mvb + P.uc * mvc;
+    double cmin = 1e300, cmax = -1e300, rmin = 1e300, rmax = -1e300;
+    bool ok = true;
+#pragma unroll
+    for (int eb = 0; eb < 2; ++eb) {
+      const double xb = (eb ? jw + kJB + 1 + kEps : jw - kEps) - P.taub;
+      const double dn = fma(nvb, xb, nva * arel);
+      const double cn = fma(mvb, xb, mva * arel);
+      const double rn = fma(rvb, xb, rva * arel);
+#pragma unroll
+      for (int ec = 0; ec < 2; ++ec) {
+        const double xc =
+            (ec ? kd + (kJC + 1) + kEps : kd - kEps) - P.tauc;
+        const double inv = rcp64(fma(nvc, xc, dn));
+        const double pc = fma(mvc, xc, cn) * inv;
+        const double pr = fma(rvc, xc, rn) * inv;
+        ok = ok && isfinite(pc) && isfinite(pr) && lamn * inv > 0.0;
+        cmin = fmin(cmin, pc);
+        cmax = fmax(cmax, pc);
+        rmin = fmin(rmin, pr);
+        rmax = fmax(rmax, pr);
       }
-      // computed from wave-uniform values: scalar loop control below
-      c_lo = __builtin_amdgcn_readfirstlane(c_lo);
-      c_hi = __builtin_amdgcn_readfirstlane(c_hi);
-      for (int32_t cb = c_lo; cb <= c_hi; cb += 64) {
-        const int32_t ncol = min(64, c_hi - cb + 1);
-        // ray data of column cb + lane (kk_fp_ray's terms: the row terms
-        // of a and b are exact zeros for these angles).  The c coordinate
-        // of the column's rays at this slice is affine in the row:
-        // x_c(r) = beta + alpha r (padded coordinates, float64).
-        double alpha = 0.0, beta = 0.0;
-        float fb = 0.f, ia = 0.f, alphaf = 0.f, off = 0.f;
-        int32_t t0 = -99, nrow = 0;
-        if (lane < ncol) {
-          const double fc = static_cast<double>(cb + lane);
-          const double Da = fma(fc, P.ua, P.qa);
-          const double Db = fma(fc, P.ub, P.qb);
-          const double inv = 1.0 / Da;
-          const double a1 = Db * inv;
-          const double b1 = fma(a1, P.sig, P.taub);
-          if (isfinite(a1) && isfinite(b1)) {
-            uint32_t ib;
-            kk_fp_coord(a1, b1, fi, nb1, ib, fb);
-            t0 = static_cast<int32_t>(ib) - kk::kHaloLo - jw;
-          }
-          const double D0c = fma(fc, P.uc, P.qc);
-          alpha = P.vc * inv * arel;
-          beta = fma(D0c * inv, arel, P.tauc);
-          if (!isfinite(alpha) || !isfinite(beta)) t0 = -99;
-          alphaf = static_cast<float>(alpha);
-          ia = fabsf(alphaf) > 1e-9f ? 1.f / alphaf : 0.f;
-          // a lane's window: the rows whose c coordinate lies in the open
-          // padded span (k, k + kJC + 1) of its voxels' tents, (kJC + 1)
-          // |1 / alpha| rows long, i.e. at most floor(len) + 1 integer
-          // rows.  Windows of at most kRowPad - 3 rows are read as nrow
-          // rows from the ceiling of the first row, moved 1e-3 row earlier
-          // (float32 rounding of the start is ~1e-5 row; rows outside get
-          // zero tent weight); longer ones take the exact range below.
-          const float len = static_cast<float>(kJC + 1) * fabsf(ia);
-          if (ia != 0.f && len + 3.f <= static_cast<float>(kRowPad)) {
-            nrow = static_cast<int32_t>(floorf(len + 2e-3f)) + 1;
-            off = fminf(0.f, static_cast<float>(kJC + 1) * ia) - 1e-3f;
-          }
-        }
-        // window origin: the lane's first row is k / alpha + origin
-        const float org = fmaf(-static_cast<float>(beta), ia, off);
-        crd[lane] = make_double2(alpha, beta);
-        crf[lane] = make_float4(alphaf, ia, org, fb);
-        // the column's tap row and window length, one broadcast
-        const int32_t tpk = (min(max(t0, -99), 100) + 128) | (nrow << 8);
-        for (int32_t m = 0; m < ncol; ++m) {
-          const int32_t pk = bcast(tpk, m);
-          const int32_t tm = (pk & 255) - 128;
-          if (tm < -1 || tm >= kJB) continue;
-          const int32_t nr = pk >> 8;
-          const float4 cf = crf[m];
-          const double2 cd = crd[m];
-          const float alm = cf.x, iam = cf.y;
-          const float* ycol = img + (cb + m) * cstride;
-          float colsum[kJC];
-#pragma unroll
-          for (int cc = 0; cc < kJC; ++cc) colsum[cc] = 0.f;
-          if (nr > 0) {
-            // nr rows (wave-uniform: no per-lane loop control) from the
-            // ceiling of the window's first row, clamped into the padded
-            // column (a window off the detector reads zeros)
-            const float r1 = fmaf(kf, iam, cf.z);
-            const int32_t r_lo =
-                min(max(static_cast<int32_t>(ceilf(r1)), -kRowPad),
-                    A.rows + kRowPad - nr);
-            // the window's first row in float64, relative to the centre
-            // of the lane's first voxel (padded coordinate k + 1); the
-            // rows after it in float32 offsets (|alpha u| is a few voxels,
-            // so the offsets carry ~1e-7 voxel of rounding).  A voxel's
-            // weight is the tent 1 - |x_c - centre| of the sample, equal
-            // to the forward kernel's bilinear tap weight.
-            const float loc = static_cast<float>(
-                fma(cd.x, static_cast<double>(r_lo), cd.y) - (kd + 1.0));
-            const float* yw = ycol + r_lo;
-            int32_t u = 0;
-            float uf = 0.f;   // u as a float, counted (exact)
-            for (; u + kRU <= nr; u += kRU, uf += static_cast<float>(kRU)) {
-              float y[kRU];
-#pragma unroll
-              for (int t = 0; t < kRU; ++t) y[t] = yw[u + t];
-              const float xg = fmaf(alm, uf, loc);
-#pragma unroll
-              for (int t = 0; t < kRU; ++t)
-                tent_pair(t == 0 ? xg : fmaf(alm, static_cast<float>(t), xg),
-                          y[t], colsum);
-            }
-            for (; u < nr; ++u, uf += 1.f)
-              tent_pair(fmaf(alm, uf, loc), yw[u], colsum);
-          } else {
-          // rows whose c coordinate lies in [k, k + kJC + 1) (the padded
-          // span of the lane's voxels' tents), found in float32 and
-          // widened by 1e-2 row; samples outside get zero weight below
-          int32_t r_lo = 0, r_hi = A.rows - 1;
-          if (iam != 0.f) {
-            const float r1 = fmaf(kf, iam, cf.z);
-            const float r2 = fmaf(static_cast<float>(kJC + 1), iam, r1);
-            int_range(fminf(r1, r2) - 1e-2f, fmaxf(r1, r2) + 1e-2f, A.rows,
-                      r_lo, r_hi);
-          }
-          // the lane's first row in float64 (the first voxel's centre is
-          // at padded coordinate k + 1), float32 offsets after it, tents
-          // as above; rays the forward kernel skips have yw = 0
-          const float loc = static_cast<float>(
-              fma(cd.x, static_cast<double>(r_lo), cd.y) - (kd + 1.0));
-          float du = 0.f;
-          for (int32_t r = r_lo; r <= r_hi; ++r, du += 1.f)
-            tent_pair(fmaf(alm, du, loc), ycol[r], colsum);
-          }
-          // the column's two b taps tm, tm + 1 (wave-uniform, so the
-          // tests are scalar branches): read-modify-write of the lane's
-          // own LDS words
-          const float fbm = cf.w;
-          if (tm >= 0) {
-#pragma unroll
-            for (int cc = 0; cc < kJC; ++cc)
-              g[tm][cc][lane] = fmaf(1.f - fbm, colsum[cc], g[tm][cc][lane]);
-          }
-          if (tm + 1 < kJB) {
-#pragma unroll
-            for (int cc = 0; cc < kJC; ++cc)
-              g[tm + 1][cc][lane] = fmaf(fbm, colsum[cc], g[tm + 1][cc][lane]);
-          }
-        }
-      }
-    } } else if constexpr ((PATHS & kPathGeneral) != 0) {
-      // pixels whose rays meet the support rectangle of this lane's voxels
-      // at this slice: bounding box of its projected corners.  The ray
-      // through the source-relative point X meets the detector at
-      // col = (V x Q).X / N.X, row = (Q x U).X / N.X with N = U x V
-      // (q + col U + row V = lam X, lam = U.(V x Q) / N.X > 0 in front of
-      // the source): linear forms in X, whose a and b parts (the slice and
-      // the wave's b-run) are shared by the wave; each lane adds its c part.
-      const double nva = P.ub * P.vc - P.uc * P.vb;
-      const double nvb = P.uc * P.va - P.ua * P.vc;
-      const double nvc = P.ua * P.vb - P.ub * P.va;
-      const double mva = P.vb * P.qc - P.vc * P.qb;
-      const double mvb = P.vc * P.qa - P.va * P.qc;
-      const double mvc = P.va * P.qb - P.vb * P.qa;
-      const double rva = P.qb * P.uc - P.qc * P.ub;
-      const double rvb = P.qc * P.ua - P.qa * P.uc;
-      const double rvc = P.qa * P.ub - P.qb * P.ua;
-      const double lamn = P.ua * mva + P.ub * mvb + P.uc * mvc;
-      double cmin = 1e300, cmax = -1e300, rmin = 1e300, rmax = -1e300;
-      bool ok = true;
-#pragma unroll
-      for (int eb = 0; eb < 2; ++eb) {
-        const double xb = (eb ? jw + kJB + 1 + kEps : jw - kEps) - P.taub;
-        const double dn = fma(nvb, xb, nva * arel);
-        const double cn = fma(mvb, xb, mva * arel);
-        const double rn = fma(rvb, xb, rva * arel);
-#pragma unroll
-        for (int ec = 0; ec < 2; ++ec) {
-          const double xc =
-              (ec ? kd + (kJC + 1) + kEps : kd - kEps) - P.tauc;
-          const double inv = rcp64(fma(nvc, xc, dn));
-          const double pc = fma(mvc, xc, cn) * inv;
-          const double pr = fma(rvc, xc, rn) * inv;
-          ok = ok && isfinite(pc) && isfinite(pr) && lamn * inv > 0.0;
-          cmin = fmin(cmin, pc);
-          cmax = fmax(cmax, pc);
-          rmin = fmin(rmin, pr);
-          rmax = fmax(rmax, pr);
-        }
-      }
-      int32_t c_lo = 0, c_hi = A.cols - 1, r_lo = 0, r_hi = A.rows - 1;
-      if (ok) {
-        int_range(cmin, cmax, A.cols, c_lo, c_hi);
-        int_range(rmin, rmax, A.rows, r_lo, r_hi);
-      }
-      // columns in a loop of wave-uniform length, each lane walking its
-      // own column range from its first column (a tilted rotation axis
-      // shifts the lanes' ranges against each other: a loop over their
-      // union would leave a lane idle for the difference), rows per lane.
-      // Sample coordinates: float64 at an anchor pixel
-      // (the wave's first column, the lane's first row), float32 offsets
-      // from it.  With D = q + col U + row V (kk_fp_ray's terms) and
-      // t = D_b / D_a at the anchor, x_b = arel D_b / D_a + tau_b moves by
-      // arel (dD_b - t dD_a) / D_a between the anchor and a pixel: a
-      // quantity of the box's size, so its float32 rounding is ~1e-6
-      // voxel.  Weights are the tents 1 - |x - centre| of the forward
-      // kernel's bilinear taps.
-      const int32_t wc_lo = wave_min_all(c_lo <= c_hi ? c_lo : A.cols);
-      const double fwc = static_cast<double>(wc_lo);
-      const double fr0 = static_cast<double>(r_lo);
-      const double Da0 = fma(fr0, P.va, fma(fwc, P.ua, P.qa));
-      const double Db0 = fma(fr0, P.vb, fma(fwc, P.ub, P.qb));
-      const double Dc0 = fma(fr0, P.vc, fma(fwc, P.uc, P.qc));
-      const double inv0 = rcp64(Da0);
-      const double tb = Db0 * inv0, tcv = Dc0 * inv0;
-      const float ob =
-          static_cast<float>(fma(tb, arel, P.taub) - (jw + kk::kHaloLo));
-      const float oc =
-          static_cast<float>(fma(tcv, arel, P.tauc) - (kd + kk::kHaloLo));
-      const float da0 = static_cast<float>(Da0);
-      const float tbf = static_cast<float>(tb), tcf = static_cast<float>(tcv);
-      const float arf = static_cast<float>(arel);
-      const float uaf = static_cast<float>(P.ua), ubf = static_cast<float>(P.ub),
-                  ucf = static_cast<float>(P.uc);
-      const float vaf = static_cast<float>(P.va), vbf = static_cast<float>(P.vb),
-                  vcf = static_cast<float>(P.vc);
-      const bool anchor_ok = ok && isfinite(tb) && isfinite(tcv);
-      // With u the row offset from the lane's first row and dc the column
-      // offset from the wave's first column, dA = dc ua + u va (b, c
-      // alike) and x_b = ob + arel (dB - tb dA) / (Da0 + dA): per column
-      // the numerator arel (dB - tb dA) is affine in u with slope
-      // arel (vb - tb va), and the denominator with slope va (c alike).
-      const float kvb = arf * fmaf(-tbf, vaf, vbf);
-      const float kvc = arf * fmaf(-tcf, vaf, vcf);
-      const int32_t ncol = (anchor_ok && c_lo <= c_hi) ? c_hi - c_lo + 1 : 0;
-      const int32_t wncol = wave_max_all(ncol);
-      // b-tap sums over a run of samples with the same tap index, added to
-      // the lane's LDS words when the index changes: S = sum of y w_c,
-      // T = sum of y w_c fb, so the taps t and t + 1 receive S - T and T.
-      // A run stays open from column to column while the index holds (the
-      // sums of one index add up whatever the column), so along the walk
-      // a run closes about once per b voxel crossed.  The index is kept as
-      // a float (the floor of x_b); a run reaches the LDS words only if
-      // its index lies in [-1, kJB) and is dropped otherwise.  Rows
-      // outside the lane's tents add zeros; a non-finite coordinate (a ray
-      // parallel to the slices) starts a run of its own that is dropped.
-      float tcur = -2.f;  // no run yet
-      float S[kJC], T[kJC];
-#pragma unroll
-      for (int cc = 0; cc < kJC; ++cc) S[cc] = T[cc] = 0.f;
-      // the workspace of this angle as bytes (a wave-uniform base) and a
-      // 32-bit byte offset per lane: the launcher keeps an angle's
-      // workspace below 4 GiB
-      const char* imgb = reinterpret_cast<const char*>(img);
-      const uint32_t nrow =
-          static_cast<uint32_t>(max(0, r_hi - r_lo + 1));
-      for (int32_t j = 0; j < wncol; ++j) {
-        const int32_t col = c_lo + j;  // this lane's column (in range if
-                                       // j < ncol)
-        const float dcf = static_cast<float>(col - wc_lo);
-        const float dAc = dcf * uaf;
-        const float nb0 = arf * fmaf(-tbf, dAc, dcf * ubf);
-        const float nc0 = arf * fmaf(-tcf, dAc, dcf * ucf);
-        const float den0 = da0 + dAc;
-        uint32_t o = 4u * (static_cast<uint32_t>(col) *
-                               static_cast<uint32_t>(cstride) +
-                           static_cast<uint32_t>(r_lo));
-        const uint32_t oend = o + 4u * (j < ncol ? nrow : 0u);
-        float drf = 0.f;
-        for (; o < oend; o += 4u, drf += 1.f) {
-          // the load first: its latency overlaps the coordinates below.
-          // The empty asm keeps the offset a 32-bit register (an SGPR base
-          // plus a VGPR offset), not a 64-bit pointer stepped per row.
-          asm volatile("" : "+v"(o));
-          const float yv = *reinterpret_cast<const float*>(imgb + o);
-          const float rc = __builtin_amdgcn_rcpf(fmaf(drf, vaf, den0));
-          const float xc = fmaf(fmaf(drf, kvc, nc0), rc, oc);
-          const float xb = fmaf(fmaf(drf, kvb, nb0), rc, ob);
-          const float fl = floorf(xb);
-          if (fl != tcur) {
-            close_run(g, lane, tcur, S, T);
-            tcur = fl;
-          }
-          const float yfb = yv * (xb - fl);
-          const float w0 = fmaxf(0.f, 1.f - fabsf(xc));
-          const float w1 = __builtin_amdgcn_fmed3f(0.f, xc, 2.f - xc);
-          S[0] = fmaf(yv, w0, S[0]);
-          S[1] = fmaf(yv, w1, S[1]);
-          T[0] = fmaf(yfb, w0, T[0]);
-          T[1] = fmaf(yfb, w1, T[1]);
-        }
-      }
-      close_run(g, lane, tcur, S, T);
     }
+    int32_t c_lo = 0, c_hi = A.cols - 1, r_lo = 0, r_hi = A.rows - 1;
+    if (ok) {
+      int_range(cmin, cmax, A.cols, c_lo, c_hi);
+      int_range(rmin, rmax, A.rows, r_lo, r_hi);
+    }
+    // columns in a loop of wave-uniform length, each lane walking its
+    // own column range from its first column (a tilted rotation axis
+    // shifts the lanes' ranges against each other: a loop over their
+    // union would leave a lane idle for the difference), rows per lane.
+    // Sample coordinates: float64 at an anchor pixel
+    // (the wave's first column, the lane's first row), float32 offsets
+    // from it.  With D = q + col U + row V (kk_fp_ray's terms) and
+    // t = D_b / D_a at the anchor, x_b = arel D_b / D_a + tau_b moves by
+    // arel (dD_b - t dD_a) / D_a between the anchor and a pixel: a
+    // quantity of the box's size, so its float32 rounding is ~1e-6
+    // voxel.  Weights are the tents 1 - |x - centre| of the forward
+    // kernel's bilinear taps.
+    const int32_t wc_lo = wave_min_all(c_lo <= c_hi ? c_lo : A.cols);
+    const double fwc = static_cast<double>(wc_lo);
+    const double fr0 = static_cast<double>(r_lo);
+    const double Da0 = fma(fr0, P.va, fma(fwc, P.ua, P.qa));
+    const double Db0 = fma(fr0, P.vb, fma(fwc, P.ub, P.qb));
+    const double Dc0 = fma(fr0, P.vc, fma(fwc, P.uc, P.qc));
+    const double inv0 = rcp64(Da0);
+    const double tb = Db0 * inv0, tcv = Dc0 * inv0;
+    const float ob =
+        static_cast<float>(fma(tb, arel, P.taub) - (jw + kk::kHaloLo));
+    const float oc =
+        static_cast<float>(fma(tcv, arel, P.tauc) - (kd + kk::kHaloLo));
+    const float da0 = static_cast<float>(Da0);
+    const float tbf = static_cast<float>(tb), tcf = static_cast<float>(tcv);
+    const float arf = static_cast<float>(arel);
+    const float uaf = static_cast<float>(P.ua), ubf = static_cast<float>(P.ub),
+                ucf = static_cast<float>(P.uc);
+    const float vaf = static_cast<float>(P.va), vbf = static_cast<float>(P.vb),
+                vcf = static_cast<float>(P.vc);
+    const bool anchor_ok = ok && isfinite(tb) && isfinite(tcv);
+    // With u the row offset from the lane's first row and dc the column
+    // offset from the wave's first column, dA = dc ua + u va (b, c
+    // alike) and x_b = ob + arel (dB - tb dA) / (Da0 + dA): per column
+    // the numerator arel (dB - tb dA) is affine in u with slope
+    // arel (vb - tb va), and the denominator with slope va (c alike).
+    const float kvb = arf * fmaf(-tbf, vaf, vbf);
+    const float kvc = arf * fmaf(-tcf, vaf, vcf);
+    const int32_t ncol = (anchor_ok && c_lo <= c_hi) ? c_hi - c_lo + 1 : 0;
+    const int32_t wncol = wave_max_all(ncol);
+    // b-tap sums over a run of samples with the same tap index, added to
+    // the lane's LDS words when the index changes: S = sum of y w_c,
+    // T = sum of y w_c fb, so the taps t and t + 1 receive S - T and T.
+    // A run stays open from column to column while the index holds (the
+    // sums of one index add up whatever the column), so along the walk
+    // a run closes about once per b voxel crossed.  The index is kept as
+    // a float (the floor of x_b); a run reaches the LDS words only if
+    // its index lies in [-1, kJB) and is dropped otherwise.  Rows
+    // outside the lane's tents add zeros; a non-finite coordinate (a ray
+    // parallel to the slices) starts a run of its own that is dropped.
+    float tcur = -2.f;  // no run yet
+    float S[kJC], T[kJC];
+#pragma unroll
+    for (int cc = 0; cc < kJC; ++cc) S[cc] = T[cc] = 0.f;
+    // the workspace of this angle as bytes (a wave-uniform base) and a
+    // 32-bit byte offset per lane: the launcher keeps an angle's
+    // workspace below 4 GiB
+    const char* imgb = reinterpret_cast<const char*>(img);
+    const uint32_t nrow =
+        static_cast<uint32_t>(max(0, r_hi - r_lo + 1));
+    for (int32_t j = 0; j < wncol; ++j) {
+      const int32_t col = c_lo + j;  // this lane's column (in range if
+                                     // j < ncol)
+      const float dcf = static_cast<float>(col - wc_lo);
+      const float dAc = dcf * uaf;
+      const float nb0 = arf * fmaf(-tbf, dAc, dcf * ubf);
+      const float nc0 = arf * fmaf(-tcf, dAc, dcf * ucf);
+      const float den0 = da0 + dAc;
+      uint32_t o = 4u * (static_cast<uint32_t>(col) *
+                             static_cast<uint32_t>(cstride) +
+                         static_cast<uint32_t>(r_lo));
+      const uint32_t oend = o + 4u * (j < ncol ? nrow : 0u);
+      float drf = 0.f;
+      for (; o < oend; o += 4u, drf += 1.f) {
+        // the load first: its latency overlaps the coordinates below.
+        // The empty asm keeps the offset a 32-bit register (an SGPR base
+        // plus a VGPR offset), not a 64-bit pointer stepped per row.
+        asm volatile("" : "+v"(o));
+        const float yv = *reinterpret_cast<const float*>(imgb + o);
+        const float rc = __builtin_amdgcn_rcpf(fmaf(drf, vaf, den0));
+        const float xc = fmaf(fmaf(drf, kvc, nc0), rc, oc);
+        const float xb = fmaf(fmaf(drf, kvb, nb0), rc, ob);
+        const float fl = floorf(xb);
+        if (fl != tcur) {
+          close_run(g, lane, tcur, S, T);
+          tcur = fl;
+        }
+        const float yfb = yv * (xb - fl);
+        const float w0 = fmaxf(0.f, 1.f - fabsf(xc));
+        const float w1 = __builtin_amdgcn_fmed3f(0.f, xc, 2.f - xc);
+        S[0] = fmaf(yv, w0, S[0]);
+        S[1] = fmaf(yv, w1, S[1]);
+        T[0] = fmaf(yfb, w0, T[0]);
+        T[1] = fmaf(yfb, w1, T[1]);
+      }
+    }
+    close_run(g, lane, tcur, S, T);
   }
 
 #pragma unroll
@@ -573,6 +395,386 @@ __global__ __launch_bounds__(kThreads, PATHS == 3 ? 5 : 6) void cone_fp_t_kernel
         A.vol[o] = v;
     }
   }
+}
+
+// ---------------------------------------------------------------------------
+// Column-coherent angles (circular orbits).
+//
+// The b coordinate of a sample depends on the detector column alone, and the
+// c coordinate is affine in the row.  So the columns that reach a wavefront's
+// 8 b voxels are an interval per angle, the same for all lanes; a column's
+// sum over the rows that reach a lane's two c voxels enters two neighbouring
+// b voxels with the column's weights.  What bounds it is the number of vector
+// instructions and of row loads per (wavefront, column), in balance (profiled
+// at 256^3, 360 angles of 384^2: vector unit 79 % busy, address unit 76 %):
+// * rows come in loads of four per lane (unaligned dwordx4): at the lanes'
+//   stride of two voxels a single dword costs the same 16 cycles;
+// * the b voxels are registers.  The walk over tap rows is unrolled, so each
+//   column adds to registers known at compile time, instead of four LDS
+//   read-modify-writes per column;
+// * a column's float64 data (about 120 instructions) is computed one column
+//   per lane for 64 columns at a time, taken across angles (an angle has
+//   about 11 per wavefront), and read back as an LDS broadcast and scalars;
+// * the number of rows per window is a template parameter, picked for 64
+//   columns at a time, and taps that are outside every lane's tent (the
+//   first row's second voxel, the last rows' first) are left out;
+// * a workgroup's slices are neighbours, which read nearly the same rows;
+//   its other wavefronts share out the angles and are added up at the end,
+//   which fills the chip for small volumes (and halves the length of the
+//   float32 sums: error against float64 1.3e-7 instead of 2.5e-7).
+// Measured with 256^3 / 360 angles of 384^2: 5.2 ms, before 10.2 ms (dword
+// row loads, an angle's columns at a time, sums in LDS); 128^3 / 128 angles:
+// 0.25 ms, before 0.67 ms; 64^3 / 64 angles: 0.09 ms, before 0.31 ms.
+// 16 voxels along b halve the work at run borders, but need a third of the
+// wavefronts' room: 7.1 ms.  One c voxel per lane: 7.1 ms.
+
+constexpr int kColSlices = 4;  // slices (wavefronts) per workgroup part
+constexpr int kColB = 8;       // voxels along b per lane
+// Wavefronts of one part from which a workgroup shares its angles out to two
+// parts, below to four (measured, two against four: 16384 5.23 / 5.45 ms,
+// 9600 1.26 / 1.24 ms, 2048 0.32 / 0.25 ms, 512 0.12 / 0.09 ms).
+constexpr int64_t kColSplit2 = 12288;
+// Marks a column whose record has whole voxels apart (whole_s).
+constexpr uint64_t kWhole = uint64_t(1) << 63;
+
+// Consecutive rows of a column, at any element alignment.
+typedef float f32x2_u __attribute__((ext_vector_type(2), aligned(4)));
+typedef float f32x3_u __attribute__((ext_vector_type(3), aligned(4)));
+typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
+
+// max(0, 1 - |x|), one instruction (|x| and the clamp to [0, 1] are free)
+__device__ __forceinline__ float tent(float x) {
+  float w;
+  asm("v_sub_f32_e64 %0, 1.0, |%1| clamp" : "=v"(w) : "v"(x));
+  return w;
+}
+
+template <int SPLIT>
+__global__ __launch_bounds__(64 * kColSlices * SPLIT, 8) void
+cone_fp_t_col_kernel(
+    const kk::FpAngle* __restrict__ tab, FptArgs A) {
+  const int32_t groups = (A.na + kColSlices - 1) / kColSlices;
+  const int64_t total = int64_t(groups) * A.tiles_b * A.tiles_c;
+  int64_t bid = kk_xcd_remap(blockIdx.x, total, kSliceRun / kColSlices);
+  const int32_t wave =
+      __builtin_amdgcn_readfirstlane(int32_t(threadIdx.x) >> 6);
+  const int32_t sub = wave / kColSlices;
+  const int32_t i = static_cast<int32_t>(bid % groups) * kColSlices +
+                    wave % kColSlices;
+  bid /= groups;
+  const int32_t jw = static_cast<int32_t>(bid % A.tiles_b) * kColB;
+  const int32_t k0 = static_cast<int32_t>(bid / A.tiles_b) * (64 * kJC);
+  const int32_t lane = threadIdx.x & 63;
+  const uint32_t cstride = A.rows + 2 * kRowPad;
+  const uint64_t angle_elems = static_cast<uint64_t>(cstride) * A.cols;
+  // this part's angles (none for slices past the volume)
+  const int32_t per = (A.n_angles + SPLIT - 1) / SPLIT;
+  const int32_t q_end = i < A.na ? min(A.n_angles, (sub + 1) * per) : 0;
+
+  __shared__ float4 rec_s[kColSlices * SPLIT][64][2];
+  __shared__ float whole_s[kColSlices * SPLIT][64];
+  __shared__ int3 run_s[kColSlices * SPLIT][64];
+  float4(*rec)[2] = rec_s[wave];
+  float* whole = whole_s[wave];
+  int3* run = run_s[wave];
+
+  float acc[kColB][kJC];
+#pragma unroll
+  for (int t = 0; t < kColB; ++t)
+#pragma unroll
+    for (int cc = 0; cc < kJC; ++cc) acc[t][cc] = 0.f;
+
+  for (int32_t q0 = sub * per; q0 < q_end; q0 += 64) {
+    // the column intervals of the next 64 angles, one angle per lane:
+    // columns whose b coordinate at this slice lies in [jw, jw + kColB + 1);
+    // a1 = (x_b - taub) / arel, and for these angles
+    // a1 = (col ub + qb) / (col ua + qa)
+    // (converted where they are used: kept as doubles for the whole walk,
+    // these cost the registers of another resident wavefront)
+    int32_t ii = i, jj = jw;
+    asm volatile("" : "+s"(ii), "+s"(jj));
+    int32_t l_ang = 0, l_lo = 0, l_n = 0;
+    if (q0 + lane < q_end) {
+      l_ang = A.angles[q0 + lane];
+      const kk::FpAngle& P = tab[l_ang];
+      if (P.colc) {
+        // (reciprocals to ~1e-14, far inside the widening by kEps)
+        const double ra = rcp64(static_cast<double>(ii) + P.sig);
+        const double t1 = (jj - kEps - P.taub) * ra;
+        const double t2 = (jj + kColB + 1 + kEps - P.taub) * ra;
+        const double d1 = fma(t1, P.ua, -P.ub), d2 = fma(t2, P.ua, -P.ub);
+        int32_t c_lo = 0, c_hi = A.cols - 1;
+        if (d1 * d2 > 0.0) {
+          const double c1 = fma(-t1, P.qa, P.qb) * rcp64(d1);
+          const double c2 = fma(-t2, P.qa, P.qb) * rcp64(d2);
+          if (isfinite(c1) && isfinite(c2))
+            int_range(fmin(c1, c2), fmax(c1, c2), A.cols, c_lo, c_hi);
+        }
+        l_lo = c_lo;
+        l_n = max(0, c_hi - c_lo + 1);
+      }
+    }
+    // the intervals' columns one after the other: an angle's run starts at
+    // the sum of the counts before it
+    int32_t end = l_n;
+#pragma unroll
+    for (int s = 1; s < 64; s <<= 1) {
+      const int32_t v = __shfl_up(end, s);
+      end += lane >= s ? v : 0;
+    }
+    const int32_t n_all = bcast(end, 63);
+    run[lane] = make_int3(end, l_ang, l_lo - (end - l_n));
+    for (int32_t g0 = 0; g0 < n_all; g0 += 64) {
+      // column g0 + lane of the runs: its rays (kk_fp_ray's terms: the row
+      // terms of a and b are exact zeros for these angles) and the c
+      // coordinate of its rows at this slice, beta + alpha r (padded
+      // coordinates)
+      int32_t t0 = -99, nr = 0;
+      uint64_t base = 0;
+      float iaf = 0.f, o1 = 0.f, ah = 0.f, al = 0.f, x0 = 0.f, fb = 0.f,
+            hi = 0.f, xw = 0.f;
+      bool neg = false;
+      int32_t is = i, nbs = A.nb + 1, ks = k0 + 1;
+      asm volatile("" : "+s"(is), "+s"(nbs), "+s"(ks));
+      if (g0 + lane < n_all) {
+        int32_t q = 0;   // the first run that ends after g0 + lane
+#pragma unroll
+        for (int s = 32; s > 0; s >>= 1)
+          if (run[q + s - 1].x <= g0 + lane) q += s;
+        const int3 r = run[q];
+        const kk::FpAngle& P = tab[r.y];
+        const int32_t col = r.z + g0 + lane;
+        const double fi = static_cast<double>(is);
+        const double arel = fi + P.sig;
+        const double fc = static_cast<double>(col);
+        const double inv = rcp64x2(fma(fc, P.ua, P.qa));
+        const double a1 = fma(fc, P.ub, P.qb) * inv;
+        const double b1 = fma(a1, P.sig, P.taub);
+        const double s = inv * arel;
+        double alpha = P.vc * s;
+        // c offset of row 0 from the tile's first voxel
+        double xb = fma(fma(fc, P.uc, P.qc), s, P.tauc) -
+                    static_cast<double>(ks);
+        if (isfinite(b1) && isfinite(alpha) && isfinite(xb)) {
+          uint32_t ib;
+          kk_fp_coord(a1, b1, fi, static_cast<double>(nbs), ib, fb);
+          t0 = static_cast<int32_t>(ib) - kk::kHaloLo - jw;
+          neg = alpha < 0.0;
+          if (neg) {  // mirrored: from the tile's last voxel, downwards
+            alpha = -alpha;
+            xb = (64 * kJC - 1) - xb;
+          }
+          ah = static_cast<float>(alpha);
+          al = static_cast<float>(alpha - static_cast<double>(ah));
+          // A lane's window: the rows whose c coordinate lies in the open
+          // span (-1, kJC) of its voxels' tents, (kJC + 1) / alpha rows long,
+          // i.e. at most floor(len) + 1 integer rows from the ceiling of
+          // the first one, moved 1e-3 row earlier (float32 rounding is
+          // below 1e-4 row; rows outside get zero weight).  Longer ones
+          // than the zero rows around a column allow are walked lane by
+          // lane (nr > kRowPad).
+          const double ia = ah > 1e-6f ? rcp64(alpha) : 0.0;
+          iaf = static_cast<float>(ia);
+          const float len = static_cast<float>(kJC + 1) * iaf;
+          nr = iaf == 0.f || len + 3.f > static_cast<float>(kRowPad)
+                   ? kRowPad + 1
+                   : static_cast<int32_t>(floorf(len + 2e-3f)) + 1;
+          const double r1 = (-1.0 - xb) * ia;
+          const double rb =
+              floor(fmin(fmax(r1, -kRowPad), static_cast<double>(A.rows)));
+          o1 = static_cast<float>(fmax(r1 - rb, -1e7)) - 1e-3f;
+          // Whole voxels of the offset apart where the base is not the first
+          // row of lane 0's window but the detector's edge: kept in x0, they
+          // would cost its low bits.
+          double xr = fma(alpha, rb, xb);
+          if (rb != floor(r1)) {
+            xw = static_cast<float>(fmin(fmax(floor(xr), -4e6), 4e6));
+            xr -= static_cast<double>(xw);
+          }
+          x0 = static_cast<float>(xr);
+          const int32_t rbi = static_cast<int32_t>(rb);
+          hi = static_cast<float>(A.rows - rbi);
+          base = r.y * angle_elems + static_cast<uint32_t>(col) * cstride +
+                 static_cast<uint32_t>(kRowPad + rbi) +
+                 (xw != 0.f ? kWhole : 0);
+        }
+      }
+      rec[lane][0] = make_float4(iaf, o1, ah, al);
+      rec[lane][1] = make_float4(x0, hi, fb, 1.f - fb);
+      whole[lane] = xw;
+      for (int sgn = 0; sgn < 2; ++sgn) {
+        const bool mine = t0 != -99 && neg == (sgn != 0);
+        if (__ballot(mine) == 0) continue;
+        const int32_t tt = mine ? t0 : -99;
+        const int32_t nn = mine ? nr : 0;
+        const float lv = static_cast<float>(kJC * (sgn ? 63 - lane : lane));
+        // one column, windows of at most W rows: the lane's sums over it
+        auto column = [&](int32_t l, auto w, auto dr, float* cs, float2& f) {
+          constexpr int W = decltype(w)::value;
+          constexpr bool D = decltype(dr)::value;
+          const uint32_t blo =
+              static_cast<uint32_t>(bcast(static_cast<int32_t>(base), l));
+          const uint32_t bhi = static_cast<uint32_t>(
+              bcast(static_cast<int32_t>(base >> 32), l));
+          const float* yc =
+              A.yw + (((static_cast<uint64_t>(bhi) << 32) | blo) & ~kWhole);
+          const float4 ra = rec[l][0], rb = rec[l][1];
+          f = make_float2(rb.z, rb.w);
+          const float du = __builtin_amdgcn_fmed3f(
+              ceilf(fmaf(lv, ra.x, ra.y)), 0.f, rb.y);
+          const char* p = reinterpret_cast<const char*>(yc) +
+                          (static_cast<uint32_t>(du) << 2);
+          float lx = lv;
+          if (bhi >> 31) lx -= whole[l];
+          const float x = fmaf(ra.w, du, fmaf(ra.z, du, -lx)) + rb.x;
+          if constexpr (W == 0) {
+            // rows one by one, up to the end of the lane's window
+            const float end =
+                ra.x == 0.f
+                    ? rb.y - 1.f
+                    : fminf(floorf(fmaf(lv, ra.x, ra.y) + 2e-2f +
+                                   static_cast<float>(kJC + 1) * ra.x),
+                            rb.y - 1.f);
+            cs[0] = 0.f;
+            cs[1] = 0.f;
+            for (float d = du; d <= end; d += 1.f, p += 4) {
+              const float xd = fmaf(ra.w, d, fmaf(ra.z, d, -lx)) + rb.x;
+              const float y = *reinterpret_cast<const float*>(p);
+              cs[0] = fmaf(y, tent(xd), cs[0]);
+              cs[1] = fmaf(y, tent(xd - 1.f), cs[1]);
+            }
+            return;
+          } else {
+            float y[W];
+#pragma unroll
+            for (int t = 0; t < W; t += 4) {
+              if (t + 4 <= W) {
+                const f32x4_u v = *reinterpret_cast<const f32x4_u*>(p + 4 * t);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) y[t + e] = v[e];
+              } else if (t + 3 == W) {
+                const f32x3_u v = *reinterpret_cast<const f32x3_u*>(p + 4 * t);
+                y[t] = v[0];
+                y[t + 1] = v[1];
+                y[t + 2] = v[2];
+              } else if (t + 2 == W) {
+                const f32x2_u v = *reinterpret_cast<const f32x2_u*>(p + 4 * t);
+                y[t] = v[0];
+                y[t + 1] = v[1];
+              } else {
+                y[t] = *reinterpret_cast<const float*>(p + 4 * t);
+              }
+            }
+#pragma unroll
+            for (int t = 0; t < W; ++t) {
+              const float xt =
+                  t == 0 ? x : fmaf(ra.z, static_cast<float>(t), x);
+              if (!D || t < (2 * W + 2) / 3)
+                cs[0] = t == 0 ? y[t] * tent(xt)
+                               : fmaf(y[t], tent(xt), cs[0]);
+              const float w1 = __builtin_amdgcn_fmed3f(0.f, xt, 2.f - xt);
+              if (t == (D ? 1 : 0))
+                cs[1] = y[t] * w1;
+              else if (t > 0)
+                cs[1] = fmaf(y[t], w1, cs[1]);
+            }
+          }
+        };
+        auto walk = [&](auto w, auto dr) {
+#pragma unroll
+          for (int t = -1; t < kColB; ++t) {
+            uint64_t mask = __ballot(tt == t);
+            while (mask != 0) {
+              const int32_t l = __builtin_ctzll(mask);
+              mask &= mask - 1;
+              float cs[kJC];
+              float2 f;
+              column(l, w, dr, cs, f);
+              auto add = [&](float c0, float c1) {
+                if (t >= 0) acc[t][0] = fmaf(f.y, c0, acc[t][0]);
+                if (t + 1 < kColB) acc[t + 1][0] = fmaf(f.x, c0, acc[t + 1][0]);
+                if (t >= 0) acc[t][1] = fmaf(f.y, c1, acc[t][1]);
+                if (t + 1 < kColB) acc[t + 1][1] = fmaf(f.x, c1, acc[t + 1][1]);
+              };
+              if (sgn == 0)
+                add(cs[0], cs[kJC - 1]);
+              else
+                add(cs[kJC - 1], cs[0]);
+            }
+          }
+        };
+        // below one c voxel per row the first row reaches no lane's second
+        // voxel, and the last ones (from 2 / alpha on) no lane's first
+        const bool D = __ballot(mine && ah > 0.999f) == 0;
+        if (__ballot(nn > (D ? kRowPad : 4)) != 0)
+          walk(std::integral_constant<int, 0>{}, std::false_type{});
+        else if (!D && __ballot(nn > 2) == 0)
+          walk(std::integral_constant<int, 2>{}, std::false_type{});
+        else if (!D && __ballot(nn > 3) == 0)
+          walk(std::integral_constant<int, 3>{}, std::false_type{});
+        else if (!D)
+          walk(std::integral_constant<int, 4>{}, std::false_type{});
+        else if (__ballot(nn > 4) == 0)
+          walk(std::integral_constant<int, 4>{}, std::true_type{});
+        else if (__ballot(nn > 5) == 0)
+          walk(std::integral_constant<int, 5>{}, std::true_type{});
+        else if (__ballot(nn > 6) == 0)
+          walk(std::integral_constant<int, 6>{}, std::true_type{});
+        else if (__ballot(nn > 7) == 0)
+          walk(std::integral_constant<int, 7>{}, std::true_type{});
+        else if (__ballot(nn > 8) == 0)
+          walk(std::integral_constant<int, 8>{}, std::true_type{});
+        else if (__ballot(nn > 12) == 0)
+          walk(std::integral_constant<int, 12>{}, std::true_type{});
+        else
+          walk(std::integral_constant<int, kRowPad>{}, std::true_type{});
+      }
+    }
+  }
+  if constexpr (SPLIT > 1) {
+    __shared__ float part[kColSlices][kColB * kJC][64];
+    for (int s = 1; s < SPLIT; ++s) {
+      if (sub == s)
+#pragma unroll
+        for (int t = 0; t < kColB; ++t)
+#pragma unroll
+          for (int cc = 0; cc < kJC; ++cc)
+            part[wave % kColSlices][t * kJC + cc][lane] = acc[t][cc];
+      __syncthreads();
+      if (sub == 0)
+#pragma unroll
+        for (int t = 0; t < kColB; ++t)
+#pragma unroll
+          for (int cc = 0; cc < kJC; ++cc)
+            acc[t][cc] += part[wave % kColSlices][t * kJC + cc][lane];
+      __syncthreads();
+    }
+    if (sub != 0) return;
+  }
+  if (i >= A.na) return;
+#pragma unroll
+  for (int cc = 0; cc < kJC; ++cc) {
+    const int32_t kc = k0 + lane * kJC + cc;
+    if (kc >= A.nc) break;
+#pragma unroll
+    for (int t = 0; t < kColB; ++t) {
+      const int32_t j = jw + t;
+      if (j >= A.nb) break;
+      const int64_t o = i * A.sa + j * A.sb + kc * A.sc;
+      A.vol[o] = A.mode == 1 ? A.vol[o] + acc[t][cc] : acc[t][cc];
+    }
+  }
+}
+
+int64_t col_grid(FptArgs& A) {
+  A.tiles_b = (A.nb + kColB - 1) / kColB;
+  A.tiles_c = (A.nc + 64 * kJC - 1) / (64 * kJC);
+  return int64_t((A.na + kColSlices - 1) / kColSlices) * A.tiles_b * A.tiles_c;
+}
+int64_t general_grid(FptArgs& A) {
+  A.tiles_b = (A.nb + kJB * kWaves - 1) / (kJB * kWaves);
+  A.tiles_c = (A.nc + 64 * kJC - 1) / (64 * kJC);
+  return int64_t(A.na) * A.tiles_b * A.tiles_c;
 }
 
 }  // namespace
@@ -641,28 +843,29 @@ int kk::fp_transpose_launch(const kk_plan_s* plan, const float* proj,
     A.na = vol_shape[a];
     A.nb = vol_shape[b];
     A.nc = vol_shape[c];
-    A.tiles_b = (A.nb + kJB * kWaves - 1) / (kJB * kWaves);
-    A.tiles_c = (A.nc + 64 * kJC - 1) / (64 * kJC);
-    const int64_t blocks = int64_t(A.na) * A.tiles_b * A.tiles_c;
-    if (blocks >= (int64_t(1) << 31))
-      return kk::fail(KK_ERR_UNSUPPORTED, "kk_cone_fp_transpose: grid");
-    const dim3 grid(static_cast<unsigned>(blocks));
     for (int32_t q0 = 0; q0 < n; q0 += chunk) {
       A.angles = plan->fr_idx + plan->fr_start[a] + q0;
       A.n_angles = std::min(chunk, n - q0);
-      A.mode = (first && !additive) ? 0 : 1;
-      first = false;
-      if (plan->fp_all_colc)
-        hipLaunchKernelGGL(cone_fp_t_kernel<kPathColumn>, grid,
-                           dim3(kThreads), 0, st, plan->fp, A);
-      else if (!plan->fp_any_colc)
-        hipLaunchKernelGGL(cone_fp_t_kernel<kPathGeneral>, grid,
-                           dim3(kThreads), 0, st, plan->fp, A);
-      else
-        hipLaunchKernelGGL((cone_fp_t_kernel<kPathColumn | kPathGeneral>),
-                           grid, dim3(kThreads), 0, st, plan->fp, A);
-      hipError_t e = hipGetLastError();
-      if (e != hipSuccess) return kk::hip_fail(e, "cone_fp_t_kernel");
+      for (int colc = 1; colc >= 0; --colc) {
+        if (colc ? !plan->fp_any_colc : plan->fp_all_colc) continue;
+        A.mode = (first && !additive) ? 0 : 1;
+        first = false;
+        const int64_t blocks = colc ? col_grid(A) : general_grid(A);
+        if (blocks >= (int64_t(1) << 31))
+          return kk::fail(KK_ERR_UNSUPPORTED, "kk_cone_fp_transpose: grid");
+        const dim3 grid(static_cast<unsigned>(blocks));
+        if (colc && blocks * kColSlices >= kColSplit2)
+          hipLaunchKernelGGL(cone_fp_t_col_kernel<2>, grid,
+                             dim3(64 * kColSlices * 2), 0, st, plan->fp, A);
+        else if (colc)
+          hipLaunchKernelGGL(cone_fp_t_col_kernel<4>, grid,
+                             dim3(64 * kColSlices * 4), 0, st, plan->fp, A);
+        else
+          hipLaunchKernelGGL(cone_fp_t_kernel, grid, dim3(kThreads), 0, st,
+                             plan->fp, A);
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return kk::hip_fail(e, "cone_fp_t_kernel");
+      }
     }
   }
   return KK_OK;
