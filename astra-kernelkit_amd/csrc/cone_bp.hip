@@ -27,6 +27,7 @@
 //   overlap, otherwise in runs of 16 tiles along x.
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "kk_internal.h"
 
@@ -385,7 +386,7 @@ __global__ __launch_bounds__(256, bp_min_blocks(K)) void cone_bp_kernel(
 }
 
 
-// ---- circular orbits: detector patches in LDS -----------------------------
+// ---- detector patches in LDS ----------------------------------------------
 //
 // A workgroup is a tile of 16 x 16 columns of K voxels.  Per angle it stages
 // the detector patch that the tile projects onto in LDS (from planes: the
@@ -396,9 +397,9 @@ __global__ __launch_bounds__(256, bp_min_blocks(K)) void cone_bp_kernel(
 // detector become zeros by the buffer descriptor (columns) and the zeros
 // between columns (rows), so nothing is clamped per update.
 //
-// What bounds it (MI355X): a gather from global memory costs a CU 16 cycles
-// per 64 updates (it took 20 with 16.5 vector instructions beside), the two
-// LDS reads 10, the patch ~3, vector issue ~10.  Measured: 512^3 / 720
+// What bounds circular orbits (MI355X): a gather from global memory costs a CU
+// 16 cycles per 64 updates (it took 20 with 16.5 vector instructions beside),
+// the two LDS reads 10, the patch ~3, vector issue ~10.  Measured: 512^3 / 720
 // 50.8 -> 38.0 ms, 256^3 / 360 3.2 -> 2.3 ms, 128^3 / 180 0.25 -> 0.18 ms.
 // LDS is 72% busy, vector issue about as much.
 // * Bank conflicts decide the layout: a wavefront is 8 x 8 columns and the
@@ -410,8 +411,18 @@ __global__ __launch_bounds__(256, bp_min_blocks(K)) void cone_bp_kernel(
 //   the groups' sums added at the end, where the tiles alone leave the chip
 //   idle (128^3: 0.244, 0.179 and 0.194 ms with 1, 2 and 4 parts).
 //
-// The row of an update is 64-bit fixed point (32 fraction bits), stepped by
-// one 64-bit add per voxel.
+// CIRC, circular orbits: the column and the weight are the same for a run of
+// K voxels, and the row of an update is 64-bit fixed point (32 fraction bits),
+// stepped by one 64-bit add per voxel.
+//
+// Otherwise (plans with a general angle): column, row and weight per voxel,
+// from float32 numerators around an integer base in the middle of the run and
+// one reciprocal.  26 vector instructions per update bound it (the vector unit
+// is issuing in 91% of the cycles; the pair kernel's gather took as long as
+// its instructions): 256^3 / 360 wobbling angles 4.9 -> 3.8 ms, 128^3 / 128
+// 0.27 -> 0.20 ms.  Five wavefronts per SIMD instead of four spill: 3.84 ms.
+// The reciprocal as a series around the base and addresses made in float32 were
+// no faster (3.9 ms).
 constexpr int kPatchRun = 16;                  // K
 constexpr int kPatchLanes = 64;                // rows per patch column
 constexpr int kPatchPitch = kPatchLanes + 6;   // LDS words per column
@@ -427,8 +438,9 @@ __device__ __forceinline__ uint64_t fixed_bits(double x) {
   return __builtin_bit_cast(uint64_t, x + kFixedMagic);
 }
 
-template <int K, int SPLIT>
-__global__ __launch_bounds__(256 * SPLIT, 5) void cone_bp_patch_kernel(
+template <int K, int SPLIT, bool CIRC>
+__global__ __launch_bounds__(256 * SPLIT, CIRC ? 5 : 4) void
+cone_bp_patch_kernel(
     const kk::BpAngle* __restrict__ tab, BpArgs A) {
   typedef __attribute__((address_space(3))) const float* lds_ptr;
   __shared__ float patch_s[SPLIT][kPatchCols * kPatchPitch];
@@ -469,28 +481,37 @@ __global__ __launch_bounds__(256 * SPLIT, 5) void cone_bp_patch_kernel(
     asm volatile("" : "+v"(ex), "+v"(ey));
     double ul = 1e30, uh = -1e30, vl = 1e30, vh = -1e30;
 #pragma unroll 1
-    for (int e = 0; e < 4; ++e) {
+    for (int e = 0; e < (CIRC ? 4 : 8); ++e) {
       const double x =
           min(ex + (e & 1 ? 15 : 0), A.nx - 1) - 0.5 * A.nx + 0.5;
       const double y =
           min(ey + (e & 2 ? 15 : 0), A.ny - 1) - 0.5 * A.ny + 0.5;
-      const double d = fma(y, P.dy, fma(x, P.dx, P.dw));
+      double d = fma(y, P.dy, fma(x, P.dx, P.dw));
+      double nu = fma(y, P.nuy, fma(x, P.nux, P.nuw));
+      const double z = CIRC || e < 4 ? Z0 : Z0 + (K - 1);
+      if constexpr (!CIRC) {
+        d = fma(z, P.dz, d);
+        nu = fma(z, P.nuz, nu);
+      }
       const double r =
           refine_rcp(d, __builtin_amdgcn_rcpf(static_cast<float>(d)));
-      const double u = fma(y, P.nuy, fma(x, P.nux, P.nuw)) * r;
-      const double v = fma(Z0, P.nvz, fma(y, P.nvy, fma(x, P.nvx, P.nvw))) * r;
-      const double w = fma(static_cast<double>(K - 1), P.nvz * r, v);
+      const double u = nu * r;
+      const double v = fma(z, P.nvz, fma(y, P.nvy, fma(x, P.nvx, P.nvw))) * r;
+      const double w =
+          CIRC ? fma(static_cast<double>(K - 1), P.nvz * r, v) : v;
       ul = fmin(ul, u);
       uh = fmax(uh, u);
       vl = fmin(vl, fmin(v, w));
       vh = fmax(vh, fmax(v, w));
     }
-    // (without the halo that the padded coordinates count; 1e-6 covers the
-    // rounding of the threads' own coordinates)
-    const double c0 = floor(ul - 1e-6) - kk::kHaloLo;
-    const double r0 = floor(vl - 1e-6) - kk::kHaloLo;
-    const double c1 = floor(uh + 1e-6) - kk::kHaloLo + 1;
-    const double r1 = floor(vh + 1e-6) - kk::kHaloLo + 1;
+    // (without the halo that the padded coordinates count; the widening
+    // covers the rounding of the threads' own coordinates: float64, or
+    // float32 offsets of up to 64 texels)
+    constexpr double kWide = CIRC ? 1e-6 : 1e-4;
+    const double c0 = floor(ul - kWide) - kk::kHaloLo;
+    const double r0 = floor(vl - kWide) - kk::kHaloLo;
+    const double c1 = floor(uh + kWide) - kk::kHaloLo + 1;
+    const double r1 = floor(vh + kWide) - kk::kHaloLo + 1;
     if (c1 < 0 || c0 >= A.cols || r1 < 0 || r0 >= A.rows) return;
     pc = static_cast<int32_t>(c0);
     pr = static_cast<int32_t>(r0);
@@ -547,34 +568,77 @@ __global__ __launch_bounds__(256 * SPLIT, 5) void cone_bp_patch_kernel(
     const double den = fma(Y, P.dy, fma(X, P.dx, P.dw));
     const double nu = fma(Y, P.nuy, fma(X, P.nux, P.nuw));
     const double nv = fma(Y, P.nvy, fma(X, P.nvx, P.nvw));
-    const float rf = __builtin_amdgcn_rcpf(static_cast<float>(den));
-    const double r = refine_rcp(den, rf);
-    const double u = fma(nu, r, -static_cast<double>(cc + kk::kHaloLo));
-    uint32_t iu;
-    float fu;
-    kk_split_nonneg(u, iu, fu);
-    const double v0 =
-        fma(fma(Z0, P.nvz, nv), r, -static_cast<double>(cr + kk::kHaloLo));
-    uint64_t V = fixed_bits(v0);
-    const uint64_t G = fixed_bits(P.nvz * r) -
-                       (static_cast<uint64_t>(kFixedHi) << 32);
-    const float w = rf * rf;
-    const uint32_t at =
-        patch_at + __umul24(iu, kPatchPitch * 4u) - (kFixedHi << 2);
+    if constexpr (CIRC) {
+      const float rf = __builtin_amdgcn_rcpf(static_cast<float>(den));
+      const double r = refine_rcp(den, rf);
+      const double u = fma(nu, r, -static_cast<double>(cc + kk::kHaloLo));
+      uint32_t iu;
+      float fu;
+      kk_split_nonneg(u, iu, fu);
+      const double v0 =
+          fma(fma(Z0, P.nvz, nv), r, -static_cast<double>(cr + kk::kHaloLo));
+      uint64_t V = fixed_bits(v0);
+      const uint64_t G = fixed_bits(P.nvz * r) -
+                         (static_cast<uint64_t>(kFixedHi) << 32);
+      const float w = rf * rf;
+      const uint32_t at =
+          patch_at + __umul24(iu, kPatchPitch * 4u) - (kFixedHi << 2);
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
-      uint32_t p;  // one shift-add of the row (not a 64-bit shift)
-      asm("v_lshl_add_u32 %0, %1, 2, %2"
-          : "=v"(p)
-          : "v"(static_cast<uint32_t>(V >> 32)), "v"(at));
-      const lds_ptr t = (lds_ptr)p;
-      const float l0 = fmaf(fu, t[kPatchPitch] - t[0], t[0]);
-      const float l1 = fmaf(fu, t[kPatchPitch + 1] - t[1], t[1]);
-      const float fv = static_cast<float>(static_cast<uint32_t>(V)) * 0x1p-32f;
-      acc[k] = fmaf(w, fmaf(fv, l1 - l0, l0), acc[k]);
-      V += G;
-      // (four voxels' reads in flight, within the register cap)
-      if (k % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+      for (int k = 0; k < K; ++k) {
+        uint32_t p;  // one shift-add of the row (not a 64-bit shift)
+        asm("v_lshl_add_u32 %0, %1, 2, %2"
+            : "=v"(p)
+            : "v"(static_cast<uint32_t>(V >> 32)), "v"(at));
+        const lds_ptr t = (lds_ptr)p;
+        const float l0 = fmaf(fu, t[kPatchPitch] - t[0], t[0]);
+        const float l1 = fmaf(fu, t[kPatchPitch + 1] - t[1], t[1]);
+        const float fv =
+            static_cast<float>(static_cast<uint32_t>(V)) * 0x1p-32f;
+        acc[k] = fmaf(w, fmaf(fv, l1 - l0, l0), acc[k]);
+        V += G;
+        // (four voxels' reads in flight, within the register cap)
+        if (k % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+      // Integer bases at the middle of the run (its ends are then as close
+      // as those of a run half as long), relative to the patch; per voxel,
+      // u(k) - ub = (e0u + (k - K / 2) e1u) / den(k), float32 numerators.
+      const double Zm = Z0 + K / 2;
+      const double den0 = fma(Zm, P.dz, den);
+      const double nu0 = fma(Zm, P.nuz, nu);
+      const double nv0 = fma(Zm, P.nvz, nv);
+      const double r0 = refine_rcp(
+          den0, __builtin_amdgcn_rcpf(static_cast<float>(den0)));
+      const double ub = floor(nu0 * r0), vb = floor(nv0 * r0);
+      const float e0u = static_cast<float>(fma(-ub, den0, nu0));
+      const float e1u = static_cast<float>(fma(-ub, P.dz, P.nuz));
+      const float e0v = static_cast<float>(fma(-vb, den0, nv0));
+      const float e1v = static_cast<float>(fma(-vb, P.dz, P.nvz));
+      const float d0f = static_cast<float>(den0);
+      const float dzf = static_cast<float>(P.dz);
+      const int32_t at =
+          static_cast<int32_t>(patch_at) +
+          (static_cast<int32_t>(ub) - cc - kk::kHaloLo) * (kPatchPitch * 4) +
+          (static_cast<int32_t>(vb) - cr - kk::kHaloLo) * 4;
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        const float fk = static_cast<float>(k - K / 2);
+        const float r = __builtin_amdgcn_rcpf(fmaf(fk, dzf, d0f));
+        const float du = fmaf(fk, e1u, e0u) * r;
+        const float dv = fmaf(fk, e1v, e0v) * r;
+        const float lu = floorf(du), lv = floorf(dv);
+        const float fu = du - lu, fv = dv - lv;
+        // (small integers: exact)
+        const int32_t i = static_cast<int32_t>(
+            fmaf(lu, static_cast<float>(kPatchPitch), lv));
+        uint32_t p;
+        asm("v_lshl_add_u32 %0, %1, 2, %2" : "=v"(p) : "v"(i), "v"(at));
+        const lds_ptr t = (lds_ptr)p;
+        const float l0 = fmaf(fu, t[kPatchPitch] - t[0], t[0]);
+        const float l1 = fmaf(fu, t[kPatchPitch + 1] - t[1], t[1]);
+        acc[k] = fmaf(r * r, fmaf(fv, l1 - l0, l0), acc[k]);
+        if (k % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+      }
     }
   }
 
@@ -947,45 +1011,75 @@ double steepest(double nx, double ny, double nw, double dx, double dy,
 }
 
 // Bounds of the columns and rows of the patch of any tile at any angle
-// (ext[0], ext[1]), for circular orbits (the host table in `tab`); false for
-// other geometries, and where a denominator may vanish over the volume or
-// coordinates leave the kernel's ranges.
+// (ext[0], ext[1]; the host table in `tab`); false where a denominator may
+// vanish over the volume or coordinates leave the kernel's ranges, and for
+// plans without a general angle that are not circular orbits (detectors
+// tilted in their own plane keep the pair kernel, whose arithmetic the
+// batched launches share).
 bool patch_extent(const std::vector<kk::BpAngle>& tab, const int32_t shape[3],
                   double ext[2]) {
   ext[0] = ext[1] = 0.0;
   if (tab.empty()) return false;
   for (int t = 0; t < 3; ++t)
     if (shape[t] <= 0 || shape[t] > 65536) return false;
+  bool circ = true, general = false;
+  for (const kk::BpAngle& e : tab) {
+    circ = circ && e.fast == 1;
+    general = general || e.fast == 0;
+  }
+  if (!circ && !general) return false;
   const double hx = 0.5 * (shape[0] - 1), hy = 0.5 * (shape[1] - 1);
   const double hz = 0.5 * shape[2] + kPatchRun;
   for (const kk::BpAngle& e : tab) {
-    if (e.fast != 1) return false;
     double least = INFINITY, most = 0.0;
+    double ul = INFINITY, uh = -INFINITY, vl = INFINITY, vh = -INFINITY;
     bool pos = true, neg = true;
-    for (int k = 0; k < 4; ++k) {
+    for (int k = 0; k < 8; ++k) {
       const double x = k & 1 ? hx : -hx, y = k & 2 ? hy : -hy;
-      const double d = e.dw + e.dx * x + e.dy * y;
+      const double z = k & 4 ? hz : -hz;
+      const double d = e.dw + e.dx * x + e.dy * y + e.dz * z;
       pos = pos && d > 0.0;
       neg = neg && d < 0.0;
       least = std::fmin(least, std::fabs(d));
       most = std::fmax(most, std::fabs(d));
-      const double u = (e.nuw + e.nux * x + e.nuy * y) / d;
-      const double v = (std::fabs(e.nvw + e.nvx * x + e.nvy * y) +
-                        hz * std::fabs(e.nvz)) / std::fabs(d);
-      if (!(std::fabs(u) < 1e5) || !(v < 1e5)) return false;
+      const double u = (e.nuw + e.nux * x + e.nuy * y + e.nuz * z) / d;
+      const double v = (e.nvw + e.nvx * x + e.nvy * y + e.nvz * z) / d;
+      if (!(std::fabs(u) < 1e5) || !(std::fabs(v) < 1e5)) return false;
+      ul = std::fmin(ul, u);
+      uh = std::fmax(uh, u);
+      vl = std::fmin(vl, v);
+      vh = std::fmax(vh, v);
     }
     if (!(pos || neg) || !(least > 1e-6 * most)) return false;
-    const double du = steepest(e.nux, e.nuy, e.nuw, e.dx, e.dy, e.dw, hx, hy);
-    double dv = 0.0;
-    for (int k = 0; k < 2; ++k)
-      dv = std::fmax(dv, steepest(e.nvx, e.nvy,
-                                  e.nvw + (k ? hz : -hz) * e.nvz, e.dx, e.dy,
-                                  e.dw, hx, hy));
-    const double run = (kPatchRun - 1) * std::fabs(e.nvz) / least;
-    // 15 voxels along x and y; three texels for the ends' floors and the
+    // 15 voxels along each axis; three texels for the ends' floors and the
     // second tap, and rounding
-    ext[0] = std::fmax(ext[0], 15.0 * du + 3.01);
-    ext[1] = std::fmax(ext[1], 15.0 * dv + run + 3.01);
+    if (circ) {
+      const double du =
+          steepest(e.nux, e.nuy, e.nuw, e.dx, e.dy, e.dw, hx, hy);
+      double dv = 0.0;
+      for (int k = 0; k < 2; ++k)
+        dv = std::fmax(dv, steepest(e.nvx, e.nvy,
+                                    e.nvw + (k ? hz : -hz) * e.nvz, e.dx,
+                                    e.dy, e.dw, hx, hy));
+      const double run = (kPatchRun - 1) * std::fabs(e.nvz) / least;
+      ext[0] = std::fmax(ext[0], 15.0 * du + 3.01);
+      ext[1] = std::fmax(ext[1], 15.0 * dv + run + 3.01);
+    } else {
+      // between points p and q of f = N / D (affine forms, D of one sign, so
+      // f lies between its least and greatest value at the volume's
+      // corners): f(q) - f(p) = (N' - f(p) D')(q - p) / D(q)
+      auto most_of = [&](double n, double d, double lo, double hi) {
+        return std::fmax(std::fabs(n - lo * d), std::fabs(n - hi * d));
+      };
+      const double du = most_of(e.nux, e.dx, ul, uh) +
+                        most_of(e.nuy, e.dy, ul, uh) +
+                        most_of(e.nuz, e.dz, ul, uh);
+      const double dv = most_of(e.nvx, e.dx, vl, vh) +
+                        most_of(e.nvy, e.dy, vl, vh) +
+                        most_of(e.nvz, e.dz, vl, vh);
+      ext[0] = std::fmax(ext[0], 15.0 * du / least + 3.01);
+      ext[1] = std::fmax(ext[1], 15.0 * dv / least + 3.01);
+    }
   }
   return true;
 }
@@ -1022,15 +1116,19 @@ int launch_bp_planes(const kk::BpSpec& S, hipStream_t stream) {
   // parts so that a CU (of 256) holds at least four wavefronts per SIMD
   const int64_t per_cu = (A.total_blocks + 255) / 256;
   const dim3 grid(unsigned(A.total_blocks));
-  if (per_cu >= 4)
-    hipLaunchKernelGGL((cone_bp_patch_kernel<kPatchRun, 1>), grid, dim3(256),
-                       0, stream, S.plan->bp, A);
-  else if (per_cu >= 2)
-    hipLaunchKernelGGL((cone_bp_patch_kernel<kPatchRun, 2>), grid, dim3(512),
-                       0, stream, S.plan->bp, A);
+  const int32_t parts = per_cu >= 4 ? 1 : per_cu >= 2 ? 2 : 4;
+  auto launch = [&](auto circ) {
+    constexpr bool C = decltype(circ)::value;
+    auto* kernel = parts == 1   ? &cone_bp_patch_kernel<kPatchRun, 1, C>
+                   : parts == 2 ? &cone_bp_patch_kernel<kPatchRun, 2, C>
+                                : &cone_bp_patch_kernel<kPatchRun, 4, C>;
+    hipLaunchKernelGGL(kernel, grid, dim3(256 * parts), 0, stream, S.plan->bp,
+                       A);
+  };
+  if (S.plan->bp_all_circ)
+    launch(std::true_type{});
   else
-    hipLaunchKernelGGL((cone_bp_patch_kernel<kPatchRun, 4>), grid, dim3(1024),
-                       0, stream, S.plan->bp, A);
+    launch(std::false_type{});
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return kk::hip_fail(e, "cone_bp_patch_kernel");
   return KK_OK;

@@ -247,8 +247,8 @@ class VolumeTexture:
 class ProjectionTexture:
     """Backprojection layout of projections: ``[angle][rows+3][cols+3]`` of
     (value, next-row) float2 pairs with a zero halo for the general kernel,
-    or planes (plain floats, column-major) for the kernel of circular orbits;
-    see ``include/kernelkit_hip.h``.  :attr:`data` and :attr:`ptr` are the
+    or planes (plain floats, column-major) for the patch kernel; see
+    ``include/kernelkit_hip.h``.  :attr:`data` and :attr:`ptr` are the
     pairs, made from the planes when asked for, as in
     :class:`VolumeTexture`."""
 

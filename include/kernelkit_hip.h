@@ -117,7 +117,9 @@ int kk_projections_to_bp_texture(const float* proj, int32_t n_angles,
 /* BP planes: projections as plain floats, column-major, [angle][col][rows +
  * KK_PLANE_GAP] with zeros after each column, which the launches of
  * kk_cone_bp_planes and kk_sirt_bp_update_planes read: for circular orbits
- * about z whose 16 x 16 x 16 voxel tiles project onto at most 64 x 64 pixels.
+ * about z and for plans with an angle of no special form (not for detectors
+ * tilted in their own plane alone), if the volume's 16 x 16 x 16 voxel tiles
+ * project onto at most 64 x 64 pixels.
  * kk_bp_reads_planes says whether the plan's parameters with a rows x cols
  * detector and the volume's shape are such (1) or not (0).
  * kk_residual_to_bp_planes: planes of the SIRT residual (proj - y) * R. */
@@ -374,8 +376,8 @@ int kk_fp_line_spacing(const double* params, int32_t n_angles,
 int kk_bp_table(const double* params, int32_t n_angles, void* out);
 
 /* Host-only: bounds of the detector columns and rows that any 16 x 16 x 16
- * voxel tile projects onto (out[0], out[1]); -1 if the orbit is not circular
- * about z.  What kk_bp_reads_planes decides on. */
+ * voxel tile projects onto (out[0], out[1]); -1 if there are no such bounds
+ * or the geometry is one that the pairs serve.  What kk_bp_reads_planes decides on. */
 int kk_bp_patch_extent(const double* params, int32_t n_angles,
                        const int32_t vol_shape[3], double out[2]);
 

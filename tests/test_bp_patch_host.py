@@ -22,10 +22,12 @@ def _extent(pgs, vg):
     ((50, 33, 90), 60.0, 200.0, 2.5, (0, 0, 0)),
     ((17, 80, 7), 60.0, 30.0, 3.0, (4.0, -3.0, 9.0)),
 ])
-def test_extent_covers_every_tile(shape, sod, odd, pixel, centre):
+@pytest.mark.parametrize("pert", [{}, {"wobble_deg": 1.0, "drift_px": 3.0},
+                                  {"wobble_deg": 20.0, "tilt_deg": 15.0}])
+def test_extent_covers_every_tile(shape, sod, odd, pixel, centre, pert):
     """The taps of every 16 x 16 x 16 tile (z beyond the volume to the end of
     its run) span no more columns and rows than the bounds."""
-    pgs = workloads.circular_geometry(37, sod, odd, 40, 40, pixel)
+    pgs = workloads.circular_geometry(37, sod, odd, 40, 40, pixel, **pert)
     lo = np.array(centre) - 0.5 * np.array(shape)
     vg = kk.resolve_volume_geometry(shape=shape, voxel_size=1.0,
                                     extent_min=tuple(lo),
@@ -52,9 +54,10 @@ def test_extent_covers_every_tile(shape, sod, odd, pixel, centre):
 
 def test_extent_refuses_other_geometries():
     vg = kk.resolve_volume_geometry(shape=(32, 32, 32), voxel_size=1.0)
-    for kw in (dict(tilt_deg=1.0), dict(wobble_deg=1.0)):
-        pgs = workloads.circular_geometry(8, 100.0, 50.0, 40, 40, 1.0, **kw)
-        assert _extent(pgs, vg)[1][0] < 0
-    # the source's plane crosses the volume
-    pgs = workloads.circular_geometry(8, 10.0, 50.0, 40, 40, 1.0)
+    pgs = workloads.circular_geometry(8, 100.0, 50.0, 40, 40, 1.0,
+                                      tilt_deg=1.0)
     assert _extent(pgs, vg)[1][0] < 0
+    # the source's plane crosses the volume
+    for kw in ({}, dict(wobble_deg=1.0)):
+        pgs = workloads.circular_geometry(8, 10.0, 50.0, 40, 40, 1.0, **kw)
+        assert _extent(pgs, vg)[1][0] < 0

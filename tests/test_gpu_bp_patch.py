@@ -18,10 +18,10 @@ def _dev(a):
     return torch.from_numpy(np.ascontiguousarray(a, dtype=np.float32)).cuda()
 
 
-def _case(shape, angles, rows, cols, pixel, sod=None):
+def _case(shape, angles, rows, cols, pixel, sod=None, **pert):
     sod = sod or 4.0 * max(shape)
     pgs = workloads.circular_geometry(angles, sod, 0.5 * sod, rows, cols,
-                                      pixel)
+                                      pixel, **pert)
     vg = kk.resolve_volume_geometry(shape=shape, voxel_size=1.0)
     y = np.random.default_rng(rows + cols).standard_normal(
         (angles, rows, cols)).astype(np.float32)
@@ -59,6 +59,37 @@ def test_patch_kernel_matches_oracle(size, device):
     np.testing.assert_array_equal(A.backprojector.projections.cpu().numpy(), y)
     x2 = A.T(_dev(y), out=x.clone(), additive=True)
     assert_parity(x2.cpu().numpy(), 2 * ref)
+
+
+@pytest.mark.parametrize("pert", [
+    dict(wobble_deg=1.0, drift_px=3.0),
+    dict(wobble_deg=12.0, tilt_deg=30.0, drift_px=2.0)],
+    ids=["wobble", "strong"])
+@pytest.mark.parametrize("size", SIZES, ids=lambda s: "x".join(map(str, s[0]))
+                         + f"-{s[1]}-{s[2]}x{s[3]}@{s[4]}")
+def test_general_geometries_match_oracle(size, pert, device):
+    """The same sizes on wobbling orbits (with the kernel that the plan
+    picks; all but the largest patches of the strong ones fit)."""
+    size = (*size[:5], size[5] if len(size) > 5 else 5.0 * max(size[0]))
+    pgs, vg, y = _case(*size, **pert)
+    A = kk.XrayTransform(pgs, vg)
+    assert A.backprojector.kernel.reads_planes or size[0] == (1, 1, 1) or \
+        pert["wobble_deg"] > 1
+    x = A.T(_dev(y))
+    ref = oracle.cone_bp(y, pgs, vg)
+    assert_parity(x.cpu().numpy(), ref)
+    x2 = A.T(_dev(y), out=x.clone(), additive=True)
+    assert_parity(x2.cpu().numpy(), 2 * ref)
+
+
+def test_mixed_angles_match_oracle(device):
+    """Circular, tilted and wobbling angles in one plan."""
+    pgs, vg, y = _case((40, 36, 33), 12, 50, 60, 1.1)
+    pgs = pgs[:4] + _case((40, 36, 33), 12, 50, 60, 1.1, tilt_deg=3.0)[0][
+        4:8] + _case((40, 36, 33), 12, 50, 60, 1.1, wobble_deg=2.0)[0][8:]
+    A = kk.XrayTransform(pgs, vg)
+    assert A.backprojector.kernel.reads_planes
+    assert_parity(A.T(_dev(y)).cpu().numpy(), oracle.cone_bp(y, pgs, vg))
 
 
 def test_axis_orders_and_texture_across_geometries(device):
