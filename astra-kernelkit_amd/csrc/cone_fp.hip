@@ -13,19 +13,15 @@
 //   memory); each output pixel is written exactly once;
 // * the volume is read from slice-major frame textures of (value,
 //   b-neighbour) float2 pairs with a zero halo (kk_internal.h), so a sample
-//   is: one FMA per coordinate, a clamp into the halo, v_cvt_u32 + v_fract
-//   for the tap index and weight (the slice index itself is converted to
-//   float64 with scalar integer instructions), and ONE 16-byte load for
-//   all four taps (~15 VALU instructions per sample in the unclamped
-//   interior; measured on MI355X at 512^3 / 720 angles the kernel keeps
-//   the texture-address units ~85% busy, ~14 cycles per 64-lane gather,
-//   and the VALU about as busy: it is close to both issue limits);
-// * sample coordinates are evaluated directly, x_b(i) = a1*i + beta, instead
-//   of the reference's running sums, so the per-sample error does not grow
-//   along the ray;
-// * lanes of a wavefront are 64 consecutive detector rows of one column and
-//   every thread traces R rows 64 apart.  For rotation about z this makes a
-//   wave sample consecutive z voxels of the same (x or y) row, contiguous
+//   is: one 64-bit add per coordinate, whose high word is the tap index and
+//   low word the weight, one minimum into the halo, and ONE 16-byte load for
+//   all four taps;
+// * sample coordinates are 64-bit fixed point, a1*i + beta to 2^-33 voxel per
+//   slice from the middle one: below the weights' float32 rounding, where the
+//   reference's float32 running sums grow along the ray;
+// * lanes of a wavefront are 32 consecutive detector rows of two neighbouring
+//   columns (fp_lanes).  For rotation about z this makes a
+//   wave sample consecutive z voxels of the same (x or y) rows, contiguous
 //   memory;
 // * the slice loop is wave-uniform: it covers the union of the wave's ray
 //   supports (samples outside a ray's support clamp into the zero halo), so
@@ -41,15 +37,11 @@
 //   neighbouring column tiles (angle fastest), groups ordered angle group
 //   -> column-tile group -> row band, and each group's ids go to one XCD:
 //   neighbouring angles and columns read nearly the same texture lines, so
-//   its L2 serves them (measured on MI355X at 512^3 / 720 angles: 86.9 ms
-//   with 16 x 8, 91.0 ms with runs of 64 angles of one column tile, 110 ms
-//   with column tiles fastest and workgroups dealt round-robin to the
-//   XCDs; 16 x 4, 32 x 4 and 16 x 16 took 87.7, 88.1 and 90.5 ms).  In
-//   batches (256-thread workgroups) groups of 16 x 16 took the batched
-//   forward projection of the 64-problem workload from 104.8 to 98.1 ms.
+//   its L2 serves them.
 #include <algorithm>
 #include <cmath>
 #include <new>
+#include <type_traits>
 #include <vector>
 
 #include "kk_internal.h"
@@ -57,22 +49,20 @@
 namespace {
 
 constexpr int kWave = 64;
-// Detector columns per workgroup, one per wavefront.  Single problems: 16
-// (1024 threads); the wavefronts of a workgroup share one CU's L1 and move
-// through the slices nearly in step, so neighbouring columns' taps hit
-// there (measured on MI355X at 512^3 / 720 angles: 3-8% faster than 8 or
-// 4 columns).  Batches of small detectors: 4.
-constexpr int kColsSingle = 16;
+// Wavefronts per workgroup: they share one CU's L1 and move through the slices
+// nearly in step, so neighbouring columns' taps hit there (200^3 tilted 1.02,
+// 1.02 and 1.13 ms with 4, 8 and 16, 300^3 3.15, 3.28 and 3.63 ms).
+constexpr int kColsSingle = 4;
 constexpr int kColsBatch = 4;
 // The workgroups of kGroupAngles consecutive angles x kGroupCols (single
 // problems; kGroupColsBatch in batches) neighbouring column tiles go to
-// one XCD together.  An XCD holds 64 single-problem workgroups (32 CUs x
-// 2 of 1024 threads) or 256 batch workgroups (32 x 8 of 256 threads);
-// measured on MI355X: 16 x 8 and 16 x 16 were the fastest groups.  These
+// one XCD together: an XCD holds 256 workgroups of 256 threads (32 CUs x 8).
+// Measured on MI355X, 300^3 tilted: 2.98 ms with 16 x 32, 3.06 with 16 x 16,
+// 3.12 with 8 x 32, 3.21 with 8 x 16, 4.15 with 4 x 32.  These
 // are upper bounds: a group size is the one in [ceil(cap / 2), cap] that
 // pads the angles or column tiles least (group_size).
 constexpr int32_t kGroupAngles = 16;
-constexpr int32_t kGroupCols = 8;
+constexpr int32_t kGroupCols = 32;
 constexpr int32_t kGroupColsBatch = 16;
 
 // Group size for n items, at most cap: the g in [ceil(cap / 2), cap] whose
@@ -110,6 +100,7 @@ struct FpArgs {
   int64_t rs0, rs1, rs2;
   int32_t rows, cols, n_angles;
   int32_t row_tiles, col_tiles;
+  int32_t row_shift;  // a wavefront is 2^row_shift rows x 64 >> row_shift cols
   int32_t mode;  // 0: out = p, 1: out += p, 2: out = (p - y) * R
   int32_t xcd_group;
   // workgroup groups: grp_a angles x grp_c column tiles (ids past the
@@ -141,27 +132,6 @@ __device__ __forceinline__ void clip_range(float a, float beta, float n1,
   hi = fminf(hi, fmaxf(t0, t1));
 }
 
-// Narrow [lo, hi] to the slices i with 1 <= a*i + beta <= n1 - 1: one
-// voxel inside the clamp range [0, n1], which covers the float32 error of
-// this estimate (~1e-4 voxel).  A coordinate is linear in i, so for flat
-// slopes the end points decide.
-__device__ __forceinline__ void inner_range(float a, float beta, float n1,
-                                            float& lo, float& hi) {
-  if (fabsf(a) < 1e-3f) {
-    const float e0 = fmaf(a, lo, beta), e1 = fmaf(a, hi, beta);
-    if (!(fminf(e0, e1) >= 1.f && fmaxf(e0, e1) <= n1 - 1.f)) {
-      lo = 3e38f;
-      hi = -3e38f;
-    }
-    return;
-  }
-  const float inv = 1.f / a;
-  const float t0 = (1.f - beta) * inv;
-  const float t1 = (n1 - 1.f - beta) * inv;
-  lo = fmaxf(lo, fminf(t0, t1));
-  hi = fminf(hi, fmaxf(t0, t1));
-}
-
 // Bilinear value from the 16-byte tap record (v[b][c], v[b+1][c],
 // v[b][c+1], v[b+1][c+1]): lerp along b, then along c.
 __device__ __forceinline__ float bilerp(kk_float4u t, float fb, float fc) {
@@ -178,45 +148,93 @@ struct SliceTaps {
   float fc[R];
 };
 
-// Coordinates, weights and tap loads of slice i for R rays.  COLC (NB = 1):
-// the b slope/intercept are shared by the R rays.  CLAMP = false: every
-// coordinate is known to lie inside the clamp range, which is then skipped.
-template <int R, int NB, bool CLAMP>
-__device__ __forceinline__ void fetch_slice(
-    const char* __restrict__ frame, uint32_t sab, uint32_t sbb, double nb1,
-    double nc1, const double (&a1)[NB], const double (&b1)[NB],
-    const double (&a2)[R], const double (&b2)[R], int32_t i,
-    SliceTaps<R, NB>& s) {
-  constexpr bool COLC = NB == 1;
-  const double fi = kk_uniform_i2d(i);
-  const char* slice = frame + static_cast<size_t>(i) * sab;
-  uint32_t offb = 0;
-  if constexpr (COLC) {
-    uint32_t ib;
-    if constexpr (CLAMP)
-      kk_fp_coord(a1[0], b1[0], fi, nb1, ib, s.fb[0]);
-    else
-      kk_fp_coord_in(a1[0], b1[0], fi, ib, s.fb[0]);
-    offb = __umul24(ib, sbb);
-    // one multiply for the R rays (not a multiply-add per ray)
-    asm volatile("" : "+v"(offb));
+// x as 64-bit fixed point with 32 fraction bits (|x| < 2^31).
+__device__ __forceinline__ int64_t to_fixed(double x) {
+  const double fl = floor(x);
+  const uint32_t lo = static_cast<uint32_t>(
+      fmin(fma(x - fl, 4294967296.0, 0.5), 4294967295.0));
+  return static_cast<int64_t>(
+      (static_cast<uint64_t>(static_cast<uint32_t>(static_cast<int32_t>(fl)))
+       << 32) |
+      lo);
+}
+
+// Coordinates of a thread's R rays at a slice, and their steps per slice, as
+// 64-bit fixed point (to_fixed): the high word is the padded element, the low
+// word the weight.  NB = 1: the b coordinate is shared by the R rays (column-
+// coherent angles).  Coordinates outside the volume (below the halo: a
+// negative element, huge as unsigned) go to element n + 1, whose taps are all
+// halo zeros whatever the weight: one unsigned minimum.
+//
+// (A sample took float64 coordinates before, their clamps or a second pass for
+// the slices that lie inside for a whole wavefront: 27 vector instructions a
+// gather, now 22.  200^3 tilted 1.40 -> 1.00 ms together with fp_lanes, 300^3
+// 4.83 -> 3.0 ms, 400^3 / 200 wobbling angles 10.3 -> 8.0 ms, 64^3 58 -> 46 us.
+// The address units are 63% busy, 16 cycles a gather; a deeper pipeline was
+// slower, so what is left is the L2's latency and the L1's misses.)
+template <int R, int NB>
+struct RayWalk {
+  int64_t b[NB], c[R];
+  int64_t gb[NB], gc[R];
+};
+
+// Coordinate a i + b at slice mid, the middle of the slices that the ray
+// meets, and its step: the step's rounding (2^-33 voxel per slice) adds up over
+// half of them at most, and cancels in the ray's sum (a ray that only grazes
+// the volume, whose sum a reconstruction divides by, loses no accuracy).
+// A ray nearly parallel to the slices, whose coordinates leave the fixed-point
+// range, is inside the volume (n1 - 1 voxels) at one slice at most: it has its
+// coordinate there, and at the others one outside.
+__device__ __forceinline__ void fixed_ray(double a, double b, int32_t na,
+                                          int32_t mid, float n1, int64_t& at,
+                                          int64_t& step) {
+  constexpr double kRange = 1073741824.0;  // 2^30
+  double g = a, x = fma(a, static_cast<double>(mid), b);
+  int32_t far = 0;
+  if (!(fabs(a) * static_cast<double>(na) + fabs(b) < kRange)) {
+    const double r = __builtin_amdgcn_rcp(a);
+    const double i = rint(fmin(
+        fmax((0.5 * n1 - b) * fma(r, fma(-a, r, 1.0), r), 0.0), na - 1.0));
+    x = fmin(fmax(fma(a, i, b), -kRange), kRange);
+    g = copysign(kRange / 2 / static_cast<double>(na), a);
+    far = mid - static_cast<int32_t>(i);
   }
+  step = to_fixed(g);
+  at = to_fixed(x) + static_cast<int64_t>(far) * step;
+}
+
+__device__ __forceinline__ void split_fixed(int64_t x, uint32_t n1,
+                                            uint32_t& idx, float& frac) {
+  const uint64_t u = static_cast<uint64_t>(x);
+  idx = min(static_cast<uint32_t>(u >> 32), n1);
+  frac = static_cast<float>(static_cast<uint32_t>(u)) * 0x1p-32f;
+}
+
+// Weights and tap loads of one slice for R rays; the walk moves on to the
+// next.
+template <int R, int NB>
+__device__ __forceinline__ void fetch_slice(const char* __restrict__ slice,
+                                            uint32_t sbb, uint32_t nb1,
+                                            uint32_t nc1, RayWalk<R, NB>& w,
+                                            SliceTaps<R, NB>& s) {
+  uint32_t ob = 0;
 #pragma unroll
   for (int k = 0; k < R; ++k) {
-    uint32_t ob = offb;
-    if constexpr (!COLC) {
+    if (k < NB) {
       uint32_t ib;
-      if constexpr (CLAMP)
-        kk_fp_coord(a1[k], b1[k], fi, nb1, ib, s.fb[k]);
-      else
-        kk_fp_coord_in(a1[k], b1[k], fi, ib, s.fb[k]);
+      split_fixed(w.b[k], nb1, ib, s.fb[k]);
       ob = __umul24(ib, sbb);
+      // one multiply for the R rays (not a multiply-add per ray)
+      if constexpr (NB == 1) asm volatile("" : "+v"(ob));
+      w.b[k] += w.gb[k];
+      asm volatile("" : "+v"(w.b[k]));
     }
     uint32_t ic;
-    if constexpr (CLAMP)
-      kk_fp_coord(a2[k], b2[k], fi, nc1, ic, s.fc[k]);
-    else
-      kk_fp_coord_in(a2[k], b2[k], fi, ic, s.fc[k]);
+    split_fixed(w.c[k], nc1, ic, s.fc[k]);
+    w.c[k] += w.gc[k];
+    // (coordinates stay one register pair each, stepped: the optimizer would
+    // split them into words and multiples of the step)
+    asm volatile("" : "+v"(w.c[k]));
     s.t[k] = kk_ld4(slice, ob + (ic << 3));
   }
 }
@@ -229,9 +247,9 @@ __device__ __forceinline__ void add_slice(const SliceTaps<R, NB>& s,
     acc[k] += bilerp(s.t[k], s.fb[NB == 1 ? 0 : k], s.fc[k]);
 }
 
-// One tracing pass over slices [i0, i1] (wave-uniform) for R rays of a
-// thread.  PIPE software-pipelines the pass: the taps of slice i + 1 are
-// requested before slice i is interpolated, so a wavefront keeps two
+// Trace slices [i0, i1] (wave-uniform) for R rays of a thread from their
+// coordinates at i0.  PIPE software-pipelines the pass: the taps of slice
+// i + 1 are requested before slice i is interpolated, so a wavefront keeps two
 // slices of gathers in flight (two register buffers, the loop unrolled by
 // two so that they swap roles without copies; the request past i1 repeats
 // slice i1 and is discarded).  The scheduling barriers keep each request
@@ -239,21 +257,17 @@ __device__ __forceinline__ void add_slice(const SliceTaps<R, NB>& s,
 // next to their use).  Measured on MI355X at 512^3 / 720 angles: 5% faster
 // than one slice in flight; three slices in flight (at 6 instead of 8
 // wavefronts per SIMD, for the registers) are no faster than two.
-template <int R, int NB, bool CLAMP, bool PIPE>
+template <int R, int NB, bool PIPE>
 __device__ __forceinline__ void trace(const kk::FpAngle& P,
                                       const char* __restrict__ frame,
-                                      const double (&a1)[NB],
-                                      const double (&b1)[NB],
-                                      const double (&a2)[R],
-                                      const double (&b2)[R], int32_t i0,
+                                      RayWalk<R, NB>& w, int32_t i0,
                                       int32_t i1, float (&acc)[R]) {
-  if (i0 > i1) return;
-  const double nb1 = static_cast<double>(P.nb + 1);
-  const double nc1 = static_cast<double>(P.nc + 1);
+  const uint32_t nb1 = static_cast<uint32_t>(P.nb) + 1;
+  const uint32_t nc1 = static_cast<uint32_t>(P.nc) + 1;
   const uint32_t sab = P.sab, sbb = P.sbb;
   auto fetch = [&](int32_t i, SliceTaps<R, NB>& s) {
-    fetch_slice<R, NB, CLAMP>(frame, sab, sbb, nb1, nc1, a1, b1, a2, b2,
-                              min(i, i1), s);
+    fetch_slice<R, NB>(frame + static_cast<size_t>(min(i, i1)) * sab, sbb,
+                       nb1, nc1, w, s);
   };
   if constexpr (!PIPE) {
     for (int32_t i = i0; i <= i1; ++i) {
@@ -263,18 +277,87 @@ __device__ __forceinline__ void trace(const kk::FpAngle& P,
     }
   } else {
     SliceTaps<R, NB> A, B;
-    fetch(i0, A);
-    for (int32_t i = i0;;) {
+    int32_t i = i0;
+    if ((i1 - i0) % 2 == 0) {
+      fetch(i, A);
+      add_slice(A, acc);
+      if (++i > i1) return;
+    }
+    fetch(i, A);
+    for (; i < i1; i += 2) {
       fetch(i + 1, B);
       __builtin_amdgcn_sched_barrier(0);
       add_slice(A, acc);
-      if (++i > i1) break;
-      fetch(i + 1, A);
+      fetch(i + 2, A);
       __builtin_amdgcn_sched_barrier(0);
       add_slice(B, acc);
-      if (++i > i1) break;
     }
   }
+}
+
+// Rays that graze the volume.  The fixed-point coordinates are good to ~1e-10
+// voxel, the weights made of them to 1e-10 of a voxel's value: less than their
+// float32 rounding except right at the low faces (padded coordinates just above
+// 0), where a float64 coordinate gives a weight of 24 good bits however small it
+// is.  A reconstruction divides by the sums of weights, so rays that nowhere
+// reach deeper than kGraze into the volume are traced again in float64, over
+// their own few slices.
+constexpr float kGraze = 0x1p-6f;
+
+// Narrows [lo, hi] to the slices where a i + b lies in [0, n1] (to 1e-3 voxel
+// too many) and [dlo, dhi] to those where it is at least kGraze.
+__device__ __forceinline__ void graze_range(float a, float b, float n1,
+                                            float& lo, float& hi, float& dlo,
+                                            float& dhi) {
+  const float inv = 1.f / (fabsf(a) > 1e-7f ? a : 1e-7f);
+  const float t = -b * inv, g = kGraze * inv, w = n1 * inv;
+  const float e = 1e-3f * fabsf(inv);
+  lo = fmaxf(lo, fminf(t, t + w) - e);
+  hi = fminf(hi, fmaxf(t, t + w) + e);
+  dlo = fmaxf(dlo, fminf(t + g, t + w));
+  dhi = fminf(dhi, fmaxf(t + g, t + w));
+}
+__device__ __forceinline__ bool grazes(double a1, double b1, double a2,
+                                       double b2, float nb1, float nc1,
+                                       float last, float& lo, float& hi) {
+  float dlo = 0.f, dhi = last;
+  lo = 0.f;
+  hi = last;
+  graze_range(static_cast<float>(a1), static_cast<float>(b1), nb1, lo, hi,
+              dlo, dhi);
+  graze_range(static_cast<float>(a2), static_cast<float>(b2), nc1, lo, hi,
+              dlo, dhi);
+  lo = ceilf(lo);
+  hi = floorf(hi);
+  return lo <= hi && !(ceilf(dlo) <= floorf(dhi));
+}
+
+// The sum of ray (row, col) if it grazes the volume.  taps(i, ib, ic) are the
+// four values at padded element (ib, ic) of slice i.
+template <class Taps>
+__device__ __forceinline__ bool graze_sum(const kk::FpAngle& P, int32_t row,
+                                          int32_t col, float& sum,
+                                          Taps taps) {
+  double a1, b1, a2, b2;
+  float lo, hi;
+  if (!kk_fp_ray(P, row, col, a1, b1, a2, b2) ||
+      !grazes(a1, b1, a2, b2, static_cast<float>(P.nb + 1),
+              static_cast<float>(P.nc + 1), static_cast<float>(P.na - 1), lo,
+              hi))
+    return false;
+  const double nb1 = static_cast<double>(P.nb + 1);
+  const double nc1 = static_cast<double>(P.nc + 1);
+  sum = 0.f;
+  for (int32_t i = static_cast<int32_t>(lo); i <= static_cast<int32_t>(hi);
+       ++i) {
+    const double fi = static_cast<double>(i);
+    uint32_t ib, ic;
+    float fb, fc;
+    kk_fp_coord(a1, b1, fi, nb1, ib, fb);
+    kk_fp_coord(a2, b2, fi, nc1, ic, fc);
+    sum += bilerp(taps(i, ib, ic), fb, fc);
+  }
+  return true;
 }
 
 // One workgroup's tile (row band rt, angle, column tile ct) of logical
@@ -287,90 +370,84 @@ __device__ __forceinline__ void fp_tile_at(
     int32_t ang, int32_t ct, int32_t rt) {
   constexpr int NB = ALL_COLC ? 1 : R;
   const int32_t lane = int32_t(threadIdx.x) & (kWave - 1);
-  const int32_t col = ct * COLS + int32_t(threadIdx.x) / kWave;
-  const int32_t row0 = rt * (kWave * R) + lane;
+  const int32_t rows = 1 << A.row_shift;  // of a wavefront
+  const int32_t col =
+      ((ct * COLS + int32_t(threadIdx.x) / kWave) << (6 - A.row_shift)) +
+      (lane >> A.row_shift);
+  const int32_t row0 = rt * (rows * R) + (lane & (rows - 1));
 
   const kk::FpAngle& P = tab[ti];
   const float nb1 = static_cast<float>(P.nb + 1);
   const float nc1 = static_cast<float>(P.nc + 1);
   const float last = static_cast<float>(P.na - 1);
 
-  double a1[NB], b1[NB], a2[R], b2[R];
+  RayWalk<R, NB> w;
   float wscale[R];
   int32_t ilo = 0x7fffffff, ihi = -1;
-  float jl = 0.f, jh = last;  // this thread's rays all inside
+  int32_t mb[NB], mc[R];  // slices of the coordinates in w
+  bool graze = false;
 #pragma unroll
   for (int k = 0; k < R; ++k) {
-    const int32_t row = row0 + kWave * k;
+    const int32_t row = row0 + rows * k;
     // rays outside the detector, or parallel to the slices, contribute
-    // nothing: they are parked at padded coordinate 1 (inside every
-    // range, so also valid for unclamped passes) with weight 0 (for
+    // nothing: they are parked at padded coordinate 1 with weight 0 (for
     // column-coherent angles the b part of every ray of the thread equals
     // that of its first ray)
-    double ra1, rb1;
+    double a1, b1, a2, b2;
     const bool ok = row < A.rows && col < A.cols &&
-                    kk_fp_ray(P, row, col, ra1, rb1, a2[k], b2[k]);
-    if (k < NB) {
-      a1[k] = ok ? ra1 : 0.0;
-      b1[k] = ok ? rb1 : 1.0;
-    }
-    wscale[k] = 0.f;
-    if (!ok) {
-      a2[k] = 0.0;
-      b2[k] = 1.0;
-      continue;
-    }
-    wscale[k] = kk_fp_weight(P, ra1, a2[k]);
-    const float fa1 = static_cast<float>(ra1), fb1 = static_cast<float>(rb1);
-    const float fa2 = static_cast<float>(a2[k]);
-    const float fb2 = static_cast<float>(b2[k]);
+                    kk_fp_ray(P, row, col, a1, b1, a2, b2);
+    wscale[k] = ok ? kk_fp_weight(P, a1, a2) : 0.f;
+    a1 = ok ? a1 : 0.0;
+    b1 = ok ? b1 : 1.0;
+    a2 = ok ? a2 : 0.0;
+    b2 = ok ? b2 : 1.0;
     float lo = 0.f, hi = last;
-    clip_range(fa1, fb1, nb1, last, lo, hi);
-    clip_range(fa2, fb2, nc1, last, lo, hi);
-    if (lo <= hi + 2.f) {
+    clip_range(static_cast<float>(a1), static_cast<float>(b1), nb1, last, lo,
+               hi);
+    clip_range(static_cast<float>(a2), static_cast<float>(b2), nc1, last, lo,
+               hi);
+    float glo, ghi;
+    graze = graze || (ok && grazes(a1, b1, a2, b2, nb1, nc1, last, glo, ghi));
+    const int32_t mid = static_cast<int32_t>(
+        fminf(fmaxf(0.5f * (lo + hi), 0.f), last));
+    if (k < NB) {
+      mb[k] = mid;
+      fixed_ray(a1, b1, P.na, mid, nb1, w.b[k], w.gb[k]);
+    }
+    mc[k] = mid;
+    fixed_ray(a2, b2, P.na, mid, nc1, w.c[k], w.gc[k]);
+    if (ok && lo <= hi + 2.f) {
       ilo = min(ilo, max(0, static_cast<int32_t>(floorf(lo)) - 1));
       ihi = max(ihi, min(P.na - 1, static_cast<int32_t>(ceilf(hi)) + 1));
     }
-    inner_range(fa1, fb1, nb1, jl, jh);
-    inner_range(fa2, fb2, nc1, jl, jh);
   }
   ilo = kk_wave_min(ilo);
   ihi = kk_wave_max(ihi);
-  // slices where every ray of the wave is inside: no clamps there
-  int32_t jlo = 1, jhi = 0;
-  if (jl <= jh) {
-    jlo = max(0, static_cast<int32_t>(ceilf(jl)));
-    jhi = min(P.na - 1, static_cast<int32_t>(floorf(jh)));
-  }
-  jlo = max(kk_wave_max(jlo), ilo);
-  jhi = min(kk_wave_min(jhi), ihi);
 
   float acc[R];
 #pragma unroll
   for (int k = 0; k < R; ++k) acc[k] = 0.f;
-  const char* frame = A.tex + P.tex_off;
   if (ilo <= ihi) {
-    // clamped head, unclamped interior, clamped tail (or one clamped pass)
-    const bool split = jlo <= jhi;
-    const int32_t h1 = split ? jlo - 1 : ihi;
-    if constexpr (ALL_COLC) {
-      trace<R, 1, true, PIPE>(P, frame, a1, b1, a2, b2, ilo, h1, acc);
-      if (split) {
-        trace<R, 1, false, PIPE>(P, frame, a1, b1, a2, b2, jlo, jhi, acc);
-        trace<R, 1, true, PIPE>(P, frame, a1, b1, a2, b2, jhi + 1, ihi,
-                                acc);
-      }
-    } else {
-      if (P.colc) {
-        const double a1c[1] = {a1[0]}, b1c[1] = {b1[0]};
-        trace<R, 1, true, PIPE>(P, frame, a1c, b1c, a2, b2, ilo, ihi, acc);
-      } else {
-        trace<R, R, true, PIPE>(P, frame, a1, b1, a2, b2, ilo, h1, acc);
-        if (split) {
-          trace<R, R, false, PIPE>(P, frame, a1, b1, a2, b2, jlo, jhi,
-                                   acc);
-          trace<R, R, true, PIPE>(P, frame, a1, b1, a2, b2, jhi + 1, ihi,
-                                  acc);
+#pragma unroll
+    for (int k = 0; k < NB; ++k)
+      w.b[k] += static_cast<int64_t>(ilo - mb[k]) * w.gb[k];
+#pragma unroll
+    for (int k = 0; k < R; ++k)
+      w.c[k] += static_cast<int64_t>(ilo - mc[k]) * w.gc[k];
+    const char* frame = A.tex + P.tex_off;
+    trace<R, NB, PIPE>(P, frame, w, ilo, ihi, acc);
+    if (graze) {
+#pragma unroll 1
+      for (int32_t k = 0; k < R; ++k) {
+        float v;
+        if (row0 + rows * k < A.rows &&
+            graze_sum(P, row0 + rows * k, col, v,
+                      [&](int32_t i, uint32_t ib, uint32_t ic) {
+                        return kk_ld4(frame + static_cast<size_t>(i) * P.sab,
+                                      __umul24(ib, P.sbb) + (ic << 3));
+                      })) {
+#pragma unroll
+          for (int t = 0; t < R; ++t) acc[t] = t == k ? v : acc[t];
         }
       }
     }
@@ -378,7 +455,7 @@ __device__ __forceinline__ void fp_tile_at(
 
 #pragma unroll
   for (int k = 0; k < R; ++k) {
-    const int32_t row = row0 + kWave * k;
+    const int32_t row = row0 + rows * k;
     if (row >= A.rows || col >= A.cols) continue;
     float val = acc[k] * wscale[k];
     const int64_t o = ang * A.os0 + row * A.os1 + col * A.os2;
@@ -438,24 +515,17 @@ __device__ __forceinline__ void fp_tile(const kk::FpAngle* __restrict__ tab,
   }
 }
 
-// Register caps: 8 wavefronts per SIMD up to two rows per thread, 6 at
-// four (5 in the batch kernel), whose float64 ray data would otherwise
-// spill.
-constexpr int fp_min_blocks(int r) {
-  return (r <= 2 ? 32 : 24) / kColsSingle;
-}
-constexpr int fp_batch_min_blocks(int r) {
-  return (r <= 2 ? 32 : 20) / kColsBatch;
-}
-// Slice pipelining where the second tap buffer fits the register cap
-// without spilling.
-constexpr bool fp_pipe(int r) { return r <= 2; }
-constexpr bool fp_batch_pipe(int r) { return r <= 1; }
+// Wavefronts per SIMD (register caps): 8 up to two rows per thread, 5 at
+// four.
+constexpr int fp_waves(int r) { return r <= 2 ? 8 : 5; }
+// Slice pipelining: with one row per thread (200^3 tilted 1.06 ms, without
+// 1.25; with two rows 1.30 and 1.18).
+constexpr bool fp_pipe(int r) { return r <= 1; }
 
 // PTRS: output through the table of entry pointers (kk_cone_fp_ptrs); a
 // separate instantiation, so the plain kernel's code is unchanged.
 template <int R, bool ALL_COLC, bool PTRS>
-__global__ __launch_bounds__(kColsSingle * kWave, fp_min_blocks(R)) void cone_fp_kernel(
+__global__ __launch_bounds__(kColsSingle * kWave, fp_waves(R)) void cone_fp_kernel(
     const kk::FpAngle* __restrict__ tab, FpArgs A) {
   fp_tile<R, ALL_COLC, fp_pipe(R), kColsSingle, false, PTRS>(
       tab, A, kk_xcd_remap(blockIdx.x, A.total_blocks, A.xcd_group));
@@ -498,16 +568,6 @@ constexpr int32_t kLineGroupCols = 32;    // (16 x 16: 58.7 ms)
 constexpr int kLineChunks = 4;                  // windows up to 4 x 64
 constexpr int kLineWords = 64 * kLineChunks;    // LDS words per wavefront
 constexpr int64_t kLineEps = int64_t(1) << 18;  // 2^-14 voxel, fixed point
-
-// x as 64-bit fixed point with 32 fraction bits (|x| < 2^31).
-__device__ __forceinline__ int64_t to_fixed(double x) {
-  const double fl = floor(x);
-  const uint32_t lo = static_cast<uint32_t>((x - fl) * 4294967296.0);
-  return static_cast<int64_t>(
-      (static_cast<uint64_t>(static_cast<uint32_t>(static_cast<int32_t>(fl)))
-       << 32) |
-      lo);
-}
 
 __device__ __forceinline__ int64_t bcast64(int64_t v, int32_t lane) {
   const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_readlane(
@@ -626,13 +686,16 @@ __global__ __launch_bounds__(kLineWaves * kWave, 8) void cone_fp_line_kernel(
 
   double a1 = 0.0, b1 = 0.0, a2[R], b2[R];
   int32_t ilo = 0x7fffffff, ihi = -1;
+  bool graze = false;
 #pragma unroll
   for (int k = 0; k < R; ++k) {
     // rows past the detector repeat the last one (not written out)
     const int32_t row = min(row0 + kWave * k + lane, A.rows - 1);
     // (no ray is parallel to the slices: line_spacing)
     kk_fp_ray(P, row, col, a1, b1, a2[k], b2[k]);
-    float lo = 0.f, hi = last;
+    float lo, hi;
+    graze = graze || grazes(a1, b1, a2[k], b2[k], nb1, nc1, last, lo, hi);
+    lo = 0.f, hi = last;
     clip_range(static_cast<float>(a1), static_cast<float>(b1), nb1, last, lo,
                hi);
     clip_range(static_cast<float>(a2[k]), static_cast<float>(b2[k]), nc1, last,
@@ -720,6 +783,26 @@ __global__ __launch_bounds__(kLineWaves * kWave, 8) void cone_fp_line_kernel(
 #undef KK_LINE
     }
   }
+  if (graze) {
+    const uint32_t sbb = static_cast<uint32_t>(P.nc + kk::kHalo) * 4u;
+    const uint64_t sab = static_cast<uint64_t>(P.nb + kk::kHalo) * sbb;
+    const char* frame = A.tex + (P.tex_off >> 1);
+#pragma unroll 1
+    for (int32_t k = 0; k < R; ++k) {
+      float x;
+      if (graze_sum(P, min(row0 + kWave * k + lane, A.rows - 1), col, x,
+                    [&](int32_t i, uint32_t ib, uint32_t ic) {
+                      const float* v = reinterpret_cast<const float*>(
+                          frame + i * sab + static_cast<uint64_t>(ib) * sbb) +
+                          ic;
+                      const float* u = v + sbb / 4;
+                      return kk_float4u{v[0], u[0], v[1], u[1]};
+                    })) {
+#pragma unroll
+        for (int t = 0; t < R; ++t) acc[t] = t == k ? x : acc[t];
+      }
+    }
+  }
 #pragma unroll
   for (int k = 0; k < R; ++k) {
     const int32_t row = row0 + kWave * k + lane;
@@ -744,18 +827,30 @@ __global__ __launch_bounds__(kLineWaves * kWave, 8) void cone_fp_line_kernel(
 
 namespace {
 
-// Rows per thread: 2 unless the detector has at most 64 rows (measured on
-// MI355X: 2 beats 4 by 9-30% at 256^3..512^3, the float64 coordinates of
-// four rays costing occupancy).
-int auto_rows_per_thread(int32_t rows, int32_t rpt) {
-  if (rpt == 1 || rpt == 2 || rpt == 4) return rpt;
-  return rows > 64 ? 2 : 1;
+// Rows per thread, and rows of a wavefront (2^shift; the other lanes are
+// neighbouring columns), where the caller leaves them open.  Single problems:
+// one row, wavefronts of 32 x 2.  Measured, 1 row x 64, 1 x 32, 2 x 64, 2 x 32
+// and 4 x 16 (139, 213 and 319 rows: 150 x 141 x 93, 200^3 and 300^3 tilted):
+// 0.49, 0.45, 0.52, 0.50 and 0.45 ms; 1.05, 1.00, 1.25, 1.28 and 1.05 ms; 3.40,
+// 3.15, 4.97, 4.58 and 3.76 ms: two or four rows of a thread lie too far apart
+// to share lines of the L1, and bands of 64 rows are cut up less well.
+// Batches: two rows, wavefronts of 16 x 4 (bands of 32 rows): 16 problems of
+// 96 rows and 6 of 240, whole SIRT calls, 7.68 and 26.6 ms against 8.02 and
+// 27.3 with 1 x 32 and 8.43 and 31.1 with 2 x 64.
+struct FpLanes {
+  int32_t rpt, row_shift;
+};
+FpLanes fp_lanes(int32_t rows, int32_t rpt, bool batch) {
+  if (rpt != 1 && rpt != 2 && rpt != 4) rpt = batch && rows > 16 ? 2 : 1;
+  int32_t s = batch || rpt == 4 ? 4 : 5;
+  while (s > 0 && (1 << (s - 1)) >= rows) --s;  // few rows: more columns
+  return {rpt, s};
 }
 
 // Validate one forward-projection problem and fill its kernel arguments
-// for `rpt` rows per thread and workgroup groups of at most `cap_angles` x
+// for `lanes` and workgroup groups of at most `cap_angles` x
 // `cap_cols` column tiles.
-int make_fp_args(const kk::FpSpec& S, int32_t rpt, int32_t cols_per_block,
+int make_fp_args(const kk::FpSpec& S, FpLanes lanes, int32_t cols_per_block,
                  int32_t cap_angles, int32_t cap_cols, FpArgs& A) {
   using kk::fail;
   if (S.plan == nullptr || !S.plan->fp_set)
@@ -796,8 +891,11 @@ int make_fp_args(const kk::FpSpec& S, int32_t rpt, int32_t cols_per_block,
   A.rows = S.rows;
   A.cols = S.cols;
   A.n_angles = S.plan->fp_n;
-  A.row_tiles = (S.rows + kWave * rpt - 1) / (kWave * rpt);
-  A.col_tiles = (S.cols + cols_per_block - 1) / cols_per_block;
+  A.row_shift = lanes.row_shift;
+  const int32_t band = lanes.rpt << lanes.row_shift;
+  const int32_t wide = cols_per_block << (6 - lanes.row_shift);
+  A.row_tiles = (S.rows + band - 1) / band;
+  A.col_tiles = (S.cols + wide - 1) / wide;
   A.mode = S.mode;
   A.grp_a = group_size(A.n_angles, cap_angles);
   A.grp_c = group_size(A.col_tiles, cap_cols);
@@ -819,7 +917,7 @@ struct FpItem {
 };
 
 template <int R, bool ALL_COLC>
-__global__ __launch_bounds__(kColsBatch * kWave, fp_batch_min_blocks(R)) void cone_fp_batch_kernel(
+__global__ __launch_bounds__(kColsBatch * kWave, fp_waves(R)) void cone_fp_batch_kernel(
     const FpItem* __restrict__ items, const int64_t* __restrict__ first,
     int32_t n, int64_t total) {
   for (int64_t g = blockIdx.x; g < total; g += gridDim.x) {
@@ -833,7 +931,7 @@ __global__ __launch_bounds__(kColsBatch * kWave, fp_batch_min_blocks(R)) void co
     }
     const FpItem& it = items[lo];
     const int64_t local = g - first[lo];
-    fp_tile<R, ALL_COLC, fp_batch_pipe(R), kColsBatch, true>(it.tab, it.args,
+    fp_tile<R, ALL_COLC, fp_pipe(R), kColsBatch, true>(it.tab, it.args,
                kk_xcd_remap(local, it.args.total_blocks, it.args.xcd_group));
   }
 }
@@ -897,12 +995,12 @@ int fp_batch_build(const std::vector<FpSpec>& specs, int32_t rows_per_thread,
   if (specs.empty()) return fail(KK_ERR_INVALID, "empty forward batch");
   int32_t max_rows = 0;
   for (const FpSpec& S : specs) max_rows = S.rows > max_rows ? S.rows : max_rows;
-  const int32_t rpt = auto_rows_per_thread(max_rows, rows_per_thread);
+  const FpLanes lanes = fp_lanes(max_rows, rows_per_thread, true);
   std::vector<FpItem> items(specs.size());
   std::vector<int64_t> first(specs.size());
   int64_t total = 0;
   for (size_t p = 0; p < specs.size(); ++p) {
-    const int rc = make_fp_args(specs[p], rpt, kColsBatch, kGroupAngles,
+    const int rc = make_fp_args(specs[p], lanes, kColsBatch, kGroupAngles,
                                 kGroupColsBatch, items[p].args);
     if (rc != KK_OK) return rc;
     items[p].tab = specs[p].plan->fp;
@@ -913,7 +1011,7 @@ int fp_batch_build(const std::vector<FpSpec>& specs, int32_t rows_per_thread,
   if (b == nullptr) return fail(KK_ERR_INVALID, "out of host memory");
   b->n = static_cast<int32_t>(specs.size());
   b->total = total;
-  b->rpt = rpt;
+  b->rpt = lanes.rpt;
   b->all_colc = true;
   for (const FpSpec& S : specs) b->all_colc = b->all_colc && S.plan->fp_all_colc;
   hipError_t e = hipMalloc(&b->items, sizeof(FpItem) * items.size());
@@ -1015,9 +1113,11 @@ namespace {
 
 int launch_fp_spec(const kk::FpSpec& S, int32_t rows_per_thread,
                    hipStream_t stream) {
-  const int32_t rpt = auto_rows_per_thread(S.rows, rows_per_thread);
+  const FpLanes lanes = fp_lanes(S.rows, rows_per_thread, false);
+  const int32_t rpt = lanes.rpt;
   FpArgs A;
-  const int rc = make_fp_args(S, rpt, kColsSingle, kGroupAngles, kGroupCols, A);
+  const int rc = make_fp_args(S, lanes, kColsSingle, kGroupAngles,
+                              kGroupCols, A);
   if (rc != KK_OK) return rc;
   const dim3 grid(static_cast<unsigned>(A.total_blocks));
   const bool c = S.plan->fp_all_colc, p = S.ptrs != nullptr;
@@ -1097,7 +1197,7 @@ int launch_fp_planes(const kk::FpSpec& S, hipStream_t stream) {
                     "kk_cone_fp_planes: not a geometry for planes (see "
                     "kk_fp_reads_planes)");
   FpArgs A;
-  const int rc = make_fp_args(S, r, kLineWaves, kLineGroupAngles,
+  const int rc = make_fp_args(S, {r, 6}, kLineWaves, kLineGroupAngles,
                               kLineGroupCols, A);
   if (rc != KK_OK) return rc;
   const dim3 grid(static_cast<unsigned>(A.total_blocks));
