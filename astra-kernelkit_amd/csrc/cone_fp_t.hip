@@ -27,9 +27,10 @@
 //      row step has no a/b part): below.
 //    * cone_fp_t_kernel, other geometries: each lane projects the support
 //      rectangle of its voxels (at its slice) onto the detector and walks
-//      the pixels of the bounding box; the b taps, whose index differs per
-//      lane, are summed in the lane's own LDS words (one read-modify-write
-//      pair per sample instead of a select over all registers).
+//      the pixels of the bounding box, a column's rows unrolled; the b taps,
+//      whose index differs per lane, are summed in the lane's own LDS words
+//      (one read-modify-write of three taps per column instead of a select
+//      over all registers).
 //    A plan with both kinds of angles launches both; each skips the other's.
 // Candidate intervals are widened by 1e-6 voxel in coordinate space, far
 // above the float64 rounding of the sample coordinates; samples outside
@@ -43,8 +44,6 @@ namespace {
 
 constexpr int kJB = 8;       // voxels along b per lane
 constexpr int kJC = 2;       // consecutive voxels along c per lane
-constexpr int kWaves = 4;    // wavefronts per workgroup (b-runs)
-constexpr int kThreads = 64 * kWaves;
 constexpr double kEps = 1e-6;
 
 struct FptArgs {
@@ -191,12 +190,84 @@ __device__ __forceinline__ void close_run(float (*g)[kJC][64], int32_t lane,
   for (int cc = 0; cc < kJC; ++cc) S[cc] = T[cc] = 0.f;
 }
 
+// Consecutive rows of a column, at any element alignment.
+typedef float f32x2_u __attribute__((ext_vector_type(2), aligned(4)));
+typedef float f32x3_u __attribute__((ext_vector_type(3), aligned(4)));
+typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
+
+// max(0, 1 - |x|), one instruction (|x| and the clamp to [0, 1] are free)
+__device__ __forceinline__ float tent(float x) {
+  float w;
+  asm("v_sub_f32_e64 %0, 1.0, |%1| clamp" : "=v"(w) : "v"(x));
+  return w;
+}
+
+// min(max(x, 0), 1), 0 for NaN, one instruction
+__device__ __forceinline__ float unit(float x) {
+  float w;
+  asm("v_max_f32_e64 %0, %1, %1 clamp" : "=v"(w) : "v"(x));
+  return w;
+}
+__device__ __forceinline__ float unit_neg(float x) {
+  float w;
+  asm("v_max_f32_e64 %0, -%1, -%1 clamp" : "=v"(w) : "v"(x));
+  return w;
+}
+
+// W consecutive rows, four per load
+template <int W>
+__device__ __forceinline__ void load_rows(const char* p, float* y) {
+#pragma unroll
+  for (int t = 0; t < W; t += 4) {
+    if (t + 4 <= W) {
+      const f32x4_u v = *reinterpret_cast<const f32x4_u*>(p + 4 * t);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[t + e] = v[e];
+    } else if (t + 3 == W) {
+      const f32x3_u v = *reinterpret_cast<const f32x3_u*>(p + 4 * t);
+      y[t] = v[0];
+      y[t + 1] = v[1];
+      y[t + 2] = v[2];
+    } else if (t + 2 == W) {
+      const f32x2_u v = *reinterpret_cast<const f32x2_u*>(p + 4 * t);
+      y[t] = v[0];
+      y[t + 1] = v[1];
+    } else {
+      y[t] = *reinterpret_cast<const float*>(p + 4 * t);
+    }
+  }
+}
+
 // Value of lane `l` of a wavefront (l wave-uniform), in scalar registers.
 __device__ __forceinline__ int32_t bcast(int32_t v, int32_t l) {
   return __builtin_amdgcn_readlane(v, l);
 }
 
-__global__ __launch_bounds__(kThreads, 6) void cone_fp_t_kernel(
+// Other geometries.
+//
+// Bound by vector instructions: about 20 per row of a column and lane, 55 per
+// column (coordinates, three b taps read, added to and written back in LDS),
+// and the lanes whose box has fewer rows or columns than the wavefront's
+// largest idle for the difference.  So a column's rows are unrolled (four per
+// load, no loop or per-row test), the reciprocal of the perspective is taken
+// once per column, and the b taps go to LDS once per column; row by row, with
+// a reciprocal each and a run of equal b taps flushed wherever one lane's tap
+// changed (40 % of the rows), a row took about 37 slots.
+// A workgroup is one b-run of one slice whose wavefronts share out the angles:
+// enough wavefronts for small volumes, and shorter float32 sums.
+// Measured (one launch per axis, wobbling angles, before -> now): 256^3 / 360
+// angles of 384^2 19.4 -> 12.7 ms, 128^3 / 128 of 192^2 1.59 -> 0.67 ms,
+// 64^3 / 64 of 96^2 0.75 -> 0.13 ms; of that the unrolled columns 13.7 -> 10.0
+// and the shares 10.0 -> 9.1 ms at 256^3 / 256 angles.
+//
+// Workgroups from which the angles go to 4 shares, and to 8 (fewer: 16).
+// Measured in ms for 4 / 8 / 16 shares: 128 workgroups 0.095 / 0.067 / 0.053,
+// 512 0.178 / 0.133 / 0.129, 1152 0.40 / 0.34 / 0.37, 2048 0.77 / 0.67 / 0.80,
+// 3400 1.52 / 1.50 / 1.81, 8280 3.17 / 3.21 / 4.36, 16384 9.1 / 9.1 / 12.0.
+constexpr int64_t kGenShares4 = 4096, kGenShares8 = 640;
+
+template <int SHARES>
+__global__ __launch_bounds__(64 * SHARES, 6) void cone_fp_t_kernel(
     const kk::FpAngle* __restrict__ tab, FptArgs A) {
   // slice fastest, then b tile, then c tile; runs of kSliceRun
   // consecutive ids (neighbouring slices of one tile, which read nearly
@@ -209,9 +280,10 @@ __global__ __launch_bounds__(kThreads, 6) void cone_fp_t_kernel(
   const int32_t tc = static_cast<int32_t>(bid / A.tiles_b);
   const int32_t lane = threadIdx.x & 63;
   const int32_t k = (tc * 64 + lane) * kJC;  // first of the lane's c voxels
-  const int32_t jw = (tb * kWaves + static_cast<int32_t>(threadIdx.x >> 6)) *
-                     kJB;
-  if (jw >= A.nb) return;  // no barriers below: idle wavefronts may leave
+  const int32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int32_t jw = tb * kJB;
+  const int32_t per = (A.n_angles + SHARES - 1) / SHARES;
+  const int32_t q_end = min(A.n_angles, (wave + 1) * per);
 
   const double fi = static_cast<double>(i);
   const double kd = static_cast<double>(k);
@@ -222,14 +294,14 @@ __global__ __launch_bounds__(kThreads, 6) void cone_fp_t_kernel(
   // ordering are needed; taps just outside the b-run are not written out.
   // The run flushes use a spare row on either side of it (g[-1], g[kJB]).
   constexpr int kSpare = 1;
-  __shared__ float gacc[kWaves][kJB + 2 * kSpare][kJC][64];
-  float(*g)[kJC][64] = gacc[threadIdx.x >> 6] + kSpare;
+  __shared__ float gacc[SHARES][kJB + 2 * kSpare][kJC][64];
+  float(*g)[kJC][64] = gacc[wave] + kSpare;
 #pragma unroll
   for (int t = -kSpare; t < kJB + kSpare; ++t)
 #pragma unroll
     for (int cc = 0; cc < kJC; ++cc) g[t][cc][lane] = 0.f;
 
-  for (int32_t q = 0; q < A.n_angles; ++q) {
+  for (int32_t q = wave * per; q < q_end; ++q) {
     const int32_t ang = A.angles[q];
     const kk::FpAngle& P = tab[ang];
     const float* img = A.yw + ang * angle_elems + kRowPad;
@@ -318,18 +390,122 @@ __global__ __launch_bounds__(kThreads, 6) void cone_fp_t_kernel(
     // arel (vb - tb va), and the denominator with slope va (c alike).
     const float kvb = arf * fmaf(-tbf, vaf, vbf);
     const float kvc = arf * fmaf(-tcf, vaf, vcf);
-    const int32_t ncol = (anchor_ok && c_lo <= c_hi) ? c_hi - c_lo + 1 : 0;
+    const int32_t ncol =
+        anchor_ok && c_lo <= c_hi && r_lo <= r_hi ? c_hi - c_lo + 1 : 0;
     const int32_t wncol = wave_max_all(ncol);
-    // b-tap sums over a run of samples with the same tap index, added to
-    // the lane's LDS words when the index changes: S = sum of y w_c,
-    // T = sum of y w_c fb, so the taps t and t + 1 receive S - T and T.
-    // A run stays open from column to column while the index holds (the
-    // sums of one index add up whatever the column), so along the walk
-    // a run closes about once per b voxel crossed.  The index is kept as
-    // a float (the floor of x_b); a run reaches the LDS words only if
-    // its index lies in [-1, kJB) and is dropped otherwise.  Rows
-    // outside the lane's tents add zeros; a non-finite coordinate (a ray
-    // parallel to the slices) starts a run of its own that is dropped.
+    const int32_t wnrow = wave_max_all(ncol > 0 ? r_hi - r_lo + 1 : 0);
+    // Short windows, all rows of a column unrolled: with g(u) = u / (1 +
+    // eps u) and eps = va / den at the column's first row, both
+    // coordinates are A + B g.  eps u is tiny for any usual geometry, so g
+    // takes three terms of its series (what is left out, B u (eps u)^3, is
+    // below 1e-7 voxel by the bound here), and the window's samples span
+    // less than one voxel along b: three tap rows from the floor of the
+    // smaller end, added to the lane's words once per column.
+    {
+      const float w = static_cast<float>(wnrow);
+      const float d1 = fmaf(static_cast<float>(c_lo - wc_lo), uaf, da0);
+      const float d2 = fmaf(static_cast<float>(c_hi - wc_lo), uaf, da0);
+      const float dm = fminf(fabsf(d1), fabsf(d2));
+      // (the slopes B are kvb / den and kvc / den up to the offsets inside
+      // the box, which eps makes small)
+      const bool fit = wnrow <= kRowPad && d1 * d2 > 0.f &&
+                       fabsf(vaf) * w <= 2e-3f * dm &&
+                       fabsf(kvb) * w <= 0.9f * dm &&
+                       fabsf(kvc) * w <= 16.f * dm;
+      if (__ballot(ncol > 0 && !fit) == 0) {
+        auto walk = [&](auto ww) {
+          constexpr int W = decltype(ww)::value;
+          uint32_t o = 4u * (static_cast<uint32_t>(c_lo) *
+                                 static_cast<uint32_t>(cstride) +
+                             static_cast<uint32_t>(r_lo));
+          float dcf = static_cast<float>(c_lo - wc_lo);
+          for (int32_t j = 0; j < wncol; ++j) {
+            if (j < ncol) {
+              asm volatile("" : "+v"(o));
+              float y[W];
+              load_rows<W>(reinterpret_cast<const char*>(img) + o, y);
+              const float dAc = dcf * uaf;
+              const float rc = __builtin_amdgcn_rcpf(da0 + dAc);
+              const float ab = arf * fmaf(-tbf, dAc, dcf * ubf) * rc;
+              const float ac = arf * fmaf(-tcf, dAc, dcf * ucf) * rc;
+              const float Bb = fmaf(-ab, vaf, kvb) * rc;
+              const float Bc = fmaf(-ac, vaf, kvc) * rc;
+              const float eps = vaf * rc;
+              const float xb0 = ab + ob, xc0 = ac + oc;
+              const float t0 = __builtin_amdgcn_fmed3f(
+                  floorf(fminf(xb0, fmaf(Bb, static_cast<float>(W - 1), xb0))),
+                  -1.f, static_cast<float>(kJB - 2));
+              // relative to the middle tap row; what lies outside the
+              // three rows adds to the spare rows, or nothing
+              const float hb0 = xb0 - (t0 + 1.f);
+              float P[3][kJC];
+#pragma unroll
+              for (int r = 0; r < 3; ++r)
+#pragma unroll
+                for (int cc = 0; cc < kJC; ++cc) P[r][cc] = 0.f;
+#pragma unroll
+              for (int t = 0; t < W; ++t) {
+                const float u = static_cast<float>(t);
+                const float gu =
+                    t == 0 ? 0.f
+                           : fmaf(fmaf(eps, u * u * u, -u * u), eps, u);
+                const float xc = t == 0 ? xc0 : fmaf(Bc, gu, xc0);
+                const float h = t == 0 ? hb0 : fmaf(Bb, gu, hb0);
+                const float u0 = y[t] * tent(xc);
+                const float u1 = y[t] * tent(xc - 1.f);
+                const float g0 = unit_neg(h), g1 = tent(h), g2 = unit(h);
+                P[0][0] = fmaf(u0, g0, P[0][0]);
+                P[0][1] = fmaf(u1, g0, P[0][1]);
+                P[1][0] = fmaf(u0, g1, P[1][0]);
+                P[1][1] = fmaf(u1, g1, P[1][1]);
+                P[2][0] = fmaf(u0, g2, P[2][0]);
+                P[2][1] = fmaf(u1, g2, P[2][1]);
+              }
+              float* p = &g[static_cast<int32_t>(t0)][0][lane];
+              // rows are kJC * 64 words apart, c voxels 64 words; all
+              // reads before the writes
+              float v[3 * kJC];
+#pragma unroll
+              for (int r = 0; r < 3 * kJC; ++r) v[r] = p[64 * r];
+#pragma unroll
+              for (int r = 0; r < 3 * kJC; ++r)
+                p[64 * r] = v[r] + P[r / kJC][r % kJC];
+            }
+            o += 4u * static_cast<uint32_t>(cstride);
+            dcf += 1.f;
+          }
+        };
+        if (wnrow <= 2)
+          walk(std::integral_constant<int, 2>{});
+        else if (wnrow <= 3)
+          walk(std::integral_constant<int, 3>{});
+        else if (wnrow <= 4)
+          walk(std::integral_constant<int, 4>{});
+        else if (wnrow <= 5)
+          walk(std::integral_constant<int, 5>{});
+        else if (wnrow <= 6)
+          walk(std::integral_constant<int, 6>{});
+        else if (wnrow <= 7)
+          walk(std::integral_constant<int, 7>{});
+        else if (wnrow <= 8)
+          walk(std::integral_constant<int, 8>{});
+        else if (wnrow <= 12)
+          walk(std::integral_constant<int, 12>{});
+        else
+          walk(std::integral_constant<int, kRowPad>{});
+        continue;
+      }
+    }
+    // Other windows, row by row: b-tap sums over a run of samples with the
+    // same tap index, added to the lane's LDS words when the index changes:
+    // S = sum of y w_c, T = sum of y w_c fb, so the taps t and t + 1
+    // receive S - T and T.  A run stays open from column to column while
+    // the index holds (the sums of one index add up whatever the column),
+    // so along the walk a run closes about once per b voxel crossed.  The
+    // index is kept as a float (the floor of x_b); a run reaches the LDS
+    // words only if its index lies in [-1, kJB) and is dropped otherwise.
+    // Rows outside the lane's tents add zeros; a non-finite coordinate (a
+    // ray parallel to the slices) starts a run of its own that is dropped.
     float tcur = -2.f;  // no run yet
     float S[kJC], T[kJC];
 #pragma unroll
@@ -379,15 +555,22 @@ __global__ __launch_bounds__(kThreads, 6) void cone_fp_t_kernel(
     close_run(g, lane, tcur, S, T);
   }
 
+  // the shares' sums, each wavefront some of the b voxels
+  __syncthreads();
+  constexpr int kPart = (kJB + SHARES - 1) / SHARES;
+  if (wave * kPart >= kJB) return;
 #pragma unroll
   for (int cc = 0; cc < kJC; ++cc) {
     const int32_t kc = k + cc;
     if (kc >= A.nc) break;
 #pragma unroll
-    for (int t = 0; t < kJB; ++t) {
+    for (int e = 0; e < kPart; ++e) {
+      const int32_t t = wave * kPart + e;
       const int32_t j = jw + t;
       if (j >= A.nb) break;
-      const float v = g[t][cc][lane];
+      float v = 0.f;
+#pragma unroll
+      for (int s = 0; s < SHARES; ++s) v += gacc[s][t + kSpare][cc][lane];
       const int64_t o = i * A.sa + j * A.sb + kc * A.sc;
       if (A.mode == 1)
         A.vol[o] += v;
@@ -436,18 +619,6 @@ constexpr int kColB = 8;       // voxels along b per lane
 constexpr int64_t kColSplit2 = 12288;
 // Marks a column whose record has whole voxels apart (whole_s).
 constexpr uint64_t kWhole = uint64_t(1) << 63;
-
-// Consecutive rows of a column, at any element alignment.
-typedef float f32x2_u __attribute__((ext_vector_type(2), aligned(4)));
-typedef float f32x3_u __attribute__((ext_vector_type(3), aligned(4)));
-typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
-
-// max(0, 1 - |x|), one instruction (|x| and the clamp to [0, 1] are free)
-__device__ __forceinline__ float tent(float x) {
-  float w;
-  asm("v_sub_f32_e64 %0, 1.0, |%1| clamp" : "=v"(w) : "v"(x));
-  return w;
-}
 
 template <int SPLIT>
 __global__ __launch_bounds__(64 * kColSlices * SPLIT, 8) void
@@ -646,25 +817,7 @@ cone_fp_t_col_kernel(
             return;
           } else {
             float y[W];
-#pragma unroll
-            for (int t = 0; t < W; t += 4) {
-              if (t + 4 <= W) {
-                const f32x4_u v = *reinterpret_cast<const f32x4_u*>(p + 4 * t);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) y[t + e] = v[e];
-              } else if (t + 3 == W) {
-                const f32x3_u v = *reinterpret_cast<const f32x3_u*>(p + 4 * t);
-                y[t] = v[0];
-                y[t + 1] = v[1];
-                y[t + 2] = v[2];
-              } else if (t + 2 == W) {
-                const f32x2_u v = *reinterpret_cast<const f32x2_u*>(p + 4 * t);
-                y[t] = v[0];
-                y[t + 1] = v[1];
-              } else {
-                y[t] = *reinterpret_cast<const float*>(p + 4 * t);
-              }
-            }
+            load_rows<W>(p, y);
 #pragma unroll
             for (int t = 0; t < W; ++t) {
               const float xt =
@@ -772,8 +925,8 @@ int64_t col_grid(FptArgs& A) {
   return int64_t((A.na + kColSlices - 1) / kColSlices) * A.tiles_b * A.tiles_c;
 }
 int64_t general_grid(FptArgs& A) {
-  A.tiles_b = (A.nb + kJB * kWaves - 1) / (kJB * kWaves);
   A.tiles_c = (A.nc + 64 * kJC - 1) / (64 * kJC);
+  A.tiles_b = (A.nb + kJB - 1) / kJB;
   return int64_t(A.na) * A.tiles_b * A.tiles_c;
 }
 
@@ -860,8 +1013,14 @@ int kk::fp_transpose_launch(const kk_plan_s* plan, const float* proj,
         else if (colc)
           hipLaunchKernelGGL(cone_fp_t_col_kernel<4>, grid,
                              dim3(64 * kColSlices * 4), 0, st, plan->fp, A);
+        else if (blocks >= kGenShares4)
+          hipLaunchKernelGGL(cone_fp_t_kernel<4>, grid, dim3(64 * 4), 0, st,
+                             plan->fp, A);
+        else if (blocks >= kGenShares8)
+          hipLaunchKernelGGL(cone_fp_t_kernel<8>, grid, dim3(64 * 8), 0, st,
+                             plan->fp, A);
         else
-          hipLaunchKernelGGL(cone_fp_t_kernel, grid, dim3(kThreads), 0, st,
+          hipLaunchKernelGGL(cone_fp_t_kernel<16>, grid, dim3(64 * 16), 0, st,
                              plan->fp, A);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return kk::hip_fail(e, "cone_fp_t_kernel");
