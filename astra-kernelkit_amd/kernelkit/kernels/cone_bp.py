@@ -23,6 +23,14 @@ from kernelkit.kernel import (BaseKernel, KernelMemoryUnpreparedException,
 from kernelkit.kernels.cone_fp import detector_shape
 
 
+def _cross(a, b):
+    """Row-wise cross product of ``N x 3`` arrays: ``np.cross`` to the bit,
+    without its axis handling (20 us a call, six calls per reconstruction)."""
+    a = np.concatenate((a, a[:, :2]), axis=1)
+    b = np.concatenate((b, b[:, :2]), axis=1)
+    return a[:, 1:4] * b[:, 2:5] - a[:, 2:5] * b[:, 1:4]
+
+
 def _world_strides(tensor, volume_axes) -> list:
     """Element strides of world axes (x, y, z) of an array whose axis k is
     world axis ``volume_axes[k]``."""
@@ -267,7 +275,7 @@ class VoxelDrivenConeBP(BaseKernel):
         V = seq.v * seq.detector.pixel_height[:, None]
         s = seq.source_position
         d = seq.detector_extent_min
-        uxv = np.cross(U, V)
+        uxv = _cross(U, V)
         if with_adjoint_scaling:
             cr = uxv * np.array([vs[1] * vs[2], vs[0] * vs[2], vs[0] * vs[1]])
             k = np.sqrt(np.linalg.norm(cr, axis=1))
@@ -276,13 +284,13 @@ class VoxelDrivenConeBP(BaseKernel):
             k = np.ones(len(s))
 
         def det3(a, b, c):
-            return np.einsum("ij,ij->i", a, np.cross(b, c))
+            return np.einsum("ij,ij->i", a, _cross(b, c))
 
         smd = s - d
         out = np.empty((len(s), 12))
-        out[:, 0:3] = k[:, None] * np.cross(V, smd)
+        out[:, 0:3] = k[:, None] * _cross(V, smd)
         out[:, 3] = k * det3(s, V, d)
-        out[:, 4:7] = k[:, None] * np.cross(smd, U)
+        out[:, 4:7] = k[:, None] * _cross(smd, U)
         out[:, 7] = -k * det3(s, U, d)
         out[:, 8:11] = -k[:, None] * uxv
         out[:, 11] = k * det3(U, V, s)

@@ -61,3 +61,18 @@ def test_extent_refuses_other_geometries():
     for kw in ({}, dict(wobble_deg=1.0)):
         pgs = workloads.circular_geometry(8, 10.0, 50.0, 40, 40, 1.0, **kw)
         assert _extent(pgs, vg)[1][0] < 0
+
+
+@pytest.mark.parametrize("n", [0, 1, 7])
+def test_cross_products_are_numpys_to_the_bit(n):
+    from kernelkit.kernels.cone_bp import _cross
+    r = np.random.default_rng(n)
+    a, b = r.normal(size=(n, 3)), r.normal(size=(3, n)).T
+    assert np.array_equal(_cross(a, b), np.cross(a, b))
+
+
+def test_isotropic_voxels_of_equal_close_and_unequal_sizes():
+    for step, expected in ((0.0, True), (2e-6, True), (1e-3, False)):
+        vg = kk.VolumeGeometry((4, 4, 4), (1.0, 1.0, 1.0 + step),
+                               (-2.0, -2.0, -2.0), (2.0, 2.0, 2.0))
+        assert vg.has_isotropic_voxels() is expected
