@@ -404,15 +404,20 @@ __device__ __forceinline__ void fp_tile_at(
     float lo = 0.f, hi = last;
     clip_range(static_cast<float>(a1), static_cast<float>(b1), nb1, last, lo,
                hi);
+    const float lob = lo, hib = hi;
     clip_range(static_cast<float>(a2), static_cast<float>(b2), nc1, last, lo,
                hi);
     float glo, ghi;
     graze = graze || (ok && grazes(a1, b1, a2, b2, nb1, nc1, last, glo, ghi));
-    const int32_t mid = static_cast<int32_t>(
-        fminf(fmaxf(0.5f * (lo + hi), 0.f), last));
+    auto middle = [&](float l, float h) {
+      return static_cast<int32_t>(fminf(fmaxf(0.5f * (l + h), 0.f), last));
+    };
+    const int32_t mid = middle(lo, hi);
     if (k < NB) {
-      mb[k] = mid;
-      fixed_ray(a1, b1, P.na, mid, nb1, w.b[k], w.gb[k]);
+      // column-coherent angles: the column's own middle, so that rays have
+      // the same bits whichever rays share their b coordinate
+      mb[k] = P.colc ? middle(lob, hib) : mid;
+      fixed_ray(a1, b1, P.na, mb[k], nb1, w.b[k], w.gb[k]);
     }
     mc[k] = mid;
     fixed_ray(a2, b2, P.na, mid, nc1, w.c[k], w.gc[k]);
