@@ -1,0 +1,47 @@
+"""The exact transpose's unrolled walk where a column's rows are rounded up to
+the next unrolled length (9 -> 12, 13 -> 16) and their slope along b is at its
+limit, against the FP64 oracle: relative L2 <= 1e-5, pointwise <= 1e-4 *
+max|ref| (the parity bar)."""
+import numpy as np
+import pytest
+
+import oracle
+from conftest import assert_parity
+
+pytestmark = pytest.mark.gpu
+
+kk = pytest.importorskip("kernelkit")
+from kernelkit.geom.proj import Detector, ProjectionGeometry  # noqa: E402
+
+
+def _rolled_orbit(angles, rows, cols, height, roll, sod=150.0, width=1.2):
+    """Orbit of magnification 1.5 about an axis ``roll`` degrees off z, the
+    same way at all angles (rows then move one way along b)."""
+    det = Detector(rows=rows, cols=cols, pixel_height=height,
+                   pixel_width=width)
+    c, s = np.cos(np.deg2rad(roll)), np.sin(np.deg2rad(roll))
+    tilt = np.array([[1.0, 0.0, 0.0], [0.0, c, -s], [0.0, s, c]])
+    out = []
+    for k in range(angles):
+        t = 2 * np.pi * k / angles + 0.09
+        R = tilt @ np.array([[np.cos(t), -np.sin(t), 0.0],
+                             [np.sin(t), np.cos(t), 0.0], [0.0, 0.0, 1.0]])
+        out.append(ProjectionGeometry(
+            R @ [-sod, 0.0, 0.0], R @ [0.5 * sod, 0.3, -0.4], det,
+            u=R @ [0.0, 1.0, 0.0], v=R @ [0.0, 0.0, 1.0]))
+    return out
+
+
+# rows per voxel: windows of 9 (up to 12) and of 13 rows (up to 16)
+@pytest.mark.parametrize("sign", [1, -1])
+@pytest.mark.parametrize("roll", [9.5, 10.0, 10.5, 10.9])
+@pytest.mark.parametrize("fine", [1.75, 1.8, 1.85, 1.92, 2.7, 2.75, 2.8])
+def test_padded_windows(fine, roll, sign, device):
+    import torch
+    rows = int(30 * fine) + 2
+    pgs = _rolled_orbit(7, rows, 50, 1.5 / fine, sign * roll)
+    vg = kk.resolve_volume_geometry(shape=(23, 18, 21), voxel_size=1.0)
+    y = np.random.default_rng(1).uniform(size=(len(pgs), rows, 50))
+    got = kk.XrayTransform(pgs, vg).matched_T(
+        torch.from_numpy(y.astype(np.float32)).cuda()).cpu().numpy()
+    assert_parity(got, oracle.cone_fp_transpose(y, pgs, vg))
