@@ -15,7 +15,6 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
-import gc
 import os
 import sys
 import threading
@@ -349,6 +348,36 @@ def stream_ptr(stream=None) -> ctypes.c_void_p:
     raise TypeError(f"not a stream: {type(stream).__name__}")
 
 
+def release(destructor: str, ptr: ctypes.c_void_p) -> None:
+    """Call the library's ``destructor`` on ``ptr``; while this thread
+    captures (:meth:`Graph.capture`), once the capture has ended: a free of
+    device memory, by the cycle collector for one, ends a capture."""
+    try:
+        held = getattr(_local, "held", None)
+        if held is not None:
+            held.append((destructor, ptr))
+        elif _lib is not None:
+            getattr(_lib, destructor)(ptr)
+    except Exception:  # interpreter shutdown
+        pass
+
+
+@contextlib.contextmanager
+def _holding_releases():
+    """Holds this thread's :func:`release` calls back until the (outermost)
+    block is left."""
+    if getattr(_local, "held", None) is not None:
+        yield
+        return
+    _local.held = held = []
+    try:
+        yield
+    finally:
+        _local.held = None
+        for destructor, ptr in held:
+            release(destructor, ptr)
+
+
 class Plan:
     """Owner of a library plan (per-angle device tables)."""
 
@@ -363,11 +392,8 @@ class Plan:
 
     def __del__(self):
         ptr = getattr(self, "_ptr", None)
-        if ptr is not None and ptr.value and _lib is not None:
-            try:
-                _lib.kk_plan_destroy(ptr)
-            except Exception:  # interpreter shutdown
-                pass
+        if ptr is not None and ptr.value:
+            release("kk_plan_destroy", ptr)
             self._ptr = None
 
 
@@ -386,11 +412,8 @@ class Batch:
 
     def __del__(self):
         ptr = getattr(self, "_ptr", None)
-        if ptr is not None and ptr.value and _lib is not None:
-            try:
-                _lib.kk_batch_destroy(ptr)
-            except Exception:  # interpreter shutdown
-                pass
+        if ptr is not None and ptr.value:
+            release("kk_batch_destroy", ptr)
             self._ptr = None
 
 
@@ -410,11 +433,8 @@ class Filter:
 
     def __del__(self):
         ptr = getattr(self, "_ptr", None)
-        if ptr is not None and ptr.value and _lib is not None:
-            try:
-                _lib.kk_filter_destroy(ptr)
-            except Exception:  # interpreter shutdown
-                pass
+        if ptr is not None and ptr.value:
+            release("kk_filter_destroy", ptr)
             self._ptr = None
 
 
@@ -447,11 +467,8 @@ class Stream:
 
     def __del__(self):
         ptr = getattr(self, "_ptr", None)
-        if ptr is not None and ptr.value and _lib is not None:
-            try:
-                _lib.kk_stream_destroy(ptr)
-            except Exception:  # interpreter shutdown
-                pass
+        if ptr is not None and ptr.value:
+            release("kk_stream_destroy", ptr)
             self._ptr = None
 
 
@@ -481,11 +498,8 @@ class Event:
 
     def __del__(self):
         ptr = getattr(self, "_ptr", None)
-        if ptr is not None and ptr.value and _lib is not None:
-            try:
-                _lib.kk_event_destroy(ptr)
-            except Exception:  # interpreter shutdown
-                pass
+        if ptr is not None and ptr.value:
+            release("kk_event_destroy", ptr)
             self._ptr = None
 
 
@@ -504,25 +518,21 @@ class Graph:
     @classmethod
     def capture(cls, fn) -> "Graph":
         s = Stream()
-        # no cycle collection while capturing: it may free device memory of
-        # objects long out of use (plans of dropped operators), which a
-        # capture does not survive
-        collects = gc.isenabled()
-        gc.disable()
-        check(lib().kk_graph_begin_capture(s.ptr))
-        try:
-            with use_stream(s.ptr):
-                fn()
-        except BaseException:
-            dead = _vp()
-            if lib().kk_graph_end_capture(s.ptr, ctypes.byref(dead)) == KK_OK:
-                lib().kk_graph_destroy(dead)
-            raise
-        finally:
-            if collects:
-                gc.enable()
         exec_ptr = _vp()
-        check(lib().kk_graph_end_capture(s.ptr, ctypes.byref(exec_ptr)))
+        # objects dropped meanwhile (plans of operators long out of use, when
+        # a cycle collection meets them) are freed after the capture
+        with _holding_releases():
+            check(lib().kk_graph_begin_capture(s.ptr))
+            try:
+                with use_stream(s.ptr):
+                    fn()
+            except BaseException:
+                dead = _vp()
+                if lib().kk_graph_end_capture(
+                        s.ptr, ctypes.byref(dead)) == KK_OK:
+                    lib().kk_graph_destroy(dead)
+                raise
+            check(lib().kk_graph_end_capture(s.ptr, ctypes.byref(exec_ptr)))
         return cls(exec_ptr)
 
     @property
@@ -534,11 +544,8 @@ class Graph:
 
     def __del__(self):
         ptr = getattr(self, "_ptr", None)
-        if ptr is not None and ptr.value and _lib is not None:
-            try:
-                _lib.kk_graph_destroy(ptr)
-            except Exception:  # interpreter shutdown
-                pass
+        if ptr is not None and ptr.value:
+            release("kk_graph_destroy", ptr)
             self._ptr = None
 
 

@@ -88,11 +88,8 @@ class _Buffer:
 
     def __del__(self):
         ptr = getattr(self, "ptr", 0)
-        if ptr and _native._lib is not None:
-            try:
-                _native._lib.kk_free(ctypes.c_void_p(ptr))
-            except Exception:  # interpreter shutdown
-                pass
+        if ptr:
+            _native.release("kk_free", ctypes.c_void_p(ptr))
             self.ptr = 0
 
 
