@@ -110,6 +110,16 @@ def _alloc(n: int, like=None, device=None):
     return _dev.empty((int(n),), like=like)
 
 
+def _after_allocation(stream) -> None:
+    """Let ``stream`` wait for the current stream, on which memory just
+    allocated may still be in use by the work of its last owner."""
+    cur, other = _native.stream_ptr(), _native.stream_ptr(stream)
+    if (cur.value or 0) != (other.value or 0):
+        done = _native.Event()
+        done.record(cur)
+        _native.check(_native.lib().kk_stream_wait_event(other, done.ptr))
+
+
 class Texture:
     """Snapshot of an array, the analogue of a CUDA array behind a texture
     object (``kernel.py:47-119``): a contiguous float32 device copy in the
@@ -151,7 +161,8 @@ class VolumeTexture:
     ``update(..., planes=True)`` builds planes only.  :attr:`data` and
     :attr:`ptr` are the pairs: they are made from the planes when first
     asked for, and count as the texture's content from then on (a caller may
-    write them), until the next update.
+    write them), until the next update.  A kernel that reads pairs takes
+    :meth:`pairs_ptr`, made from the planes for that launch, on its stream.
     """
 
     def __init__(self, world_shape, mask: int, device=None, like=None):
@@ -178,9 +189,20 @@ class VolumeTexture:
         if self._pairs is None:
             self._pairs = self._buffer(self._n)
         if self._holds_planes:
-            self._planes_to_pairs()
+            self._planes_to_pairs(None)
             self._holds_planes = False
         return self._pairs
+
+    def pairs_ptr(self, stream=None) -> int:
+        """Device address of the pairs for launches on ``stream``, converted
+        there if the content is held as planes (which it stays)."""
+        if not self._holds_planes:
+            return self.ptr
+        if self._pairs is None:
+            self._pairs = self._buffer(self._n)
+            _after_allocation(stream)
+        self._planes_to_pairs(stream)
+        return self._pairs.data_ptr()
 
     @property
     def ptr(self):
@@ -195,7 +217,7 @@ class VolumeTexture:
     def covers(self, mask: int) -> bool:
         return (int(mask) & ~self.mask) == 0
 
-    def _planes_to_pairs(self):
+    def _planes_to_pairs(self, stream):
         # a frame of planes is a strided view of the volume in itself
         off = 0
         src = self._planes.data_ptr()
@@ -211,7 +233,7 @@ class VolumeTexture:
             _native.check(_native.lib().kk_volume_to_fp_texture(
                 _native._vp(src + 4 * first), _native.i32(self.world_shape),
                 _native.i64(st), 1 << a, _native._vp(dst + 8 * off),
-                _native.stream_ptr()))
+                _native.stream_ptr(stream)))
             off += self.world_shape[a] * tb * tc
 
     def update(self, volume, volume_axes=(0, 1, 2), stream=None,
@@ -273,12 +295,7 @@ class ProjectionTexture:
         if self._pairs is None:
             self._pairs = self._buffer(self._n)
         if self._holds_planes:
-            n, rows, cols = self.shape
-            pitch = rows + _native.PLANE_GAP
-            _native.check(_native.lib().kk_projections_to_bp_texture(
-                _native._vp(self._planes.data_ptr()), *self.shape,
-                _native.i64((cols * pitch, 1, pitch)),
-                _native._vp(self._pairs.data_ptr()), _native.stream_ptr()))
+            self._planes_to_pairs(None)
             self._holds_planes = False
         return self._pairs
 
@@ -291,6 +308,25 @@ class ProjectionTexture:
         """Device address of the planes, None unless the texture's content
         is held as such."""
         return self._planes.data_ptr() if self._holds_planes else None
+
+    def _planes_to_pairs(self, stream):
+        n, rows, cols = self.shape
+        pitch = rows + _native.PLANE_GAP
+        _native.check(_native.lib().kk_projections_to_bp_texture(
+            _native._vp(self._planes.data_ptr()), *self.shape,
+            _native.i64((cols * pitch, 1, pitch)),
+            _native._vp(self._pairs.data_ptr()), _native.stream_ptr(stream)))
+
+    def pairs_ptr(self, stream=None) -> int:
+        """Device address of the pairs for launches on ``stream``, as in
+        :class:`VolumeTexture`."""
+        if not self._holds_planes:
+            return self.ptr
+        if self._pairs is None:
+            self._pairs = self._buffer(self._n)
+            _after_allocation(stream)
+        self._planes_to_pairs(stream)
+        return self._pairs.data_ptr()
 
     def hold_planes(self) -> int:
         """Device address of the planes, which become the texture's content
@@ -415,7 +451,9 @@ class BaseKernel(ABC):
 
     Kernels work in place and return nothing; a call launches device work
     asynchronously on the current stream and allocates nothing, so it can be
-    captured in a HIP graph (``docs/user_guide/kernels.rst:16-21``).
+    captured in a HIP graph (``docs/user_guide/kernels.rst:16-21``); only the
+    first call that is handed a texture in another layout than the kernel
+    reads (:meth:`VolumeTexture.pairs_ptr`) allocates that.
     ``compile()`` loads the gfx950 library and creates the kernel's plan.
     """
 

@@ -213,7 +213,8 @@ class VoxelDrivenConeBP(BaseKernel):
                 self.reads_planes_for(rows, cols, volume_geometry):
             launch, tex = _native.lib().kk_cone_bp_planes, planes
         else:
-            launch, tex = _native.lib().kk_cone_bp, textures.ptr
+            launch = _native.lib().kk_cone_bp
+            tex = textures.pairs_ptr(stream)
         _native.check(launch(
             self._plan.ptr, _native._vp(tex), n, rows, cols,
             _native._vp(volume.data_ptr()), _native.i32(volume_geometry.shape),

@@ -382,7 +382,7 @@ class RayDrivenConeFP(BaseKernel):
                 _native.stream_ptr(stream)))
             return
         _native.check(_native.lib().kk_cone_fp_ptrs(
-            self._plan.ptr, _native._vp(tex.ptr),
+            self._plan.ptr, _native._vp(tex.pairs_ptr(stream)),
             _native._vp(table.data_ptr()), self._proj_axs[0],
             _native.i64(strides), rows, cols, 1 if additive else 0,
             _native.stream_ptr(stream)))
@@ -398,7 +398,8 @@ class RayDrivenConeFP(BaseKernel):
                 _native.stream_ptr(stream)))
             return
         _native.check(_native.lib().kk_cone_fp(
-            self._plan.ptr, _native._vp(tex.ptr), _native._vp(proj.data_ptr()),
+            self._plan.ptr, _native._vp(tex.pairs_ptr(stream)),
+            _native._vp(proj.data_ptr()),
             _native.i64(strides), rows, cols, 1 if additive else 0,
             _native.stream_ptr(stream)))
 
