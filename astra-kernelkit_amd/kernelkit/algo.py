@@ -22,7 +22,7 @@ from kernelkit import _native, device
 from kernelkit.geom.proj import Beam, ProjectionGeometry
 from kernelkit.geom.vol import VolumeGeometry
 from kernelkit.kernel import (BaseKernel, ProjectionTexture, as_device_array,
-                              default_device, is_device_array)
+                              default_device, is_device_array, reads_planes)
 from kernelkit.kernels.cone_bp import VoxelDrivenConeBP
 from kernelkit.operator import XrayTransform
 from kernelkit.processing import filter_into, filter_rows_into
@@ -82,7 +82,7 @@ def bp(projections: Any, projection_geometry, volume_geometry: VolumeGeometry,
         if projection_axes != (0, 1, 2):
             raise NotImplementedError()
         tex = ProjectionTexture(*proj.shape, like=proj)
-        if K.reads_planes:
+        if reads_planes(K):
             filtered = device.empty(tuple(proj.shape), like=proj)
             filter_rows_into(proj, filtered, geoms=list(projection_geometry),
                              filter=filter)

@@ -483,3 +483,9 @@ class BaseKernel(ABC):
     @property
     def is_compiled(self) -> bool:
         return getattr(self, "_plan", None) is not None
+
+
+def reads_planes(kernel) -> bool:
+    """Whether ``kernel`` takes textures held as planes (a class of the
+    caller's own that says nothing about it gets pairs)."""
+    return bool(getattr(kernel, "reads_planes", False))

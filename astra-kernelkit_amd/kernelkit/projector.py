@@ -20,8 +20,8 @@ import numpy as np
 
 from kernelkit.geom.proj import ProjectionGeometry, ProjectionGeometrySequence
 from kernelkit.geom.vol import VolumeGeometry
-from kernelkit.kernel import (BaseKernel, VolumeTexture, as_device_array,
-                              is_device_array)
+from kernelkit.kernel import (BaseKernel, ProjectionTexture, VolumeTexture,
+                              as_device_array, is_device_array, reads_planes)
 from kernelkit.kernels.cone_bp import VoxelDrivenConeBP
 from kernelkit.kernels.cone_fp import RayDrivenConeFP
 
@@ -232,13 +232,13 @@ class ForwardProjector(Projector):
             tex = VolumeTexture(world, mask, like=as_device_array(value))
             self._texture = tex
         tex.update(value, self.volume_axes,
-                   planes=self._K.reads_planes and not pairs)
+                   planes=reads_planes(self._K) and not pairs)
 
     def _update_params(self):
         super()._update_params()
         tex = getattr(self, "_texture", None)
         if (tex is not None and tex.planes is not None
-                and not self._K.reads_planes):
+                and not reads_planes(self._K)):
             tex.data  # noqa: B018 -- the set volume as the new kernel reads it
 
     @volume.deleter
@@ -393,14 +393,15 @@ class BackProjector(Projector):
             raise ValueError("Can only use layered texture when the first "
                              "projection axis is 0.")
         value = as_device_array(value)
+        layout = {"pairs": True} if pairs else {}
         self._textures = self._K.projection_texture(
-            value, getattr(self, "_textures", None), pairs)
+            value, getattr(self, "_textures", None), **layout)
 
     def _update_params(self):
         super()._update_params()
         tex = getattr(self, "_textures", None)
-        if (tex is not None and tex.planes is not None
-                and not self._K.reads_planes):
+        if (isinstance(tex, ProjectionTexture) and tex.planes is not None
+                and not reads_planes(self._K)):
             tex.data  # noqa: B018 -- as the new kernel reads them
 
     @projections.deleter
