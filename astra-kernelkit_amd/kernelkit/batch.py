@@ -180,6 +180,8 @@ class BatchSirt:
             batch._check(masks, batch.domain_shapes, "mask")
         else:
             masks = [None] * len(batch)
+        for op, vg in zip(batch.ops, batch.vgs):
+            op.backprojector.kernel.check_voxels(vg)
         self.y, self.x, self.C, self.R, self.p = ys, [], [], [], []
         self.masks = masks
         self.res_tex = []

@@ -185,10 +185,7 @@ class VoxelDrivenConeBP(BaseKernel):
                 f"Volume has a dtype '{volume.dtype}'. However, currently"
                 " there is only support for dtype=float32.")
         volume = _dev.asarray(volume)
-        if not volume_geometry.has_isotropic_voxels():
-            raise NotImplementedError(
-                f"`{self.__class__.__name__}` is not tested with anisotropic "
-                "voxels yet.")
+        self.check_voxels(volume_geometry)
         if not self.is_compiled:
             raise KernelNotCompiledException(
                 "Please compile the kernel with `compile()`.")
@@ -221,6 +218,13 @@ class VoxelDrivenConeBP(BaseKernel):
             _native.i64(_world_strides(volume, self._vol_axs)),
             float(volume_geometry.voxel_volume()), 1 if additive else 0,
             _native.stream_ptr(stream)))
+    def check_voxels(self, volume_geometry: VolumeGeometry) -> None:
+        """Refuse volumes that the kernel is not made for."""
+        if not volume_geometry.has_isotropic_voxels():
+            raise NotImplementedError(
+                f"`{self.__class__.__name__}` is not tested with anisotropic "
+                "voxels yet.")
+
 
     def projection_texture(self, projections,
                            texture: ProjectionTexture | None = None,
