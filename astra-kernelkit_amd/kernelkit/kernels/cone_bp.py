@@ -82,8 +82,7 @@ class VoxelDrivenConeBP(BaseKernel):
         self._proj_axs = tuple(projection_axes)
         self._params_are_set = False
         self._n_params = 0
-        self._planes_key = None
-        self._reads_planes = False
+        self._planes = (None, False)   # for which sizes, and the answer
 
     @property
     def volume_axes(self):
@@ -145,8 +144,7 @@ class VoxelDrivenConeBP(BaseKernel):
             self._plan.ptr, _native.f64_ptr(arr), n))
         self._n_params = n
         self._params_are_set = True
-        self._planes_key = None
-        self._reads_planes = False
+        self._planes = (None, False)
         if projection_geometry is not None and volume_geometry is not None:
             rows, cols = detector_shape(projection_geometry)
             self.reads_planes_for(rows, cols, volume_geometry)
@@ -156,17 +154,18 @@ class VoxelDrivenConeBP(BaseKernel):
         """Whether the parameters set with their geometries are ones that the
         kernel backprojects from planes
         (:class:`~kernelkit.kernel.ProjectionTexture`)."""
-        return self._reads_planes
+        return self._planes[1]
 
     def reads_planes_for(self, rows, cols, volume_geometry) -> bool:
         """:attr:`reads_planes` for a detector and volume given."""
         key = (rows, cols, tuple(volume_geometry.shape))
-        if key != self._planes_key:
-            self._planes_key = key
-            self._reads_planes = bool(_native.lib().kk_bp_reads_planes(
+        planes = self._planes
+        if key != planes[0]:
+            planes = (key, bool(_native.lib().kk_bp_reads_planes(
                 self._plan.ptr, rows, cols,
-                _native.i32(volume_geometry.shape)))
-        return self._reads_planes
+                _native.i32(volume_geometry.shape))))
+            self._planes = planes
+        return planes[1]
 
     def __call__(self, textures, volume, volume_geometry: VolumeGeometry, *,
                  additive: bool = True, stream=None):
@@ -218,13 +217,13 @@ class VoxelDrivenConeBP(BaseKernel):
             _native.i64(_world_strides(volume, self._vol_axs)),
             float(volume_geometry.voxel_volume()), 1 if additive else 0,
             _native.stream_ptr(stream)))
+
     def check_voxels(self, volume_geometry: VolumeGeometry) -> None:
         """Refuse volumes that the kernel is not made for."""
         if not volume_geometry.has_isotropic_voxels():
             raise NotImplementedError(
                 f"`{self.__class__.__name__}` is not tested with anisotropic "
                 "voxels yet.")
-
 
     def projection_texture(self, projections,
                            texture: ProjectionTexture | None = None,

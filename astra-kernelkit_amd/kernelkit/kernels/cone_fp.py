@@ -193,10 +193,10 @@ class RayDrivenConeFP(BaseKernel):
         _native.check(_native.lib().kk_set_params_fp(
             self._plan.ptr, _native.f64_ptr(self._params), n, axes_ptr,
             rows, cols, _native.i32(vg.shape), _native.f64(vg.voxel_size)))
-        self._uploaded_key = key
         self._frame_mask = int(_native.lib().kk_fp_frame_mask(self._plan.ptr))
         self._reads_planes = bool(_native.lib().kk_fp_reads_planes(
             self._plan.ptr, rows, cols))
+        self._uploaded_key = key
 
     @property
     def frame_mask(self) -> int:
