@@ -18,7 +18,7 @@ class _StubLibrary:
             if name.endswith("_elems"):
                 return 64
             if name in ("kk_malloc", "kk_filter_create"):
-                args[0]._obj.value = 0x4000
+                args[0]._obj.value = 0   # nothing to free
             return _native.KK_OK
         return call
 
