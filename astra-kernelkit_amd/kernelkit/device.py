@@ -443,9 +443,13 @@ def to_host(x, out=None) -> np.ndarray:
         x = x.detach()
         torch = _torch_module()
         if (x.is_cuda and x.dtype == torch.float32 and x.is_contiguous()
+                and not x.is_neg()     # (its bytes are not its values)
                 and 4 * x.numel() >= _THREADED_COPY
                 and x.device.index == torch.cuda.current_device()):
-            direct = (isinstance(out, np.ndarray) and out.dtype == np.float32
+            # (an array class of its own, a masked one for instance, may mean
+            # more by an assignment than the bytes)
+            direct = (type(out) in (np.ndarray, np.memmap)
+                      and out.dtype == np.float32
                       and out.shape == tuple(x.shape)
                       and out.flags.c_contiguous and out.flags.writeable)
             host = out if direct else np.empty(tuple(x.shape), np.float32)
