@@ -8,7 +8,6 @@
 // C caller do the same through this library alone.
 #include <algorithm>
 #include <cstring>
-#include <system_error>
 #include <thread>
 
 #include "kk_internal.h"
@@ -24,22 +23,31 @@ constexpr int64_t kHostPiece = int64_t(2) << 20;
 constexpr int kHostWorkers = 6;
 
 // One worker's pieces w, w + workers, ...: the first error, or success.
+// Without pinned memory to be had, the runtime copies into the pageable.
 hipError_t copy_pieces(int device, char* dst, const char* src, int64_t bytes,
                        int w, int workers, hipStream_t stream) {
   hipError_t e = hipSetDevice(device);
   if (e != hipSuccess) return e;
   void* buf = nullptr;
   hipEvent_t done = nullptr;
-  e = hipHostMalloc(&buf, size_t(std::min(kHostPiece, bytes)), 0);
-  if (e == hipSuccess)
-    e = hipEventCreateWithFlags(&done, hipEventDisableTiming);
+  if (hipHostMalloc(&buf, size_t(std::min(kHostPiece, bytes)), 0) !=
+      hipSuccess) {
+    buf = nullptr;
+    (void)hipGetLastError();  // not the next launch's error
+  }
+  e = hipEventCreateWithFlags(&done, hipEventDisableTiming);
   for (int64_t at = w * kHostPiece; e == hipSuccess && at < bytes;
        at += workers * kHostPiece) {
     const size_t n = size_t(std::min(kHostPiece, bytes - at));
-    e = hipMemcpyAsync(buf, src + at, n, hipMemcpyDeviceToHost, stream);
-    if (e == hipSuccess) e = hipEventRecord(done, stream);
-    if (e == hipSuccess) e = hipEventSynchronize(done);
-    if (e == hipSuccess) std::memcpy(dst + at, buf, n);
+    e = hipMemcpyAsync(buf ? buf : dst + at, src + at, n,
+                       hipMemcpyDeviceToHost, stream);
+    if (e != hipSuccess) break;
+    e = hipEventRecord(done, stream);
+    // (the buffer is written until then, whatever failed)
+    const hipError_t s = e == hipSuccess ? hipEventSynchronize(done)
+                                         : hipStreamSynchronize(stream);
+    if (e == hipSuccess) e = s;
+    if (e == hipSuccess && buf) std::memcpy(dst + at, buf, n);
   }
   if (done) hipEventDestroy(done);
   if (buf) hipHostFree(buf);
@@ -155,8 +163,8 @@ extern "C" int kk_copy_to_host(void* dst, const void* src, int64_t bytes,
   for (int w = 1; w < workers; ++w) {
     try {
       threads[w] = std::thread(work, w);
-    } catch (const std::system_error&) {
-      // no thread to be had: this thread does its share below
+    } catch (...) {
+      // no thread or no memory for one: this thread does its share below
     }
   }
   work(0);
