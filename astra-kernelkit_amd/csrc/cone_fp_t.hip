@@ -400,13 +400,11 @@ __global__ __launch_bounds__(64 * SHARES, 6) void cone_fp_t_kernel(
     // takes three terms of its series (what is left out, B u (eps u)^3, is
     // below 1e-7 voxel by the bound here), and the window's samples span
     // less than one voxel along b: three tap rows from the floor of the
-    // smaller end, added to the lane's words once per column.  The rows
-    // that fill the window up to an unrolled length W lie outside the
-    // lanes' boxes: they may pass the three tap rows, but add nothing to a
-    // voxel (and do not count as ends, which the bound is not for).
+    // smaller end, added to the lane's words once per column.
     {
-      const float w = static_cast<float>(wnrow);
-      const float wlast = w - 1.f;  // the last row of the longest box
+      // (with the rows that fill the window up to an unrolled length)
+      const float w = static_cast<float>(
+          wnrow <= 8 ? wnrow : (wnrow <= 12 ? 12 : kRowPad));
       const float d1 = fmaf(static_cast<float>(c_lo - wc_lo), uaf, da0);
       const float d2 = fmaf(static_cast<float>(c_hi - wc_lo), uaf, da0);
       const float dm = fminf(fabsf(d1), fabsf(d2));
@@ -437,7 +435,7 @@ __global__ __launch_bounds__(64 * SHARES, 6) void cone_fp_t_kernel(
               const float eps = vaf * rc;
               const float xb0 = ab + ob, xc0 = ac + oc;
               const float t0 = __builtin_amdgcn_fmed3f(
-                  floorf(fminf(xb0, fmaf(Bb, wlast, xb0))),
+                  floorf(fminf(xb0, fmaf(Bb, static_cast<float>(W - 1), xb0))),
                   -1.f, static_cast<float>(kJB - 2));
               // relative to the middle tap row; what lies outside the
               // three rows adds to the spare rows, or nothing

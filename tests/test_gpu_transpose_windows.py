@@ -1,7 +1,6 @@
-"""The exact transpose's unrolled walk where a column's rows are rounded up to
-the next unrolled length (9 -> 12, 13 -> 16) and their slope along b is at its
-limit, against the FP64 oracle: relative L2 <= 1e-5, pointwise <= 1e-4 *
-max|ref| (the parity bar)."""
+"""The exact transpose's walks at the edges of their windows and shares, against
+the FP64 oracle: relative L2 <= 1e-5, pointwise <= 1e-4 * max|ref| (the parity
+bar)."""
 import numpy as np
 import pytest
 
@@ -11,6 +10,7 @@ from conftest import assert_parity
 pytestmark = pytest.mark.gpu
 
 kk = pytest.importorskip("kernelkit")
+from kernelkit import workloads  # noqa: E402
 from kernelkit.geom.proj import Detector, ProjectionGeometry  # noqa: E402
 
 
@@ -32,7 +32,9 @@ def _rolled_orbit(angles, rows, cols, height, roll, sod=150.0, width=1.2):
     return out
 
 
-# rows per voxel: windows of 9 (up to 12) and of 13 rows (up to 16)
+# The unrolled walk where a column's rows are rounded up to the next unrolled
+# length (9 -> 12, 13 -> 16) and their slope along b is at its limit.  Rows per
+# voxel: windows of 9 and of 13 rows.
 @pytest.mark.parametrize("sign", [1, -1])
 @pytest.mark.parametrize("roll", [9.5, 10.0, 10.5, 10.9])
 @pytest.mark.parametrize("fine", [1.75, 1.8, 1.85, 1.92, 2.7, 2.75, 2.8])
@@ -42,6 +44,47 @@ def test_padded_windows(fine, roll, sign, device):
     pgs = _rolled_orbit(7, rows, 50, 1.5 / fine, sign * roll)
     vg = kk.resolve_volume_geometry(shape=(23, 18, 21), voxel_size=1.0)
     y = np.random.default_rng(1).uniform(size=(len(pgs), rows, 50))
+    got = kk.XrayTransform(pgs, vg).matched_T(
+        torch.from_numpy(y.astype(np.float32)).cuda()).cpu().numpy()
+    assert_parity(got, oracle.cone_fp_transpose(y, pgs, vg))
+
+
+# circular orbits of windows longer than the unrolled ones, all of the plan's
+# angles or not (rows four at a time, or one by one), and around the rule's line
+@pytest.mark.parametrize("tilted", [False, True])
+@pytest.mark.parametrize("fine", [2.9, 3.2, 3.6, 5.0, 6.1, 11.0])
+def test_long_windows_of_circular_orbits(fine, tilted, device):
+    import torch
+    rows = int(20 * fine) + 3
+    pgs = []
+    for kw in [{}] + [dict(tilt_deg=3.0)] * tilted:
+        for g in workloads.circular_geometry(5, 120.0, 60.0, rows, 40, 1.1,
+                                             **kw):
+            det = Detector(rows=rows, cols=40, pixel_height=1.5 / fine,
+                           pixel_width=1.1)
+            pgs.append(ProjectionGeometry(g.source_position,
+                                          g.detector_position, det, u=g.u,
+                                          v=g.v))
+    vg = kk.resolve_volume_geometry(shape=(20, 17, 19), voxel_size=1.0)
+    y = np.random.default_rng(2).uniform(size=(len(pgs), rows, 40))
+    got = kk.XrayTransform(pgs, vg).matched_T(
+        torch.from_numpy(y.astype(np.float32)).cuda()).cpu().numpy()
+    assert_parity(got, oracle.cone_fp_transpose(y, pgs, vg))
+
+
+# angles of a launch per share: 1, 2, 4, 8 and 16 shares (volumes of few and of
+# many workgroups)
+@pytest.mark.parametrize("shape,angles", [
+    ((20, 18, 17), 1), ((20, 18, 17), 2), ((20, 18, 17), 7),
+    ((20, 18, 17), 24), ((20, 18, 17), 70), ((90, 80, 5), 9),
+    ((90, 80, 5), 40), ((300, 280, 3), 4), ((300, 280, 3), 12)], ids=str)
+def test_shares_of_the_angles(shape, angles, device):
+    import torch
+    m = max(shape)
+    pgs = workloads.circular_geometry(angles, 3.0 * m, 1.5 * m, 12, 40,
+                                      1.7 * m / 40, wobble_deg=0.5, seed=3)
+    vg = kk.resolve_volume_geometry(shape=shape, voxel_size=1.0)
+    y = np.random.default_rng(5).uniform(size=(angles, 12, 40))
     got = kk.XrayTransform(pgs, vg).matched_T(
         torch.from_numpy(y.astype(np.float32)).cuda()).cpu().numpy()
     assert_parity(got, oracle.cone_fp_transpose(y, pgs, vg))
