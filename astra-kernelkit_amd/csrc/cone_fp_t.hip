@@ -531,27 +531,34 @@ __global__ __launch_bounds__(64 * SHARES, 6) void cone_fp_t_kernel(
                          static_cast<uint32_t>(r_lo));
       const uint32_t oend = o + 4u * (j < ncol ? nrow : 0u);
       float drf = 0.f;
-      for (; o < oend; o += 4u, drf += 1.f) {
-        // the load first: its latency overlaps the coordinates below.
+      // four rows per load (what it reads past the lane's box is of the
+      // column or its pad)
+      for (; o < oend; o += 16u) {
         // The empty asm keeps the offset a 32-bit register (an SGPR base
         // plus a VGPR offset), not a 64-bit pointer stepped per row.
         asm volatile("" : "+v"(o));
-        const float yv = *reinterpret_cast<const float*>(imgb + o);
-        const float rc = __builtin_amdgcn_rcpf(fmaf(drf, vaf, den0));
-        const float xc = fmaf(fmaf(drf, kvc, nc0), rc, oc);
-        const float xb = fmaf(fmaf(drf, kvb, nb0), rc, ob);
-        const float fl = floorf(xb);
-        if (fl != tcur) {
-          close_run(g, lane, tcur, S, T);
-          tcur = fl;
+        float y[4];
+        load_rows<4>(imgb + o, y);
+#pragma unroll
+        for (int t = 0; t < 4; ++t, drf += 1.f) {
+          if (t > 0 && o + 4u * t >= oend) break;
+          const float yv = y[t];
+          const float rc = __builtin_amdgcn_rcpf(fmaf(drf, vaf, den0));
+          const float xc = fmaf(fmaf(drf, kvc, nc0), rc, oc);
+          const float xb = fmaf(fmaf(drf, kvb, nb0), rc, ob);
+          const float fl = floorf(xb);
+          if (fl != tcur) {
+            close_run(g, lane, tcur, S, T);
+            tcur = fl;
+          }
+          const float yfb = yv * (xb - fl);
+          const float w0 = fmaxf(0.f, 1.f - fabsf(xc));
+          const float w1 = __builtin_amdgcn_fmed3f(0.f, xc, 2.f - xc);
+          S[0] = fmaf(yv, w0, S[0]);
+          S[1] = fmaf(yv, w1, S[1]);
+          T[0] = fmaf(yfb, w0, T[0]);
+          T[1] = fmaf(yfb, w1, T[1]);
         }
-        const float yfb = yv * (xb - fl);
-        const float w0 = fmaxf(0.f, 1.f - fabsf(xc));
-        const float w1 = __builtin_amdgcn_fmed3f(0.f, xc, 2.f - xc);
-        S[0] = fmaf(yv, w0, S[0]);
-        S[1] = fmaf(yv, w1, S[1]);
-        T[0] = fmaf(yfb, w0, T[0]);
-        T[1] = fmaf(yfb, w1, T[1]);
       }
     }
     close_run(g, lane, tcur, S, T);
