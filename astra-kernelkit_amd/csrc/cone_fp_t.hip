@@ -264,6 +264,13 @@ __device__ __forceinline__ int32_t bcast(int32_t v, int32_t l) {
 // Measured in ms for 4 / 8 / 16 shares: 128 workgroups 0.095 / 0.067 / 0.053,
 // 512 0.178 / 0.133 / 0.129, 1152 0.40 / 0.34 / 0.37, 2048 0.77 / 0.67 / 0.80,
 // 3400 1.52 / 1.50 / 1.81, 8280 3.17 / 3.21 / 4.36, 16384 9.1 / 9.1 / 12.0.
+// A share has an angle at least: wavefronts without any cost the others their
+// places.  In us with 1 / 2 / 4 / 8 / 16 shares, angles of a launch (calls of two
+// launches but for one angle), 8192 workgroups: one angle 64 / 78 / 114 / 209 /
+// 533, 2 angles 197 / 198 / 260 / 449 / 1152, 4 angles 323 / 324 / 335 / 463 /
+// 1197; 2048 workgroups: 2 angles 58 / 48 / 59 / 76 / 161, 4 angles 84 / 66 / 66 /
+// 80 / 169; 512: 2 angles 51 / 41 / 40 / 40 / 52, 8 angles 127 / 86 / 61 / 49 /
+// 59.
 constexpr int64_t kGenShares4 = 4096, kGenShares8 = 640;
 
 template <int SHARES>
@@ -939,6 +946,21 @@ int64_t general_grid(FptArgs& A) {
   return int64_t(A.na) * A.tiles_b * A.tiles_c;
 }
 
+int general_shares(int64_t blocks, int32_t n_angles) {
+  int shares = blocks >= kGenShares4 ? 4 : blocks >= kGenShares8 ? 8 : 16;
+  while (shares > 1 && n_angles < shares) shares /= 2;
+  return shares;
+}
+void launch_general(int shares, dim3 grid, hipStream_t st,
+                    const kk::FpAngle* tab, const FptArgs& A) {
+  auto* kernel = shares == 1   ? &cone_fp_t_kernel<1>
+                 : shares == 2 ? &cone_fp_t_kernel<2>
+                 : shares == 4 ? &cone_fp_t_kernel<4>
+                 : shares == 8 ? &cone_fp_t_kernel<8>
+                               : &cone_fp_t_kernel<16>;
+  hipLaunchKernelGGL(kernel, grid, dim3(64 * shares), 0, st, tab, A);
+}
+
 }  // namespace
 
 int64_t kk::fp_transpose_work_floats(const kk_plan_s* plan, int32_t rows,
@@ -1022,15 +1044,9 @@ int kk::fp_transpose_launch(const kk_plan_s* plan, const float* proj,
         else if (colc)
           hipLaunchKernelGGL(cone_fp_t_col_kernel<4>, grid,
                              dim3(64 * kColSlices * 4), 0, st, plan->fp, A);
-        else if (blocks >= kGenShares4)
-          hipLaunchKernelGGL(cone_fp_t_kernel<4>, grid, dim3(64 * 4), 0, st,
-                             plan->fp, A);
-        else if (blocks >= kGenShares8)
-          hipLaunchKernelGGL(cone_fp_t_kernel<8>, grid, dim3(64 * 8), 0, st,
-                             plan->fp, A);
         else
-          hipLaunchKernelGGL(cone_fp_t_kernel<16>, grid, dim3(64 * 16), 0, st,
-                             plan->fp, A);
+          launch_general(general_shares(blocks, A.n_angles), grid, st,
+                         plan->fp, A);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return kk::hip_fail(e, "cone_fp_t_kernel");
       }
