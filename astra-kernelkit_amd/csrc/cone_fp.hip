@@ -527,12 +527,13 @@ constexpr int fp_waves(int r) { return r <= 2 ? 8 : 5; }
 // 1.25; with two rows 1.30 and 1.18).
 constexpr bool fp_pipe(int r) { return r <= 1; }
 
+// One row per thread: whether the angles are column-coherent is the same.
 // PTRS: output through the table of entry pointers (kk_cone_fp_ptrs); a
 // separate instantiation, so the plain kernel's code is unchanged.
-template <int R, bool ALL_COLC, bool PTRS>
-__global__ __launch_bounds__(kColsSingle * kWave, fp_waves(R)) void cone_fp_kernel(
-    const kk::FpAngle* __restrict__ tab, FpArgs A) {
-  fp_tile<R, ALL_COLC, fp_pipe(R), kColsSingle, false, PTRS>(
+template <bool PTRS>
+__global__ __launch_bounds__(kColsSingle * kWave, fp_waves(1)) void
+cone_fp_kernel(const kk::FpAngle* __restrict__ tab, FpArgs A) {
+  fp_tile<1, false, fp_pipe(1), kColsSingle, false, PTRS>(
       tab, A, kk_xcd_remap(blockIdx.x, A.total_blocks, A.xcd_group));
 }
 
@@ -941,47 +942,6 @@ __global__ __launch_bounds__(kColsBatch * kWave, fp_waves(R)) void cone_fp_batch
   }
 }
 
-template <bool C, bool P>
-void launch_single(int32_t rpt, dim3 grid, hipStream_t stream,
-                   const kk::FpAngle* tab, const FpArgs& A) {
-  const dim3 block(kColsSingle * kWave);
-  switch (rpt) {
-    case 1:
-      hipLaunchKernelGGL((cone_fp_kernel<1, C, P>), grid, block, 0, stream,
-                         tab, A);
-      break;
-    case 2:
-      hipLaunchKernelGGL((cone_fp_kernel<2, C, P>), grid, block, 0, stream,
-                         tab, A);
-      break;
-    default:
-      hipLaunchKernelGGL((cone_fp_kernel<4, C, P>), grid, block, 0, stream,
-                         tab, A);
-      break;
-  }
-}
-
-template <bool C>
-void launch_batch(int32_t rpt, dim3 grid, hipStream_t stream,
-                  const FpItem* items, const int64_t* first, int32_t n,
-                  int64_t total) {
-  const dim3 block(kColsBatch * kWave);
-  switch (rpt) {
-    case 1:
-      hipLaunchKernelGGL((cone_fp_batch_kernel<1, C>), grid, block, 0, stream,
-                         items, first, n, total);
-      break;
-    case 2:
-      hipLaunchKernelGGL((cone_fp_batch_kernel<2, C>), grid, block, 0, stream,
-                         items, first, n, total);
-      break;
-    default:
-      hipLaunchKernelGGL((cone_fp_batch_kernel<4, C>), grid, block, 0, stream,
-                         items, first, n, total);
-      break;
-  }
-}
-
 }  // namespace
 
 namespace kk {
@@ -1049,12 +1009,14 @@ int fp_batch_launch(const FpBatch* b, int32_t grid_blocks,
   if (g > b->total) g = b->total;
   if (g <= 0) return KK_OK;
   const dim3 grid(static_cast<unsigned>(g));
-  if (b->all_colc)
-    launch_batch<true>(b->rpt, grid, stream, b->items, b->first, b->n,
-                       b->total);
-  else
-    launch_batch<false>(b->rpt, grid, stream, b->items, b->first, b->n,
-                        b->total);
+  auto* kernel =
+      b->rpt == 1   ? &cone_fp_batch_kernel<1, false>
+      : b->rpt == 2 ? (b->all_colc ? &cone_fp_batch_kernel<2, true>
+                                   : &cone_fp_batch_kernel<2, false>)
+                    : (b->all_colc ? &cone_fp_batch_kernel<4, true>
+                                   : &cone_fp_batch_kernel<4, false>);
+  hipLaunchKernelGGL(kernel, grid, dim3(kColsBatch * kWave), 0, stream,
+                     b->items, b->first, b->n, b->total);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return hip_fail(e, "cone_fp_batch_kernel");
   return KK_OK;
@@ -1116,24 +1078,16 @@ int sirt_residual_spec(FpSpec& S, const kk_plan* plan, const float* x_tex,
 
 namespace {
 
-int launch_fp_spec(const kk::FpSpec& S, int32_t rows_per_thread,
-                   hipStream_t stream) {
-  const FpLanes lanes = fp_lanes(S.rows, rows_per_thread, false);
-  const int32_t rpt = lanes.rpt;
+int launch_fp_spec(const kk::FpSpec& S, hipStream_t stream) {
   FpArgs A;
-  const int rc = make_fp_args(S, lanes, kColsSingle, kGroupAngles,
-                              kGroupCols, A);
+  const int rc = make_fp_args(S, fp_lanes(S.rows, 0, false), kColsSingle,
+                              kGroupAngles, kGroupCols, A);
   if (rc != KK_OK) return rc;
   const dim3 grid(static_cast<unsigned>(A.total_blocks));
-  const bool c = S.plan->fp_all_colc, p = S.ptrs != nullptr;
-  if (c && !p)
-    launch_single<true, false>(rpt, grid, stream, S.plan->fp, A);
-  else if (!c && !p)
-    launch_single<false, false>(rpt, grid, stream, S.plan->fp, A);
-  else if (c)
-    launch_single<true, true>(rpt, grid, stream, S.plan->fp, A);
-  else
-    launch_single<false, true>(rpt, grid, stream, S.plan->fp, A);
+  const dim3 block(kColsSingle * kWave);
+  auto* kernel = S.ptrs != nullptr ? &cone_fp_kernel<true>
+                                   : &cone_fp_kernel<false>;
+  hipLaunchKernelGGL(kernel, grid, block, 0, stream, S.plan->fp, A);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return kk::hip_fail(e, "cone_fp_kernel");
   return KK_OK;
@@ -1243,7 +1197,7 @@ extern "C" int kk_cone_fp(const kk_plan* plan, const float* vol_tex,
   const int rc = kk::fp_spec(S, plan, vol_tex, proj, ps, rows, cols,
                              additive);
   if (rc != KK_OK) return rc;
-  return launch_fp_spec(S, 0, static_cast<hipStream_t>(stream));
+  return launch_fp_spec(S, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int kk_cone_fp_ptrs(const kk_plan* plan, const float* vol_tex,
@@ -1258,7 +1212,7 @@ extern "C" int kk_cone_fp_ptrs(const kk_plan* plan, const float* vol_tex,
   if (rc != KK_OK) return rc;
   S.ptrs = ptrs;
   S.ptr_axis = ptr_axis;
-  return launch_fp_spec(S, 0, static_cast<hipStream_t>(stream));
+  return launch_fp_spec(S, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int kk_sirt_fp_residual(const kk_plan* plan, const float* x_tex,
@@ -1270,5 +1224,5 @@ extern "C" int kk_sirt_fp_residual(const kk_plan* plan, const float* x_tex,
   const int rc = kk::sirt_residual_spec(S, plan, x_tex, y, ys, R, rs,
                                         res_tex, n_angles, rows, cols);
   if (rc != KK_OK) return rc;
-  return launch_fp_spec(S, 0, static_cast<hipStream_t>(stream));
+  return launch_fp_spec(S, static_cast<hipStream_t>(stream));
 }
