@@ -178,6 +178,11 @@ struct RayWalk {
   int64_t gb[NB], gc[R];
 };
 
+// Slices walked from one float64 coordinate, at most: a step's rounding (2^-33
+// voxel) then adds up to 512 of them, 2^-24 voxel, like a weight's own float32
+// rounding, however long the volume's axis is.
+constexpr int32_t kSegment = 1024;
+
 // Coordinate a i + b at slice mid, the middle of the slices that the ray
 // meets, and its step: the step's rounding (2^-33 voxel per slice) adds up over
 // half of them at most, and cancels in the ray's sum (a ray that only grazes
@@ -364,7 +369,9 @@ __device__ __forceinline__ bool graze_sum(const kk::FpAngle& P, int32_t row,
 // block id `bid`.  ALL_COLC: every angle of the launch is column-coherent,
 // so a thread keeps one b slope/intercept for its R rays (fewer registers,
 // more wavefronts in flight); otherwise the angle's flag picks the path.
-template <int R, bool ALL_COLC, bool PIPE, int COLS, bool PTRS = false>
+// FAR: the plan has an axis of more than kSegment slices.
+template <int R, bool ALL_COLC, bool PIPE, int COLS, bool FAR,
+          bool PTRS = false>
 __device__ __forceinline__ void fp_tile_at(
     const kk::FpAngle* __restrict__ tab, int32_t ti, const FpArgs& A,
     int32_t ang, int32_t ct, int32_t rt) {
@@ -440,7 +447,31 @@ __device__ __forceinline__ void fp_tile_at(
     for (int k = 0; k < R; ++k)
       w.c[k] += static_cast<int64_t>(ilo - mc[k]) * w.gc[k];
     const char* frame = A.tex + P.tex_off;
-    trace<R, NB, PIPE>(P, frame, w, ilo, ihi, acc);
+    if constexpr (!FAR) {
+      trace<R, NB, PIPE>(P, frame, w, ilo, ihi, acc);
+    } else {
+#pragma unroll 1
+      for (int32_t s = ilo; s <= ihi; s += kSegment) {
+        const int32_t e = min(ihi, s + kSegment - 1), mid = s + (e - s) / 2;
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+          const int32_t row = row0 + rows * k;
+          double a1, b1, a2, b2;
+          if (!(row < A.rows && col < A.cols &&
+                kk_fp_ray(P, row, col, a1, b1, a2, b2))) {
+            a1 = a2 = 0.0;
+            b1 = b2 = 1.0;
+          }
+          if (k < NB) {
+            fixed_ray(a1, b1, P.na, mid, nb1, w.b[k], w.gb[k]);
+            w.b[k] -= static_cast<int64_t>(mid - s) * w.gb[k];
+          }
+          fixed_ray(a2, b2, P.na, mid, nc1, w.c[k], w.gc[k]);
+          w.c[k] -= static_cast<int64_t>(mid - s) * w.gc[k];
+        }
+        trace<R, NB, PIPE>(P, frame, w, s, e, acc);
+      }
+    }
     if (graze) {
 #pragma unroll 1
       for (int32_t k = 0; k < R; ++k) {
@@ -507,16 +538,16 @@ __device__ __forceinline__ bool fp_decode(const FpArgs& A, int64_t bid,
 // as a kernel argument is read in place (the compiler scalarizes it by
 // itself; the explicit copy measured 5% slower at 512^3 / 720 angles).
 template <int R, bool ALL_COLC, bool PIPE, int COLS, bool TABLE_IN_MEMORY,
-          bool PTRS = false>
+          bool FAR, bool PTRS = false>
 __device__ __forceinline__ void fp_tile(const kk::FpAngle* __restrict__ tab,
                                         const FpArgs& A, int64_t bid) {
   int32_t ang, ct, rt;
   if (!fp_decode(A, bid, ang, ct, rt)) return;
   if constexpr (TABLE_IN_MEMORY) {
     const kk::FpAngle rec = kk_uniform_load(tab + ang);
-    fp_tile_at<R, ALL_COLC, PIPE, COLS, PTRS>(&rec, 0, A, ang, ct, rt);
+    fp_tile_at<R, ALL_COLC, PIPE, COLS, FAR, PTRS>(&rec, 0, A, ang, ct, rt);
   } else {
-    fp_tile_at<R, ALL_COLC, PIPE, COLS, PTRS>(tab, ang, A, ang, ct, rt);
+    fp_tile_at<R, ALL_COLC, PIPE, COLS, FAR, PTRS>(tab, ang, A, ang, ct, rt);
   }
 }
 
@@ -530,10 +561,10 @@ constexpr bool fp_pipe(int r) { return r <= 1; }
 // One row per thread: whether the angles are column-coherent is the same.
 // PTRS: output through the table of entry pointers (kk_cone_fp_ptrs); a
 // separate instantiation, so the plain kernel's code is unchanged.
-template <bool PTRS>
+template <bool FAR, bool PTRS>
 __global__ __launch_bounds__(kColsSingle * kWave, fp_waves(1)) void
 cone_fp_kernel(const kk::FpAngle* __restrict__ tab, FpArgs A) {
-  fp_tile<1, false, fp_pipe(1), kColsSingle, false, PTRS>(
+  fp_tile<1, false, fp_pipe(1), kColsSingle, false, FAR, PTRS>(
       tab, A, kk_xcd_remap(blockIdx.x, A.total_blocks, A.xcd_group));
 }
 
@@ -563,8 +594,9 @@ cone_fp_kernel(const kk::FpAngle* __restrict__ tab, FpArgs A) {
 //
 // c coordinates are 64-bit fixed point (32 fraction bits), stepped by one
 // 64-bit add per slice: the high word is the element, the low word the
-// weight.  Their error (the slope's rounding, 2^-33 per slice) is below the
-// weights' own float32 rounding up to ~1000 slices.
+// weight.  Their error (the slope's rounding, 2^-33 voxel per slice from the
+// middle one) stays at the weights' own float32 rounding for the volumes that
+// line_spacing admits.
 // Columns (wavefronts) per workgroup.  They walk the same slices behind one
 // barrier per slice, so that neighbouring columns' rows meet in the CU's L1
 // (57.0 ms against 62.5 without; 8 and 16 columns 59.2 and 61.9 ms).
@@ -729,21 +761,24 @@ __global__ __launch_bounds__(kLineWaves * kWave, 8) void cone_fp_line_kernel(
 #pragma unroll
   for (int k = 0; k < R; ++k) acc[k] = 0.f;
   if (ilo <= ihi) {
-    const double fi = static_cast<double>(ilo);
+    // from the middle slice, where the steps' rounding cancels
+    const int32_t n = ihi - ilo + 1;
+    const double fm = static_cast<double>(ilo + n / 2);
     LineWalk<R> w;
 #pragma unroll
     for (int k = 0; k < R; ++k) {
-      w.X[k] = to_fixed(fma(a2[k], fi, b2[k]));
       w.S[k] = to_fixed(a2[k]);
+      w.X[k] = to_fixed(fma(a2[k], fm, b2[k])) -
+               static_cast<int64_t>(n / 2) * w.S[k];
     }
-    w.B = bcast64(to_fixed(fma(a1, fi, b1)), 0);
     w.SB = bcast64(to_fixed(a1), 0);
+    w.B = bcast64(to_fixed(fma(a1, fm, b1)), 0) -
+          static_cast<int64_t>(n / 2) * w.SB;
     // the window lies between the c coordinates of the first and last rows
     // (those between lie between up to the rounding that kLineEps covers);
     // which is the lower does not change along the slices
     const int64_t E0 = bcast64(w.X[0], 0), E1 = bcast64(w.X[R - 1], kWave - 1);
     const int64_t S0 = bcast64(w.S[0], 0), S1 = bcast64(w.S[R - 1], kWave - 1);
-    const int32_t n = ihi - ilo + 1;
     const bool up = E1 + (n >> 1) * S1 >= E0 + (n >> 1) * S0;
     w.E = bcast64((up ? E0 : E1) - kLineEps, 0);
     w.SE = bcast64(up ? S0 : S1, 0);
@@ -922,7 +957,7 @@ struct FpItem {
   FpArgs args;
 };
 
-template <int R, bool ALL_COLC>
+template <int R, bool ALL_COLC, bool FAR>
 __global__ __launch_bounds__(kColsBatch * kWave, fp_waves(R)) void cone_fp_batch_kernel(
     const FpItem* __restrict__ items, const int64_t* __restrict__ first,
     int32_t n, int64_t total) {
@@ -937,9 +972,17 @@ __global__ __launch_bounds__(kColsBatch * kWave, fp_waves(R)) void cone_fp_batch
     }
     const FpItem& it = items[lo];
     const int64_t local = g - first[lo];
-    fp_tile<R, ALL_COLC, fp_pipe(R), kColsBatch, true>(it.tab, it.args,
+    fp_tile<R, ALL_COLC, fp_pipe(R), kColsBatch, true, FAR>(it.tab, it.args,
                kk_xcd_remap(local, it.args.total_blocks, it.args.xcd_group));
   }
+}
+
+// Whether the plan has an axis of more than kSegment slices.
+bool fp_far(const kk_plan_s* plan) {
+  for (int a = 0; a < 3; ++a)
+    if ((plan->fp_mask & (1 << a)) && plan->fp_shape[a] > kSegment)
+      return true;
+  return false;
 }
 
 }  // namespace
@@ -953,6 +996,7 @@ struct FpBatch {
   int64_t total = 0;
   int32_t rpt = 4;
   bool all_colc = false;
+  bool far = false;
 };
 
 int fp_batch_build(const std::vector<FpSpec>& specs, int32_t rows_per_thread,
@@ -960,7 +1004,10 @@ int fp_batch_build(const std::vector<FpSpec>& specs, int32_t rows_per_thread,
   if (specs.empty()) return fail(KK_ERR_INVALID, "empty forward batch");
   int32_t max_rows = 0;
   for (const FpSpec& S : specs) max_rows = S.rows > max_rows ? S.rows : max_rows;
-  const FpLanes lanes = fp_lanes(max_rows, rows_per_thread, true);
+  bool far = false;
+  for (const FpSpec& S : specs)
+    far = far || (S.plan != nullptr && S.plan->fp_set && fp_far(S.plan));
+  const FpLanes lanes = fp_lanes(max_rows, far ? 1 : rows_per_thread, true);
   std::vector<FpItem> items(specs.size());
   std::vector<int64_t> first(specs.size());
   int64_t total = 0;
@@ -977,6 +1024,7 @@ int fp_batch_build(const std::vector<FpSpec>& specs, int32_t rows_per_thread,
   b->n = static_cast<int32_t>(specs.size());
   b->total = total;
   b->rpt = lanes.rpt;
+  b->far = far;
   b->all_colc = true;
   for (const FpSpec& S : specs) b->all_colc = b->all_colc && S.plan->fp_all_colc;
   hipError_t e = hipMalloc(&b->items, sizeof(FpItem) * items.size());
@@ -1010,11 +1058,12 @@ int fp_batch_launch(const FpBatch* b, int32_t grid_blocks,
   if (g <= 0) return KK_OK;
   const dim3 grid(static_cast<unsigned>(g));
   auto* kernel =
-      b->rpt == 1   ? &cone_fp_batch_kernel<1, false>
-      : b->rpt == 2 ? (b->all_colc ? &cone_fp_batch_kernel<2, true>
-                                   : &cone_fp_batch_kernel<2, false>)
-                    : (b->all_colc ? &cone_fp_batch_kernel<4, true>
-                                   : &cone_fp_batch_kernel<4, false>);
+      b->far        ? &cone_fp_batch_kernel<1, false, true>
+      : b->rpt == 1 ? &cone_fp_batch_kernel<1, false, false>
+      : b->rpt == 2 ? (b->all_colc ? &cone_fp_batch_kernel<2, true, false>
+                                   : &cone_fp_batch_kernel<2, false, false>)
+                    : (b->all_colc ? &cone_fp_batch_kernel<4, true, false>
+                                   : &cone_fp_batch_kernel<4, false, false>);
   hipLaunchKernelGGL(kernel, grid, dim3(kColsBatch * kWave), 0, stream,
                      b->items, b->first, b->n, b->total);
   hipError_t e = hipGetLastError();
@@ -1085,8 +1134,11 @@ int launch_fp_spec(const kk::FpSpec& S, hipStream_t stream) {
   if (rc != KK_OK) return rc;
   const dim3 grid(static_cast<unsigned>(A.total_blocks));
   const dim3 block(kColsSingle * kWave);
-  auto* kernel = S.ptrs != nullptr ? &cone_fp_kernel<true>
-                                   : &cone_fp_kernel<false>;
+  const bool far = fp_far(S.plan), ptrs = S.ptrs != nullptr;
+  auto* kernel = far ? (ptrs ? &cone_fp_kernel<true, true>
+                             : &cone_fp_kernel<true, false>)
+                     : (ptrs ? &cone_fp_kernel<false, true>
+                             : &cone_fp_kernel<false, false>);
   hipLaunchKernelGGL(kernel, grid, block, 0, stream, S.plan->fp, A);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return kk::hip_fail(e, "cone_fp_kernel");

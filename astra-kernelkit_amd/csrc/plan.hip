@@ -224,7 +224,8 @@ static int build_fp_table(const double* params, int32_t n,
 // (slices by a few, b by up to four columns' distance).  Negative if an angle
 // is not column-coherent, if a ray may run parallel to the slices (D_a
 // changes sign or nearly vanishes), if the source lies among the slices, or
-// if coordinates leave the fixed-point range.
+// if there are more slices than the line kernel's steps are good for (2048:
+// 2^-23 voxel).
 static void line_spacing(const std::vector<kk::FpAngle>& tab, int32_t rows,
                          int32_t cols, kk_plan_s& plan) {
   plan.fp_line_max = -1.0;
@@ -234,7 +235,7 @@ static void line_spacing(const std::vector<kk::FpAngle>& tab, int32_t rows,
   if (rows <= 0 || cols <= 0) return;
   double most = 0.0, sum = 0.0;
   for (const kk::FpAngle& e : tab) {
-    if (!e.colc || e.na > 16384) return;
+    if (!e.colc || e.na > 2048) return;
     const double da[2] = {e.qa, e.qa + (cols - 1) * e.ua};
     const double least = std::fmin(std::fabs(da[0]), std::fabs(da[1]));
     if (!(da[0] * da[1] > 0.0) ||

@@ -79,3 +79,12 @@ def test_fixed_point_steps_stay_below_float32_weights():
     for n in (256, 1024):
         err = np.abs((X + S * n) / 2.0 ** 32 - (a * n + b))
         assert err.max() <= (n + 2) * 2.0 ** -32
+
+
+def test_spacing_refuses_axes_longer_than_its_steps_are_good_for():
+    """Steps of 2^-32 voxel, rounded, from the middle slice: 2^-23 voxel off at
+    the ends of 2048 slices."""
+    for n, fine in ((2048, True), (2049, False)):
+        pgs = workloads.circular_geometry(1, 3.0 * n, 1.5 * n, 70, 20, 1.0)
+        vg = kk.resolve_volume_geometry(shape=(n, 8, 40), voxel_size=1.0)
+        assert bool(_spacing(pgs, vg, 70, 20)[2][0] > 0) is fine
