@@ -1147,20 +1147,53 @@ int launch_fp_spec(const kk::FpSpec& S, hipStream_t stream) {
 
 // Rows per thread of the line kernel for `rows` detector rows at the plan's
 // c spacing (0: the launch is the gather kernel's).  Costs in cycles of a
-// SIMD, fitted on MI355X at 64 to 384 rows and spacings of 0.5 to 1.7 voxels:
-// a slice costs a wavefront 72 + 30 R, the gather 72 per 64 rows, and more
-// where its lanes spread over the cache lines (spacing above 1).  The line
-// kernel then took 0.52-0.90 of the gather's time where it is chosen: at 0.7
-// voxels 128 rows 0.89 -> 0.77 ms (R = 2), 190 rows 1.52 -> 0.91 (R = 3),
-// 384 rows 5.79 -> 4.18 (R = 3); at 1.7 voxels 384 rows 7.12 -> 4.78 (R = 1).
+// SIMD, fitted on MI355X over 1400 circular geometries (volumes of 24 to 512
+// voxels, 1 to 400 angles, spacings of 0.4 to 2 voxels; calls with their texture
+// builds): a slice costs the line kernel's wavefront 72 + 30 R, the gather 66
+// per 64 rows, and more where its lanes spread over the cache lines (spacing
+// above 1), less so if the volume's pairs stay in the caches (one frame up to
+// kGatherCached bytes).
+// * The gather's wavefronts are 32 rows (fewer for fewer rows) by two columns
+//   or more, the line kernel's 64 rows of one: 388 slices, 308 angles, 4 rows
+//   at a spacing of 1.3 voxels 0.19 ms by gathers and 1.31 by lines, 32 rows at
+//   512^2 x 32, 360 angles 1.21 and 3.29.  Beyond 32 rows of a volume that the
+//   caches don't hold, both come in steps of 64 rows.
+// * Launches of few workgroups are as long as one wavefront: a slice takes 0.2
+//   us by gathers, 0.35 by lines.  256^3, one angle of 384^2 98 and 135 us, three
+//   angles 233 and 176; 128^3, 16 angles of 160^2 56 and 77 us, 64 angles 118 and
+//   110.  (Where pairs have to be built of a large volume the line is lower:
+//   they are twice the bytes.  Volumes of a few slices are as long as the call's
+//   host part either way.)
+constexpr int64_t kGatherCached = 90 << 20;
+constexpr int64_t kGatherFew = 600, kGatherFewCached = 2500;  // workgroups
+constexpr int32_t kGatherSlices = 64;
 int line_rows_per_thread(const kk_plan_s* plan, int32_t rows, int32_t cols) {
   if (!plan->fp_set || plan->fp_line_max < 0.0 || cols > plan->fp_line_cols ||
       rows > plan->fp_line_rows)
     return 0;
+  int64_t frame = 0;   // bytes of the largest frame of pairs
+  int32_t slices = 0;  // and of slices
+  for (int a = 0; a < 3; ++a) {
+    if (!(plan->fp_mask & (1 << a))) continue;
+    frame = std::max(frame, 8 * kk::frame_elems(plan->fp_shape, a));
+    slices = std::max(slices, plan->fp_shape[a]);
+  }
+  const FpLanes g = fp_lanes(rows, 0, false);
+  const int32_t g_rows = g.rpt << g.row_shift;
+  const int32_t g_cols = kColsSingle << (6 - g.row_shift);
+  const int32_t g_tiles = (rows + g_rows - 1) / g_rows;
+  const bool cached = slices >= kGatherSlices && frame <= kGatherCached;
+  if (slices >= kGatherSlices &&
+      int64_t(plan->fp_n) * g_tiles * ((cols + g_cols - 1) / g_cols) <=
+          (cached ? kGatherFewCached : kGatherFew))
+    return 0;
   const int32_t groups = (rows + kWave - 1) / kWave;
-  const double spread = std::max(0.0, 1.9 * (plan->fp_line_mean - 1.0));
+  const double spread = (cached ? 0.6 : 1.9) *
+                        std::max(0.0, plan->fp_line_mean - 1.0);
   int best = 0;
-  double best_cost = 0.92 * 72.0 * groups * (1.0 + spread);
+  double best_cost =
+      66.2 * (1.0 + spread) *
+      (cached || rows <= 32 ? g_tiles * g_rows / double(kWave) : groups);
   for (int r = 1; r <= 4; ++r) {
     // the widest window must fit (its ends' rounding and margins: 4)
     const int32_t span = std::min(kWave * r, rows) - 1;
