@@ -1084,8 +1084,21 @@ bool patch_extent(const std::vector<kk::BpAngle>& tab, const int32_t shape[3],
   return true;
 }
 
-// Whether every patch fits kPatchCols columns and kPatchLanes rows.  The
-// answer for the last detector and volume is kept with the plan.
+// Whether the patch kernel is the faster one for the volume's tiles: not where
+// half of its only layer of tiles is empty and there are more tiles than CUs to
+// hide that (180 angles, patch and pair kernel in us, x = y and z: circular
+// (512, 8) 310 and 205, (384, 8) 281 and 186, (512, 9) 310 and 376, (256, 8) 101
+// and 176; general (512, 8) 477 and 387, (384, 8) 381 and 317, (512, 9) 478 and
+// 681).
+bool patches_pay(const int32_t shape[3]) {
+  const int64_t cols = ((int64_t(shape[0]) + 15) / 16) *
+                       ((int64_t(shape[1]) + 15) / 16);
+  return shape[2] > kPatchRun / 2 || cols <= 256;
+}
+
+// Whether every patch fits kPatchCols columns and kPatchLanes rows, and the
+// patches pay.  The answer for the last detector and volume is kept with the
+// plan.
 bool patches_fit(const kk_plan_s& plan, int32_t rows, int32_t cols,
                  const int32_t shape[3]) {
   if (rows <= 0 || cols <= 0) return false;
@@ -1096,7 +1109,10 @@ bool patches_fit(const kk_plan_s& plan, int32_t rows, int32_t cols,
     double ext[2];
     const bool ok = patch_extent(plan.bp_host, shape, ext);
     plan.bp_patch_fits =
-        ok && ext[0] <= kPatchCols && ext[1] <= kPatchLanes ? 1 : 0;
+        ok && ext[0] <= kPatchCols && ext[1] <= kPatchLanes &&
+                patches_pay(shape)
+            ? 1
+            : 0;
     std::copy(shape, shape + 3, plan.bp_patch_shape);
   }
   return plan.bp_patch_fits == 1;
@@ -1113,10 +1129,15 @@ int launch_bp_planes(const kk::BpSpec& S, hipStream_t stream) {
   const int64_t pitch = int64_t(S.rows + kPatchGap) * 4;
   A.trb = uint32_t(pitch);
   A.tab_b = uint32_t(pitch * S.cols);
-  // parts so that a CU (of 256) holds at least four wavefronts per SIMD
+  // Parts so that a CU (of 256) holds four wavefronts per SIMD, on circular
+  // orbits three (tiles all resident, where two parts leave some waiting): 180
+  // angles with 1 / 2 / 4 parts, circular, 64 tiles 228 / 139 / 101 us, 288 238 /
+  // 174 / 193, 512 243 / 178 / 195, 576 272 / 282 / 281, 768 279 / 305 / 287, 1024
+  // 322 / 335 / 374; general 576 393 / 386 / 410, 768 398 / 416 / 415.
   const int64_t per_cu = (A.total_blocks + 255) / 256;
   const dim3 grid(unsigned(A.total_blocks));
-  const int32_t parts = per_cu >= 4 ? 1 : per_cu >= 2 ? 2 : 4;
+  const int32_t parts =
+      per_cu >= (S.plan->bp_all_circ ? 3 : 4) ? 1 : per_cu >= 2 ? 2 : 4;
   auto launch = [&](auto circ) {
     constexpr bool C = decltype(circ)::value;
     auto* kernel = parts == 1   ? &cone_bp_patch_kernel<kPatchRun, 1, C>

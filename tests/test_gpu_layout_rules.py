@@ -48,3 +48,18 @@ def test_forward(case, device):
     k = [0, len(pgs) // 2, len(pgs) - 1]
     assert_parity(y.cpu().numpy()[k],
                   oracle.cone_fp(vol, [pgs[i] for i in k], vg))
+
+
+# volumes of one layer of tiles, half of it empty or not, of fewer tiles than
+# CUs and of more
+@pytest.mark.parametrize("kw", [{}, dict(wobble_deg=0.5)],
+                         ids=["circular", "wobble"])
+@pytest.mark.parametrize("shape,planes", [
+    ((256, 250, 8), True), ((272, 250, 8), False), ((272, 250, 9), True),
+    ((272, 258, 1), False)], ids=str)
+def test_backprojection(shape, planes, kw, device):
+    A, pgs, vg = _operator(shape, 4, 14, 300, 1.2, **kw)
+    assert A.backprojector.kernel.reads_planes is planes
+    y = np.random.default_rng(4).uniform(size=(4, 14, 300)).astype(np.float32)
+    x = A.T(_dev(y))
+    assert_parity(x.cpu().numpy(), oracle.cone_bp(y, pgs, vg))
