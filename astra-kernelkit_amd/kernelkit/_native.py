@@ -351,7 +351,8 @@ def stream_ptr(stream=None) -> ctypes.c_void_p:
 def release(destructor: str, ptr: ctypes.c_void_p) -> None:
     """Call the library's ``destructor`` on ``ptr``; while this thread
     captures (:meth:`Graph.capture`), once the capture has ended: a free of
-    device memory, by the cycle collector for one, ends a capture."""
+    device memory, by the cycle collector for one, ends a capture.
+    (Destructors bind it: they may run when this module is no more.)"""
     try:
         held = getattr(_local, "held", None)
         if held is not None:
@@ -390,7 +391,7 @@ class Plan:
     def ptr(self) -> ctypes.c_void_p:
         return self._ptr
 
-    def __del__(self):
+    def __del__(self, release=release):
         ptr = getattr(self, "_ptr", None)
         if ptr is not None and ptr.value:
             release("kk_plan_destroy", ptr)
@@ -410,7 +411,7 @@ class Batch:
     def ptr(self) -> ctypes.c_void_p:
         return self._ptr
 
-    def __del__(self):
+    def __del__(self, release=release):
         ptr = getattr(self, "_ptr", None)
         if ptr is not None and ptr.value:
             release("kk_batch_destroy", ptr)
@@ -431,7 +432,7 @@ class Filter:
     def ptr(self) -> ctypes.c_void_p:
         return self._ptr
 
-    def __del__(self):
+    def __del__(self, release=release):
         ptr = getattr(self, "_ptr", None)
         if ptr is not None and ptr.value:
             release("kk_filter_destroy", ptr)
@@ -465,7 +466,7 @@ class Stream:
     def synchronize(self) -> None:
         check(lib().kk_stream_synchronize(self._ptr))
 
-    def __del__(self):
+    def __del__(self, release=release):
         ptr = getattr(self, "_ptr", None)
         if ptr is not None and ptr.value:
             release("kk_stream_destroy", ptr)
@@ -496,7 +497,7 @@ class Event:
                                         ctypes.byref(ms)))
         return float(ms.value)
 
-    def __del__(self):
+    def __del__(self, release=release):
         ptr = getattr(self, "_ptr", None)
         if ptr is not None and ptr.value:
             release("kk_event_destroy", ptr)
@@ -542,7 +543,7 @@ class Graph:
     def replay(self, stream=None) -> None:
         check(lib().kk_graph_launch(self._ptr, stream_ptr(stream)))
 
-    def __del__(self):
+    def __del__(self, release=release):
         ptr = getattr(self, "_ptr", None)
         if ptr is not None and ptr.value:
             release("kk_graph_destroy", ptr)

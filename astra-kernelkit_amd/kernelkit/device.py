@@ -86,10 +86,10 @@ class _Buffer:
         self.ptr = int(p.value or 0)
         self.nbytes = int(nbytes)
 
-    def __del__(self):
+    def __del__(self, release=_native.release, address=ctypes.c_void_p):
         ptr = getattr(self, "ptr", 0)
         if ptr:
-            _native.release("kk_free", ctypes.c_void_p(ptr))
+            release("kk_free", address(ptr))
             self.ptr = 0
 
 

@@ -2,6 +2,7 @@
 with library objects that die while a stream records, shown with a stub in the
 library's place."""
 import gc
+import sys
 import threading
 
 import pytest
@@ -154,3 +155,21 @@ def test_a_capture_inside_a_capture_keeps_the_outer_ones_objects(stub):
 
     _native.Graph.capture(body)
     assert "kk_plan_destroy" in s.calls
+
+
+def test_objects_that_outlive_the_module_say_nothing(stub, monkeypatch):
+    """At the interpreter's end a module's names may be gone before the last
+    objects are."""
+    stub()
+    owned = [_native.Plan(), _native.Batch(), _native.Filter(),
+             _native.Stream(), _native.Event(), device._Buffer(4),
+             _native.Graph(_native._vp(77))]
+    said = []
+    monkeypatch.setattr(sys, "unraisablehook", said.append)
+    for name in ("release", "_local", "_lib", "lib", "_vp"):
+        monkeypatch.setattr(_native, name, None)
+    monkeypatch.setattr(device, "ctypes", None)
+    monkeypatch.setattr(device, "_native", None)
+    del owned
+    gc.collect()
+    assert said == []
