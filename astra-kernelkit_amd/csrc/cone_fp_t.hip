@@ -264,13 +264,12 @@ __device__ __forceinline__ int32_t bcast(int32_t v, int32_t l) {
 // Measured in ms for 4 / 8 / 16 shares: 128 workgroups 0.095 / 0.067 / 0.053,
 // 512 0.178 / 0.133 / 0.129, 1152 0.40 / 0.34 / 0.37, 2048 0.77 / 0.67 / 0.80,
 // 3400 1.52 / 1.50 / 1.81, 8280 3.17 / 3.21 / 4.36, 16384 9.1 / 9.1 / 12.0.
-// A share has an angle at least: wavefronts without any cost the others their
-// places.  In us with 1 / 2 / 4 / 8 / 16 shares, angles of a launch (calls of two
-// launches but for one angle), 8192 workgroups: one angle 64 / 78 / 114 / 209 /
-// 533, 2 angles 197 / 198 / 260 / 449 / 1152, 4 angles 323 / 324 / 335 / 463 /
-// 1197; 2048 workgroups: 2 angles 58 / 48 / 59 / 76 / 161, 4 angles 84 / 66 / 66 /
-// 80 / 169; 512: 2 angles 51 / 41 / 40 / 40 / 52, 8 angles 127 / 86 / 61 / 49 /
-// 59.
+// No more shares than hold the angles: wavefronts without any cost the others
+// their places.  In us with 1 / 2 / 4 / 8 / 16 shares, angles of a launch: 8192
+// workgroups, one angle 64 / 78 / 114 / 209 / 533, 2 angles 197 / 198 / 260 / 449
+// / 1152, 4 angles 323 / 324 / 335 / 463 / 1197; 2048, 2 angles 58 / 48 / 59 / 76
+// / 161, 4 angles 84 / 66 / 66 / 80 / 169; 512, 2 angles 51 / 41 / 40 / 40 / 52, 8
+// angles 127 / 86 / 61 / 49 / 59 (all but the first: calls of two launches).
 constexpr int64_t kGenShares4 = 4096, kGenShares8 = 640;
 
 template <int SHARES>
@@ -977,7 +976,7 @@ void launch_columns(int parts, bool longer, dim3 grid, hipStream_t st,
 }
 int general_shares(int64_t blocks, int32_t n_angles) {
   int shares = blocks >= kGenShares4 ? 4 : blocks >= kGenShares8 ? 8 : 16;
-  while (shares > 1 && n_angles < shares) shares /= 2;
+  while (shares / 2 >= n_angles) shares /= 2;
   return shares;
 }
 void launch_general(int shares, dim3 grid, hipStream_t st,
