@@ -6,9 +6,10 @@
 // not the transpose of the forward projector.  Here every voxel sums, over
 // the (ray, slice) samples of the forward kernel that touch it, the ray's
 // value times the ray weight times the sample's bilinear weight for that
-// voxel.  Samples are recomputed with the forward kernel's arithmetic
-// (kk_fp_ray, kk_fp_weight, kk_fp_coord), so <A x, y> = <x, A^T y> up to
-// rounding.
+// voxel.  Rays and ray weights are the forward kernel's (kk_fp_ray,
+// kk_fp_weight); sample coordinates are float32 offsets from float64 anchors at
+// the lane's voxels, where the forward kernels step in 64-bit fixed point.  A
+// sample's weight so agrees to ~1e-6, and <A x, y> = <x, A^T y> up to that.
 //
 // MI355X design, two launches per ray axis group:
 // 1. ray_weight_kernel: y * (ray weight), 0 for rays the forward kernel
@@ -632,6 +633,14 @@ constexpr int kColB = 8;       // voxels along b per lane
 // parts, below to four (measured, two against four: 16384 5.23 / 5.45 ms,
 // 9600 1.26 / 1.24 ms, 2048 0.32 / 0.25 ms, 512 0.12 / 0.09 ms).
 constexpr int64_t kColSplit2 = 12288;
+// Wavefronts of one part that fill half the chip.  From there a part has six
+// angles or more, whose columns fill the 64 that are set up at a time (1 / 2 / 4
+// parts in us, angles of a launch: 16384 wavefronts, 4 angles 164 / 193 / 252, 16
+// angles 501 / 520 / 565; 9216, 2 angles 90 / 100 / 138, 8 angles 192 / 188 / 212,
+// 16 angles 347 / 324 / 334; 4800, 2 angles 40 / 48 / 63); below, no more parts
+// than hold the angles (2048, 2 angles 46 / 44 / 46, 8 angles 93 / 74 / 67).
+constexpr int64_t kColFill = 4096;
+constexpr int kColAngles = 6;
 // Marks a column whose record has whole voxels apart (whole_s).
 constexpr uint64_t kWhole = uint64_t(1) << 63;
 
@@ -965,12 +974,23 @@ int64_t general_grid(FptArgs& A) {
   return int64_t(A.na) * A.tiles_b * A.tiles_c;
 }
 
+int column_parts(int64_t blocks, int32_t n_angles) {
+  const int64_t waves = blocks * kColSlices;
+  const bool fill = waves >= kColFill;
+  int parts = waves >= kColSplit2 ? 2 : 4;
+  while (parts > 1 &&
+         (fill ? n_angles < kColAngles * parts : 2 * n_angles <= parts))
+    parts /= 2;
+  return parts;
+}
 void launch_columns(int parts, bool longer, dim3 grid, hipStream_t st,
                     const kk::FpAngle* tab, const FptArgs& A) {
-  auto* kernel = parts == 2 ? (longer ? &cone_fp_t_col_kernel<2, true>
-                                      : &cone_fp_t_col_kernel<2, false>)
-                            : (longer ? &cone_fp_t_col_kernel<4, true>
-                                      : &cone_fp_t_col_kernel<4, false>);
+  auto* kernel = parts == 1   ? (longer ? &cone_fp_t_col_kernel<1, true>
+                                        : &cone_fp_t_col_kernel<1, false>)
+                 : parts == 2 ? (longer ? &cone_fp_t_col_kernel<2, true>
+                                        : &cone_fp_t_col_kernel<2, false>)
+                              : (longer ? &cone_fp_t_col_kernel<4, true>
+                                        : &cone_fp_t_col_kernel<4, false>);
   hipLaunchKernelGGL(kernel, grid, dim3(64 * kColSlices * parts), 0, st, tab,
                      A);
 }
@@ -1067,7 +1087,7 @@ int kk::fp_transpose_launch(const kk_plan_s* plan, const float* proj,
           return kk::fail(KK_ERR_UNSUPPORTED, "kk_cone_fp_transpose: grid");
         const dim3 grid(static_cast<unsigned>(blocks));
         if (colc)
-          launch_columns(blocks * kColSlices >= kColSplit2 ? 2 : 4,
+          launch_columns(column_parts(blocks, A.n_angles),
                          plan->fp_line_max >= 0.0 &&
                              plan->fp_line_mean < kLongSpacing,
                          grid, st, plan->fp, A);

@@ -72,17 +72,20 @@ def test_long_windows_of_circular_orbits(fine, tilted, device):
     assert_parity(got, oracle.cone_fp_transpose(y, pgs, vg))
 
 
-# angles of a launch per share: 1, 2, 4, 8 and 16 shares (volumes of few and of
-# many workgroups)
+# angles of a launch per share or part: 1, 2, 4, 8 and 16 shares of general
+# geometries, 1, 2 and 4 parts of circular orbits (volumes of few and of many
+# workgroups)
+@pytest.mark.parametrize("wobble", [0.5, 0.0])
 @pytest.mark.parametrize("shape,angles", [
     ((20, 18, 17), 1), ((20, 18, 17), 2), ((20, 18, 17), 7),
     ((20, 18, 17), 24), ((20, 18, 17), 70), ((90, 80, 5), 9),
-    ((90, 80, 5), 40), ((300, 280, 3), 4), ((300, 280, 3), 12)], ids=str)
-def test_shares_of_the_angles(shape, angles, device):
+    ((90, 80, 5), 40), ((300, 280, 3), 4), ((300, 280, 3), 12),
+    ((300, 280, 3), 30), ((300, 280, 3), 60)], ids=str)
+def test_shares_of_the_angles(shape, angles, wobble, device):
     import torch
     m = max(shape)
     pgs = workloads.circular_geometry(angles, 3.0 * m, 1.5 * m, 12, 40,
-                                      1.7 * m / 40, wobble_deg=0.5, seed=3)
+                                      1.7 * m / 40, wobble_deg=wobble, seed=3)
     vg = kk.resolve_volume_geometry(shape=shape, voxel_size=1.0)
     y = np.random.default_rng(5).uniform(size=(angles, 12, 40))
     got = kk.XrayTransform(pgs, vg).matched_T(
