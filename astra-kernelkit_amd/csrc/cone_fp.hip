@@ -1164,7 +1164,9 @@ int launch_fp_spec(const kk::FpSpec& S, hipStream_t stream) {
 //   110.  (Where pairs have to be built of a large volume the line is lower:
 //   they are twice the bytes.  Volumes of a few slices are as long as the call's
 //   host part either way.)
-constexpr int64_t kGatherCached = 90 << 20;
+// * kGatherCached: 197 x 244 x 197, 82 rows, 158 angles (75 MB of pairs) 381 us by
+//   lines and 458 by gathers.
+constexpr int64_t kGatherCached = 64 << 20;
 constexpr int64_t kGatherFew = 600, kGatherFewCached = 2500;  // workgroups
 constexpr int32_t kGatherSlices = 64;
 int line_rows_per_thread(const kk_plan_s* plan, int32_t rows, int32_t cols) {
