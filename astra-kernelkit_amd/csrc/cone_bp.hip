@@ -1129,15 +1129,10 @@ int launch_bp_planes(const kk::BpSpec& S, hipStream_t stream) {
   const int64_t pitch = int64_t(S.rows + kPatchGap) * 4;
   A.trb = uint32_t(pitch);
   A.tab_b = uint32_t(pitch * S.cols);
-  // Parts so that a CU (of 256) holds four wavefronts per SIMD, on circular
-  // orbits three (tiles all resident, where two parts leave some waiting): 180
-  // angles with 1 / 2 / 4 parts, circular, 64 tiles 228 / 139 / 101 us, 288 238 /
-  // 174 / 193, 512 243 / 178 / 195, 576 272 / 282 / 281, 768 279 / 305 / 287, 1024
-  // 322 / 335 / 374; general 576 393 / 386 / 410, 768 398 / 416 / 415.
+  // parts so that a CU (of 256) holds at least four wavefronts per SIMD
   const int64_t per_cu = (A.total_blocks + 255) / 256;
   const dim3 grid(unsigned(A.total_blocks));
-  const int32_t parts =
-      per_cu >= (S.plan->bp_all_circ ? 3 : 4) ? 1 : per_cu >= 2 ? 2 : 4;
+  const int32_t parts = per_cu >= 4 ? 1 : per_cu >= 2 ? 2 : 4;
   auto launch = [&](auto circ) {
     constexpr bool C = decltype(circ)::value;
     auto* kernel = parts == 1   ? &cone_bp_patch_kernel<kPatchRun, 1, C>
