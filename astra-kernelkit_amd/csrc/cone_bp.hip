@@ -399,9 +399,13 @@ __global__ __launch_bounds__(256, bp_min_blocks(K)) void cone_bp_kernel(
 //
 // What bounds circular orbits (MI355X): a gather from global memory costs a CU
 // 16 cycles per 64 updates (it took 20 with 16.5 vector instructions beside),
-// the two LDS reads 10, the patch ~3, vector issue ~10.  Measured: 512^3 / 720
-// 50.8 -> 38.0 ms, 256^3 / 360 3.2 -> 2.3 ms, 128^3 / 180 0.25 -> 0.18 ms.
-// LDS is 72% busy, vector issue about as much.
+// the two LDS reads 10 and the patch ~3.  Measured: 512^3 / 720 50.8 -> 38.0 ms,
+// 256^3 / 360 3.2 -> 2.3 ms, 128^3 / 180 0.25 -> 0.18 ms.  At 512^3 three units
+// are near their limits, none at it alone: 190 GB beyond the L2 (patches are
+// staged whole, 2.4 times the pair kernel's bytes) at 5.5 TB/s, more than a copy
+// reaches; LDS busy in 72% of the cycles, 10% of them bank conflicts; 12.5 vector
+// instructions per update, 0.24 per SIMD and cycle (0.25 at four cycles each, which
+// plain float32 adds and multiplies undercut).
 // * Bank conflicts decide the layout: a wavefront is 8 x 8 columns and the
 //   patch pitch 64 + 6 words (512^3: 38.1 ms; pitches 64 + 1, 2, 3, 4, 5, 8,
 //   11 and 13: 47.5, 39.1, 37.9, 41.6, 38.1, 59.9, 46.0 and 42.5 ms, and at
@@ -417,9 +421,9 @@ __global__ __launch_bounds__(256, bp_min_blocks(K)) void cone_bp_kernel(
 //
 // Otherwise (plans with a general angle): column, row and weight per voxel,
 // from float32 numerators around an integer base in the middle of the run and
-// one reciprocal.  26 vector instructions per update bound it (the vector unit
-// is issuing in 91% of the cycles; the pair kernel's gather took as long as
-// its instructions): 256^3 / 360 wobbling angles 4.9 -> 3.8 ms, 128^3 / 128
+// one reciprocal.  24 vector instructions per update bound it (0.28 per SIMD and
+// cycle; LDS busy in 42% of the cycles; the pair kernel's gather took as long as its
+// instructions): 256^3 / 360 wobbling angles 4.9 -> 3.8 ms, 128^3 / 128
 // 0.27 -> 0.20 ms.  Five wavefronts per SIMD instead of four spill: 3.84 ms.
 // The reciprocal as a series around the base and addresses made in float32 were
 // no faster (3.9 ms).

@@ -170,7 +170,8 @@ __device__ __forceinline__ int64_t to_fixed(double x) {
 // the slices that lie inside for a whole wavefront: 27 vector instructions a
 // gather, now 22.  200^3 tilted 1.40 -> 1.00 ms together with fp_lanes, 300^3
 // 4.83 -> 3.0 ms, 400^3 / 200 wobbling angles 10.3 -> 8.0 ms, 64^3 58 -> 46 us.
-// The address units are 63% busy, 16 cycles a gather; a deeper pipeline was
+// The address units are busy in 87% of the cycles at 256^3 / 360 wobbling angles,
+// misses included (16 cycles a gather by themselves); a deeper pipeline was
 // slower, so what is left is the L2's latency and the L1's misses.)
 template <int R, int NB>
 struct RayWalk {

@@ -605,7 +605,8 @@ __global__ __launch_bounds__(64 * SHARES, 6) void cone_fp_t_kernel(
 // sum over the rows that reach a lane's two c voxels enters two neighbouring
 // b voxels with the column's weights.  What bounds it is the number of vector
 // instructions and of row loads per (wavefront, column), in balance (profiled
-// at 256^3, 360 angles of 384^2: vector unit 79 % busy, address unit 76 %):
+// at 256^3, 360 angles of 384^2: 0.27 vector instructions per SIMD and cycle,
+// address unit busy in 76 %):
 // * rows come in loads of four per lane (unaligned dwordx4): at the lanes'
 //   stride of two voxels a single dword costs the same 16 cycles;
 // * the b voxels are registers.  The walk over tap rows is unrolled, so each

@@ -96,10 +96,11 @@ int kk_volume_to_fp_texture(const float* vol, const int32_t vol_shape[3],
 
 /* Planes: the FP texture's frames as plain floats (no pairs), which the
  * launches of kk_cone_fp_planes read: for column-coherent geometries
- * (circular orbits about z and the like) whose neighbouring detector rows
- * sample the volume about a voxel apart or closer.  kk_fp_reads_planes says
- * whether the plan's parameters with a rows x cols detector are such
- * (1) or not (0).  Same frames and halo as the FP texture, half its size. */
+ * (circular orbits about z and the like), up to 2048 slices, where that is the
+ * faster way: rows enough for wavefronts of 64, and not only a few workgroups.
+ * kk_fp_reads_planes says whether the plan's parameters with a rows x cols
+ * detector are such (1) or not (0).  Same frames and halo as the FP texture,
+ * half its size. */
 int32_t kk_fp_reads_planes(const kk_plan* plan, int32_t rows, int32_t cols);
 int64_t kk_fp_planes_elems(const int32_t vol_shape[3], int32_t frame_mask);
 int kk_volume_to_fp_planes(const float* vol, const int32_t vol_shape[3],
@@ -119,7 +120,8 @@ int kk_projections_to_bp_texture(const float* proj, int32_t n_angles,
  * kk_cone_bp_planes and kk_sirt_bp_update_planes read: for circular orbits
  * about z and for plans with an angle of no special form (not for detectors
  * tilted in their own plane alone), if the volume's 16 x 16 x 16 voxel tiles
- * project onto at most 64 x 64 pixels.
+ * project onto at most 64 x 64 pixels, and the volume is more than eight
+ * voxels thick or of at most 256 tiles.
  * kk_bp_reads_planes says whether the plan's parameters with a rows x cols
  * detector and the volume's shape are such (1) or not (0).
  * kk_residual_to_bp_planes: planes of the SIRT residual (proj - y) * R. */
@@ -247,9 +249,11 @@ int kk_cone_bp_planes(const kk_plan* plan, const float* planes,
 
 /* Exact transpose of kk_cone_fp (matched adjoint, for gradients): every
  * (ray, slice) sample of the forward projection adds proj * scale *
- * bilinear weight to its in-volume taps, with the forward kernel's own
- * coordinate and weight arithmetic (bit-identical weights), so
- * <A x, y> = <x, A^T y> up to rounding.  No counterpart in
+ * bilinear weight to its in-volume taps.  The rays are the forward kernels'
+ * (float64), the samples' coordinates come from them by float32 offsets
+ * within a tile where those kernels take fixed-point steps along the ray: the
+ * weights agree to about 1e-6, and <A x, y> = <x, A^T y> up to rounding.  No
+ * counterpart in
  * the reference, whose autograd backward uses the voxel-driven
  * backprojector (kernelkit/torch_support.py:29-33); it replaces that call
  * where an exact gradient is wanted.  proj: (angle, row, col) strides; vol:
