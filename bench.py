@@ -13,20 +13,21 @@ does two passes of updates).
 The JSON line also carries:
 
 * ``roofline`` for the dominant kernel (the forward projection, by column
-  lines in LDS): achieved gather bytes per second = 16 B per bilinear sample
-  x samples per launch / average kernel time (HIP events on the launching
-  stream), against the gather ceiling, the rate of a kernel that fetches
-  every sample from the caches: the vector-memory return path of 64 B/clk
-  per CU x 256 CUs x 2.4 GHz, next to this run's probe rates of 16-byte
-  gathers in the projectors' access shape (``kk_probe_gather``) from L1-, L2-
-  and HBM-resident footprints.  The kernel interpolates each pair of volume
-  rows once per detector column and reads its samples from LDS, so ``frac``
-  exceeds 1;
-  ``traffic`` is the HBM bytes per launch from the rocprofv3 FETCH_SIZE +
-  WRITE_SIZE counters (scaled by a plain-copy calibration), read from
-  ``profiles/cone_fp_bp_512cube_720_traffic.json`` when present, and
-  ``traffic_GBs`` / ``traffic_frac_of_hbm`` that amount at this run's
-  kernel time against the 8 TB/s HBM peak;
+  lines in LDS): the bytes a launch moves beyond the L2 (``traffic``: rocprofv3
+  FETCH_SIZE + WRITE_SIZE counters scaled by a plain-copy calibration, read
+  from ``profiles/cone_fp_bp_512cube_720_traffic.json``) over the kernel's time
+  in this run (HIP events on the launching stream), against the 8 TB/s HBM
+  peak; ``vector`` is the same launch's nine float32 operations per bilinear
+  sample against the float32 vector peak, ``bp_kernel`` both for the
+  backprojection (twelve operations per update).
+  ``gather_equivalent``: 16 B per sample over the kernel's time against the
+  gather ceiling, the rate of a kernel that fetches every sample from the
+  caches: the vector-memory return path of 64 B/clk per CU x 256 CUs x 2.4
+  GHz, next to this run's probe rates of 16-byte gathers in the projectors'
+  access shape (``kk_probe_gather``) from L1-, L2- and HBM-resident
+  footprints.  The kernel interpolates each pair of volume rows once per
+  detector column and reads its samples from LDS, so this ratio exceeds 1 and
+  bounds nothing;
 * ``cpu_baseline``: the FP64 NumPy oracle in 16 host processes of one core
   each (``single_core``: one process), timed on a bounded sample of the
   same workload (one angle, a band of detector rows for FP and a slab of
@@ -52,6 +53,8 @@ L2_PEAK_GBS = 8 * 16 * 128 * 2.4  # GB/s: 8 XCD x 16 ch x 128 B/clk x 2.4 GHz
 # the rate at which 16-byte gathers reach the registers even from L1
 L1_RETURN_GBS = 256 * 64 * 2.4
 HBM_PEAK_GBS = 8000.0
+# float32 vector peak: 256 CUs x 128 lanes x 2 x 2.4 GHz
+VECTOR_PEAK_TFLOPS = 256 * 128 * 2 * 2.4e-3
 TRAFFIC_FILE = os.path.join(ROOT, "profiles",
                             "cone_fp_bp_512cube_720_traffic.json")
 
@@ -332,15 +335,13 @@ def _small_run(pool, vol, y, sirt_iters):
 
 def gpu_small(sirt_iters=20):
     """The same small-workload jobs on the GPU (inputs resident, HIP events
-    on the current stream): FP, BP, Ram-Lak FDK (``fdk``'s pre-weight and
-    filter fused into the BP texture, then the BP) and ``sirt_iters`` SIRT
-    iterations with their setup, in milliseconds."""
+    on the current stream): FP, BP, Ram-Lak FDK (as ``kk.fdk`` without its
+    host copy) and ``sirt_iters`` SIRT iterations with their setup, in
+    milliseconds."""
     import torch
 
     import kernelkit as kk
     from kernelkit import workloads
-    from kernelkit.kernel import ProjectionTexture
-    from kernelkit.processing import filter_into
 
     pgs, vg = workloads.config_geometry("small")
     x = torch.from_numpy(workloads.ellipsoid_phantom(vg.shape, n=10,
@@ -349,17 +350,7 @@ def gpu_small(sirt_iters=20):
     y = A(x)
     v = torch.empty_like(x)
     stream = torch.cuda.current_stream()
-    tex = ProjectionTexture(*y.shape, like=y)
-    tex.zero()
-    bptor = kk.BackProjector()
-    bptor.projection_geometry = pgs
-    bptor.volume_geometry = vg
-    bptor.volume = v
-
-    def fdk():
-        filter_into(y, tex, geoms=pgs, filter="ramlak")
-        bptor._textures = tex
-        bptor()
+    fdk = _fdk_call(pgs, vg, y, v, "ramlak")
 
     def sirt():
         kk.sirt(y, pgs, vg, iters=sirt_iters, verbose=False, return_gpu=True)
@@ -642,37 +633,47 @@ def st_cfg_repr(B, which):
     return {"tile": c.tile, "grid": c.grid}
 
 
-def algorithms_full(pgs, vg, x, iters=50):
-    """FDK (Hann) and 50 SIRT iterations of the full workload, end to end
-    on the device (inputs resident; FDK includes pre-weight + filter fused
-    into the backprojection texture; SIRT includes its setup: C, R and the
-    textures)."""
+def _fdk_call(pgs, vg, y, out, filter):
+    """FDK of device projections into ``out`` as ``kk.fdk`` runs it, minus
+    its host copy of the result: pre-weight and row filter into a buffer,
+    planes, backprojection."""
     import torch
 
     import kernelkit as kk
-
     from kernelkit.kernel import ProjectionTexture
-    from kernelkit.processing import filter_into
+    from kernelkit.processing import filter_rows_into
 
-    dev = x.device
-    A = kk.XrayTransform(pgs, vg)
-    y = A(x)
-    out = torch.empty_like(x)
-    stream = torch.cuda.current_stream(dev)
-    # FDK on the device, as algo.fdk minus its host copy of the result:
-    # pre-weight + Hann row filter fused into the BP texture, then the BP
-    tex = ProjectionTexture(*y.shape, device=dev)
-    tex.zero()
+    tex = ProjectionTexture(*y.shape, like=y)
+    filtered = torch.empty_like(y)
     bptor = kk.BackProjector()
     bptor.projection_geometry = pgs
     bptor.volume_geometry = vg
     bptor.volume = out
 
     def fdk():
-        filter_into(y, tex, geoms=pgs, filter="hann")
+        filter_rows_into(y, filtered, geoms=list(pgs), filter=filter)
+        tex.update(filtered, planes=True)
         bptor._textures = tex
         bptor()
 
+    return fdk
+
+
+def algorithms_full(pgs, vg, x, iters=50):
+    """FDK (Hann) and 50 SIRT iterations of the full workload, end to end
+    on the device (inputs resident; FDK is pre-weight + filter, texture and
+    backprojection as ``kk.fdk`` runs them; SIRT includes its setup: C, R and
+    the textures)."""
+    import torch
+
+    import kernelkit as kk
+
+    dev = x.device
+    A = kk.XrayTransform(pgs, vg)
+    y = A(x)
+    out = torch.empty_like(x)
+    stream = torch.cuda.current_stream(dev)
+    fdk = _fdk_call(pgs, vg, y, out, "hann")
     fdk()
     t_fdk = _event_ms(fdk, stream, reps=3)
     t_sirt = _event_ms(lambda: kk.sirt(y, pgs, vg, iters=iters,
@@ -689,10 +690,9 @@ def autograd_diff(ceiling=None):
     360 angles, 384^2 detector; also through the reference's default
     autograd operator (voxel-driven backprojector in the backward pass).
 
-    The transpose moves the forward projection's samples backwards: each
-    sample's four tap weights are gathered by the voxels they touch, 16 B
-    per sample as in the forward gather, so its rate against the gather
-    ``ceiling`` (GB/s) compares directly with the forward projection's."""
+    ``*_gather_ratio``: 16 B per sample over the time against the gather
+    ``ceiling`` (GB/s), the rate of a kernel that fetches every sample's four
+    taps from the caches (above 1: this one does not)."""
     import numpy as np
     import torch
 
@@ -760,11 +760,12 @@ def autograd_diff(ceiling=None):
         bw = 16 * fp_samples(pgw, vg)
         res.update({
             "gather_ceiling_GBs": ceiling,
-            "fp_frac": round(b / (t_fp * 1e-3) / 1e9 / ceiling, 4),
-            "transpose_frac": round(b / (t_t * 1e-3) / 1e9 / ceiling, 4),
-            "wobble_fp_frac": round(bw / (t_fpw * 1e-3) / 1e9 / ceiling, 4),
-            "wobble_transpose_frac": round(
-                bw / (t_tw * 1e-3) / 1e9 / ceiling, 4),
+            **{f"{name}_gather_ratio": round(
+                nbytes / (ms * 1e-3) / 1e9 / ceiling, 4)
+               for name, nbytes, ms in (
+                   ("fp", b, t_fp), ("transpose", b, t_t),
+                   ("wobble_fp", bw, t_fpw),
+                   ("wobble_transpose", bw, t_tw))},
         })
     return res
 
@@ -1009,10 +1010,28 @@ def main(argv=None):
     fp_bytes = 16 * samples
     bp_bytes = 16 * updates
     achieved = fp_bytes / (t_fp * 1e-3) / 1e9
-    traffic = None
+    traffic = bp_traffic = None
     if os.path.exists(TRAFFIC_FILE) and args.config == "full":
         with open(TRAFFIC_FILE) as f:
-            traffic = json.load(f).get("cone_fp_line_kernel_bytes")
+            rec = json.load(f)
+        traffic = rec.get("cone_fp_line_kernel_bytes")
+        bp_traffic = rec.get("cone_bp_patch_kernel_bytes")
+
+    def beyond_l2(nbytes, ms):
+        """Rate (GB/s) of the bytes beyond the L2 and its share of the
+        HBM peak."""
+        if nbytes is None:
+            return {"achieved": None, "frac": None}
+        rate = nbytes / (ms * 1e-3) / 1e9
+        return {"achieved": round(rate, 1),
+                "frac": round(rate / HBM_PEAK_GBS, 4)}
+
+    def vector(flops, ms):
+        rate = flops / (ms * 1e-3) / 1e12
+        return {"achieved_tflops": round(rate, 2),
+                "peak_tflops": round(VECTOR_PEAK_TFLOPS, 1),
+                "frac": round(rate / VECTOR_PEAK_TFLOPS, 4)}
+
     compulsory_fp = 4 * (int(np.prod(shape)) + n * rows * cols)
     out = {
         "metric": METRIC,
@@ -1040,20 +1059,28 @@ def main(argv=None):
             "bp_texture_ms": round(t_btex, 3),
         },
         "roofline": {
-            "bound": "gather",
+            "bound": "beyond_l2",
             "kernel": "cone_fp_line_kernel",
-            "achieved": round(achieved, 1),
-            # the gather ceiling: 64 B/clk/CU x 256 CUs x 2.4 GHz, which
-            # the L1-resident 16-byte gather probes of this run reach
-            # within a few percent ("gather_probes_GBs")
-            "peak": ceiling,
-            "peak_source": "64 B/clk/CU return path; L1-resident "
-                           "kk_probe_gather reaches "
-                           f"{probe_best / L1_RETURN_GBS:.3f} of it",
+            # measured beyond-L2 (fabric/HBM) bytes of the launch at this
+            # launch's time, against the HBM peak
+            **beyond_l2(traffic, t_fp),
+            "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
-            "frac": round(achieved / ceiling, 4),
-            "frac_of_best_probe": round(achieved / probe_best, 4),
             "traffic": traffic,
+            "vector": vector(9 * samples, t_fp),
+            "gather_equivalent": {
+                "rate": round(achieved, 1),
+                # the gather ceiling: 64 B/clk/CU x 256 CUs x 2.4 GHz, which
+                # the L1-resident 16-byte gather probes of this run reach
+                # within a few percent ("gather_probes_GBs")
+                "ceiling": ceiling,
+                "ceiling_source": "64 B/clk/CU return path; L1-resident "
+                                  "kk_probe_gather reaches "
+                                  f"{probe_best / L1_RETURN_GBS:.3f} of it",
+                "unit": "GB/s",
+                "ratio": round(achieved / ceiling, 4),
+                "ratio_to_l2_theoretical": round(achieved / L2_PEAK_GBS, 4),
+            },
             "algorithmic_bytes": fp_bytes,
             "bytes_per_update": round(fp_bytes / updates, 4),
             "gather_probes_GBs": gathers,
@@ -1061,19 +1088,15 @@ def main(argv=None):
                 compulsory_fp / (t_fp * 1e-3) / 1e9, 1),
             "l2_stream_GBs": round(l2_rate, 1),
             "l2_theoretical_GBs": round(L2_PEAK_GBS, 1),
-            "frac_of_l2_theoretical": round(achieved / L2_PEAK_GBS, 4),
-            "hbm_peak": HBM_PEAK_GBS,
-            # measured beyond-L2 (fabric/HBM) bytes of the launch at this
-            # launch's time, against the HBM peak
-            "traffic_GBs": (None if traffic is None else
-                            round(traffic / (t_fp * 1e-3) / 1e9, 1)),
-            "traffic_frac_of_hbm": (
-                None if traffic is None else
-                round(traffic / (t_fp * 1e-3) / 1e9 / HBM_PEAK_GBS, 4)),
             "bp_kernel": {
-                "achieved": round(bp_bytes / (t_bp * 1e-3) / 1e9, 1),
-                "frac": round(bp_bytes / (t_bp * 1e-3) / 1e9 / ceiling,
-                              4),
+                **beyond_l2(bp_traffic, t_bp),
+                "traffic": bp_traffic,
+                "vector": vector(12 * updates, t_bp),
+                "gather_equivalent": {
+                    "rate": round(bp_bytes / (t_bp * 1e-3) / 1e9, 1),
+                    "ratio": round(
+                        bp_bytes / (t_bp * 1e-3) / 1e9 / ceiling, 4),
+                },
                 "bytes_per_update": 16,
             },
         },
